@@ -88,6 +88,12 @@ __device__ __forceinline__ float atan2_xpos(float y, float x) {
   return copysignf(r, y);
 }
 
+// atan2(y, x) for x, y >= 0 not both zero (NaN at the origin).
+__device__ __forceinline__ float atan2_first(float y, float x) {
+  const float r = atan_unit(fminf(x, y) * rcp_fast(fmaxf(x, y)));
+  return y > x ? 1.570796327f - r : r;
+}
+
 // -------------------------------------------------------------- Hammersley
 // Point i of an n-point set: (i/n correctly rounded, float(bitreverse(i)) * 2^-32).
 __device__ __forceinline__ uint32_t vdc_bits(uint32_t i) { return __builtin_bitreverse32(i); }
@@ -596,6 +602,12 @@ __device__ inline f3 bcube_sample(const float4* __restrict__ cube, const Bordere
 }
 
 // ------------------------------------------------------------ wave helpers
+// Orders this wave's LDS writes before its later LDS reads from other lanes.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 __device__ __forceinline__ double wave_sum_f64(double v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

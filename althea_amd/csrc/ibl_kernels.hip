@@ -698,7 +698,10 @@ althea_status launch_prefilter_points(const float* pyr, int env_w, int env_h, in
 // GenIrradianceMap.comp:106-155 per cube texel: the Riemann sum over
 // theta_samples azimuths x phi_samples polar angles of radiance(d) cos sin,
 // read at the fixed source LOD log2(W / theta_samples), times
-// pi / (theta_samples phi_samples).
+// pi / (theta_samples phi_samples).  An even azimuth count over a source
+// whose level is at least 8 x 4 takes the folded kernel below; the kernel
+// here, one wave per texel, serves odd azimuth counts, smaller levels, and
+// two levels that are not an exact halving.
 struct IrradianceParams {
   SplitLevel lv0, lv1;  // the two source levels around LOD log2(W / theta_samples), split gather copies
   SplitLevel grid;      // their blend grid (blend)
@@ -883,24 +886,37 @@ static BlendGrid blend_grid(int w, int h, const IrradianceLod& lod) {
   return b;
 }
 
-// The theta and phi tables, then the blend grid of levels l0, l1 or their
-// split gather copy.
-size_t irradiance_workspace_bytes(int w, int h, int, int theta) {
-  int phi = irradiance_phi_samples(w, h, theta);
-  const size_t tables = align256(sizeof(float2) * theta) + align256(sizeof(float4) * std::max(phi, 1));
-  if (w <= 0 || h <= 0 || theta <= 0) return tables;
-  const IrradianceLod lod = irradiance_lod(w, h, theta);
-  const BlendGrid b = blend_grid(w, h, lod);
-  if (b.ok) return tables + 12 * b.plane;
-  return tables + split_gather_bytes(w, h, lod.l0, lod.l1);
-}
-
 struct BlendGridParams {
   int w0, h0, nx, ny;
   uint32_t off0, off1;  // pyramid texel offsets of the two levels
   double delta;
   size_t plane;
 };
+
+// Bilinear REPEAT value of the level at `off` (w x h) at texel coordinates
+// (x, y), in FP64.
+__device__ __forceinline__ void level_bilinear_f64(const float4* __restrict__ pyr, uint32_t off, int w, int h, double x,
+                                                   double y, double* v) {
+  const double fx = floor(x), fy = floor(y), ax = x - fx, ay = y - fy;
+  const int i0 = static_cast<int>(fx), j0 = static_cast<int>(fy);
+  auto at = [&](int i, int j) {
+    return pyr[off + static_cast<size_t>((j % h + h) % h) * w + (i % w + w) % w];
+  };
+  const float4 t00 = at(i0, j0), t10 = at(i0 + 1, j0), t01 = at(i0, j0 + 1), t11 = at(i0 + 1, j0 + 1);
+  const float a[4][3] = {{t00.x, t00.y, t00.z}, {t10.x, t10.y, t10.z}, {t01.x, t01.y, t01.z}, {t11.x, t11.y, t11.z}};
+  for (int k = 0; k < 3; ++k)
+    v[k] = (1.0 - ay) * ((1.0 - ax) * a[0][k] + ax * a[1][k]) + ay * ((1.0 - ax) * a[2][k] + ax * a[3][k]);
+}
+
+// The blend (1 - delta) B0 + delta B1 at fine coordinates (x0, y0), B1 at
+// x0 / 2 - 1/4 of the half-size level.
+__device__ __forceinline__ void blend_value(const float4* __restrict__ pyr, const BlendGridParams& p, double x0,
+                                            double y0, float f[3]) {
+  double b0[3], b1[3];
+  level_bilinear_f64(pyr, p.off0, p.w0, p.h0, x0, y0, b0);
+  level_bilinear_f64(pyr, p.off1, p.w0 / 2, p.h0 / 2, 0.5 * x0 - 0.25, 0.5 * y0 - 0.25, b1);
+  for (int k = 0; k < 3; ++k) f[k] = static_cast<float>((1.0 - p.delta) * b0[k] + p.delta * b1[k]);
+}
 
 // One thread per padded node (r, c): node (c - 1, r - 1) wrapped to the
 // grid, at fine coordinates (2 (n / 3) + (n % 3) / 2) per axis; its value
@@ -913,25 +929,301 @@ __global__ __launch_bounds__(256) void blend_grid_kernel(const float4* __restric
   const int r = static_cast<int>(i / W), c = static_cast<int>(i - r * W);
   auto wrap = [](int k, int n) { return k < 0 ? k + n : (k >= n ? k - n : k); };
   const int n = wrap(c - 1, p.nx), m = wrap(r - 1, p.ny);
-  const double x0 = 2.0 * (n / 3) + 0.5 * (n % 3), y0 = 2.0 * (m / 3) + 0.5 * (m % 3);
-  auto bilinear = [&](uint32_t off, int w, int h, double x, double y, double* v) {
-    const double fx = floor(x), fy = floor(y), ax = x - fx, ay = y - fy;
-    const int i0 = static_cast<int>(fx), j0 = static_cast<int>(fy);
-    auto at = [&](int i, int j) {
-      return pyr[off + static_cast<size_t>((j % h + h) % h) * w + (i % w + w) % w];
-    };
-    const float4 t00 = at(i0, j0), t10 = at(i0 + 1, j0), t01 = at(i0, j0 + 1), t11 = at(i0 + 1, j0 + 1);
-    const float a[4][3] = {{t00.x, t00.y, t00.z}, {t10.x, t10.y, t10.z}, {t01.x, t01.y, t01.z}, {t11.x, t11.y, t11.z}};
-    for (int k = 0; k < 3; ++k)
-      v[k] = (1.0 - ay) * ((1.0 - ax) * a[0][k] + ax * a[1][k]) + ay * ((1.0 - ax) * a[2][k] + ax * a[3][k]);
-  };
-  double b0[3], b1[3];
-  bilinear(p.off0, p.w0, p.h0, x0, y0, b0);
-  bilinear(p.off1, p.w0 / 2, p.h0 / 2, 0.5 * x0 - 0.25, 0.5 * y0 - 0.25, b1);
   float f[3];
-  for (int k = 0; k < 3; ++k) f[k] = static_cast<float>((1.0 - p.delta) * b0[k] + p.delta * b1[k]);
+  blend_value(pyr, p, 2.0 * (n / 3) + 0.5 * (n % 3), 2.0 * (m / 3) + 0.5 * (m % 3), f);
   reinterpret_cast<float2*>(out)[i] = make_float2(f[0], f[1]);
   out[2 * p.plane + i] = f[2];
+}
+
+// ------------------------------------------------- irradiance, folded source
+// The equirect map, the texel lattice and (with an even azimuth count) the
+// azimuth set are all symmetric under the eight sign flips F of (x, y, z):
+// the frame of texel direction F n is F times the frame of n up to a half
+// turn and a reflection of the azimuth, so the samples of the eight texels
+// F n are F times the samples of n, and a flip acts on a lookup as yaw ->
+// pi - yaw (x), yaw -> -yaw (z), pitch -> -pitch (y).  One evaluation of a
+// sample's direction, angles, cell and weights serves eight texels, whose
+// lookups read the same node of the source folded onto yaw and pitch in
+// [0, pi/2]: a folded node holds its eight images (x bit 0, z bit 1, y bit 2
+// of the slot) as eight 12-byte slots.
+//
+// Folded coordinates (either axis, E the extent): x' = angle E / 2pi + 3/2
+// (pitch: angle H / pi + 3/2), which is the source coordinate minus E / 2 - 2,
+// so the node pattern of the blend grid keeps its phase (E % 4 == 0).  Column
+// 0 is the node at x' = 1, just across the fold.  Two more columns hold the
+// precompute's pole branch (|xz| <= 0.001 reads yaw 0 whatever the signs of
+// x and z): the nodes beside yaw 0 in every slot, without the x and z flips.
+struct FoldGrid {
+  bool ok;
+  int w0, h0, blend;
+  int cols, rows;  // columns without the two pole columns
+  size_t nodes;    // stored nodes, pole columns included
+};
+constexpr int kFoldNodeBytes = 96;
+constexpr size_t kFoldMaxBytes = size_t{1} << 30;
+
+static FoldGrid fold_grid(int w, int h, int theta, const IrradianceLod& lod) {
+  FoldGrid f{};
+  if (w <= 0 || h <= 0 || theta % 2 != 0) return f;
+  const PyramidGeometry g = pyramid_geometry(w, h);
+  f.blend = lod.delta != 0.0f ? 1 : 0;
+  if (f.blend && !blend_grid(w, h, lod).ok) return f;
+  f.w0 = g.w[lod.l0];
+  f.h0 = g.h[lod.l0];
+  if (f.w0 % 8 != 0 || f.h0 % 4 != 0) return f;
+  f.cols = (f.blend ? 3 * f.w0 / 8 : f.w0 / 4) + 2;
+  f.rows = (f.blend ? 3 * f.h0 / 4 : f.h0 / 2) + 2;
+  f.nodes = static_cast<size_t>(f.cols + 2) * f.rows;
+  f.ok = kFoldNodeBytes * f.nodes <= kFoldMaxBytes;
+  return f;
+}
+
+// The theta and phi tables, then the folded grid, the blend grid of levels
+// l0, l1 or their split gather copy.
+size_t irradiance_workspace_bytes(int w, int h, int, int theta) {
+  int phi = irradiance_phi_samples(w, h, theta);
+  const size_t tables = align256(sizeof(float2) * theta) + align256(sizeof(float4) * std::max(phi, 1));
+  if (w <= 0 || h <= 0 || theta <= 0) return tables;
+  const IrradianceLod lod = irradiance_lod(w, h, theta);
+  const FoldGrid f = fold_grid(w, h, theta, lod);
+  if (f.ok) return tables + align256(kFoldNodeBytes * f.nodes);
+  const BlendGrid b = blend_grid(w, h, lod);
+  if (b.ok) return tables + 12 * b.plane;
+  return tables + split_gather_bytes(w, h, lod.l0, lod.l1);
+}
+
+struct FoldGridParams {
+  BlendGridParams src;  // w0, h0, off0, off1, delta
+  int blend, cols, rows;
+};
+
+// One thread per slot of a folded node, in storage order.
+__global__ __launch_bounds__(256) void fold_grid_kernel(const float4* __restrict__ pyr, const FoldGridParams p,
+                                                        float* __restrict__ out) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  const uint32_t cols = static_cast<uint32_t>(p.cols) + 2u;
+  if (i >= 8u * cols * static_cast<uint32_t>(p.rows)) return;
+  const int slot = static_cast<int>(i & 7u);
+  const int r = static_cast<int>((i >> 3) / cols), c = static_cast<int>((i >> 3) - static_cast<uint32_t>(r) * cols);
+  const int W = p.src.w0, H = p.src.h0;
+  const bool pole = c >= p.cols;
+  // Column k of the stored grid as x' (column 0: the node at x' = 1).
+  auto at = [&](int k) { return p.blend ? 2.0 * ((k + 2) / 3) + 0.5 * ((k + 2) % 3) : k + 1.0; };
+  double x0 = (pole ? 1.0 + (c - p.cols) : at(c)) + (0.5 * W - 2.0);
+  double y0 = at(r) + (0.5 * H - 2.0);  // the row of negative pitch
+  if (!pole && (slot & 1)) x0 = 1.5 * W - 1.0 - x0;
+  if (!pole && (slot & 2)) x0 = W - 1.0 - x0;
+  if (!(slot & 4)) y0 = H - 1.0 - y0;
+  float f[3];
+  if (p.blend) {
+    blend_value(pyr, p.src, x0, y0, f);
+  } else {
+    const int i0 = (static_cast<int>(x0) + 2 * W) % W, j0 = (static_cast<int>(y0) + 2 * H) % H;
+    const float4 t = pyr[p.src.off0 + static_cast<size_t>(j0) * W + i0];
+    f[0] = t.x, f[1] = t.y, f[2] = t.z;
+  }
+  for (int k = 0; k < 3; ++k) out[3 * static_cast<size_t>(i) + k] = f[k];
+}
+
+struct FoldParams {
+  float kx, ky;  // x' = yaw kx + 3/2, y' = pitch ky + 3/2
+  int cols;
+  uint32_t rowbytes;  // kFoldNodeBytes (cols + 2)
+  int size;
+  int theta_samples, phi_samples;
+  int theta_steps, steps;  // 8-azimuth steps per polar group, steps in all
+  double scale;            // pi / theta_samples / phi_samples
+};
+
+// Lower node (stored column or row) of folded coordinate x' and the fraction.
+template <bool kBlend>
+__device__ __forceinline__ int fold_cell(float x, float& t) {
+  if (kBlend) return blend_cell(x, t) - 2;
+  t = __builtin_amdgcn_fractf(x);
+  return cvt_floor(x) - 1;
+}
+
+// A block of 16 waves per orbit of eight texels F n; the waves take the
+// orbit's steps in turn, a step being a patch of 8 polar by 8 azimuth samples.
+// Each lane evaluates one sample of the step for n = |n| and leaves (node
+// offset with the sample's own signs as slot bits, fractions, weight) in LDS;
+// then in eight rounds lane (s, F) adds sample 8 k + s into texel F.
+// FP32 sums of 32 lookups are flushed into FP64 (kF64Sums); lanes and waves
+// combine in a fixed order.
+//
+// Bound: the gathers. A gather instruction whose lanes each read 12 or 16
+// bytes takes 16 cycles of the texture data return; the eight lanes of a
+// sample read one node's 96 bytes, so a round's loads stay at 16.5 cycles
+// (31 for 64 unrelated lookups, irradiance_cube_kernel) and the return is 93 %
+// busy, and a lookup costs about 30 VALU instead of 115.  512 x 256 source,
+// 32^2 x 6 texels, 300 x 150 samples: 1.09 -> 0.51 ms.  Measured beside it
+// for the whole precompute (0.816 ms): 16-byte slots 0.84 (4.8 MB of nodes
+// against 3.6 MB in a 4 MB L2), RG and B planes (eight narrower loads a
+// lookup) 1.05, six waves per SIMD instead of four 0.91; 4, 8 or 16 waves
+// per orbit alike, and 16 keep the GPU filled on the smallest cubes.
+constexpr int kFoldWaves = 16;
+// Azimuth and polar tables of up to this many bytes are read from LDS.
+constexpr size_t kFoldTableMax = 32768;
+
+template <bool kF64Sums, bool kBlend, bool kLds>
+__global__ __launch_bounds__(64 * kFoldWaves) void irradiance_fold_kernel(const char* __restrict__ grid,
+                                                                          const float2* __restrict__ theta_glob,
+                                                                          const float4* __restrict__ phi_glob,
+                                                                          const FoldParams p,
+                                                                          float4* __restrict__ cube) {
+  using T = typename PrefilterSums<kF64Sums>::T;
+  typedef const __attribute__((address_space(1))) char gchar;
+  typedef const __attribute__((address_space(1))) float gfloat;
+  extern __shared__ float4 s_tab[];  // the polar rows, then the azimuth rows (kLds)
+  __shared__ float4 s_rec[kFoldWaves][64];
+  __shared__ T s_part[kFoldWaves][3][8];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  float2* s_theta = reinterpret_cast<float2*>(s_tab + p.phi_samples);
+  if (kLds) {
+    for (int i = threadIdx.x; i < p.phi_samples; i += 64 * kFoldWaves) s_tab[i] = phi_glob[i];
+    for (int i = threadIdx.x; i < p.theta_samples; i += 64 * kFoldWaves) s_theta[i] = theta_glob[i];
+    __syncthreads();
+  }
+  const float4* phi_tab = kLds ? s_tab : phi_glob;
+  const float2* theta_tab = kLds ? s_theta : theta_glob;
+  const int S = p.size, half = (S + 1) / 2;
+  // The orbit's representative with no negative component, on the lattice of
+  // half-texels (cube_texel_raw_dir): the major component is S.
+  const int axis = blockIdx.x / (half * half);
+  const int rem = blockIdx.x - axis * half * half;
+  const int even = 1 - (S & 1);
+  const int cu = 2 * (rem / half) + even, cv = 2 * (rem % half) + even;
+  const int nx = axis == 0 ? S : cu, ny = axis == 1 ? S : (axis == 0 ? cu : cv), nz = axis == 2 ? S : cv;
+  const Frame fr = local_to_world(mk(static_cast<float>(nx), static_cast<float>(ny), static_cast<float>(nz)));
+  const uint32_t flip = static_cast<uint32_t>(lane & 7);
+  float4* rec = s_rec[wave];
+  T ar = 0, ag = 0, ab = 0;
+  float sr = 0.0f, sg = 0.0f, sb = 0.0f;
+  int done = 0;
+  for (int step = wave; step < p.steps; step += kFoldWaves) {
+    const int pg = step / p.theta_steps, as = step - pg * p.theta_steps;
+    const int i = as * 8 + (lane & 7), j = pg * 8 + (lane >> 3);
+    const bool valid = i < p.theta_samples && j < p.phi_samples;
+    const float2 th = theta_tab[min(i, p.theta_samples - 1)];
+    const float4 ph = phi_tab[min(j, p.phi_samples - 1)];
+    const f3 u = fr.t * ph.y, v = fr.b * ph.y, w = fr.n * ph.x;
+    const f3 d = mk(fmaf(u.x, th.x, fmaf(v.x, th.y, w.x)), fmaf(u.y, th.x, fmaf(v.y, th.y, w.y)),
+                    fmaf(u.z, th.x, fmaf(v.z, th.y, w.z)));
+    const float len_xz = sqrt_fast(fmaf(d.x, d.x, d.z * d.z));
+    const bool off_pole = len_xz > 0.001f;  // equirect_angles' branch
+    float fx, fy;
+    int col = fold_cell<kBlend>(fmaf(atan2_first(fabsf(d.z), fabsf(d.x)), p.kx, 1.5f), fx);
+    const int row =
+        fold_cell<kBlend>(fmaf(off_pole ? atan2_first(fabsf(d.y), len_xz) : 0.5f * kPi, p.ky, 1.5f), fy);
+    if (!off_pole) col = p.cols, fx = 0.5f;
+    const uint32_t signs = (__float_as_uint(d.x) >> 31) | (__float_as_uint(d.z) >> 31 << 1) |
+                           (__float_as_uint(d.y) >> 31 << 2);
+    const uint32_t off = static_cast<uint32_t>(row) * p.rowbytes + static_cast<uint32_t>(col * kFoldNodeBytes);
+    rec[lane] = make_float4(__uint_as_float(off | signs), fx, fy, valid ? ph.z : 0.0f);
+    wave_lds_sync();
+#pragma unroll 4
+    for (int k = 0; k < 8; ++k) {
+      const float4 q = rec[8 * k + (lane >> 3)];
+      const uint32_t node = __float_as_uint(q.x);  // a multiple of 32, plus the sample's sign bits
+      const uint32_t o0 = (node & ~7u) + ((node ^ flip) & 7u) * 12u;
+      gfloat* r0 = (gfloat*)((gchar*)grid + o0);
+      gfloat* r1 = (gfloat*)((gchar*)grid + (o0 + p.rowbytes));
+      LevelTaps t;
+      t.t00 = mk(r0[0], r0[1], r0[2]);
+      t.t10 = mk(r0[24], r0[25], r0[26]);
+      t.t01 = mk(r1[0], r1[1], r1[2]);
+      t.t11 = mk(r1[24], r1[25], r1[26]);
+      t.ax = q.y;
+      t.ay = q.z;
+      taps_acc(t, q.w, sr, sg, sb);
+    }
+    wave_lds_sync();  // the rounds' reads before the next step's records
+    if ((++done & 3) == 0) {
+      ar += sr, ag += sg, ab += sb;
+      sr = sg = sb = 0.0f;
+    }
+  }
+  ar += sr, ag += sg, ab += sb;
+#pragma unroll
+  for (int o = 8; o < 64; o <<= 1) {
+    ar += __shfl_xor(ar, o, 64);
+    ag += __shfl_xor(ag, o, 64);
+    ab += __shfl_xor(ab, o, 64);
+  }
+  if (lane < 8) s_part[wave][0][lane] = ar, s_part[wave][1][lane] = ag, s_part[wave][2][lane] = ab;
+  __syncthreads();
+  if (threadIdx.x >= 8) return;
+  // Texel F n; a flip of a zero component names the same texel again.
+  if (((lane & 1) && nx == 0) || ((lane & 2) && nz == 0) || ((lane & 4) && ny == 0)) return;
+  T v[3] = {0, 0, 0};
+  for (int k = 0; k < kFoldWaves; ++k)
+    for (int c = 0; c < 3; ++c) v[c] += s_part[k][c][lane];
+  const int px = (lane & 1) ? -nx : nx, py = (lane & 4) ? -ny : ny, pz = (lane & 2) ? -nz : nz;
+  int face, sc, tc;
+  if (axis == 0)
+    face = px > 0 ? 0 : 1, sc = px > 0 ? -pz : pz, tc = -py;
+  else if (axis == 1)
+    face = py > 0 ? 2 : 3, sc = px, tc = py > 0 ? pz : -pz;
+  else
+    face = pz > 0 ? 4 : 5, sc = pz > 0 ? px : -px, tc = -py;
+  const T scale = static_cast<T>(p.scale);
+  cube[(static_cast<size_t>(face) * S + (tc + S - 1) / 2) * S + (sc + S - 1) / 2] =
+      make_float4(static_cast<float>(v[0] * scale), static_cast<float>(v[1] * scale), static_cast<float>(v[2] * scale),
+                  1.0f);
+}
+
+// One lookup per sample (a blend grid, folded or not): the polar weights are
+// not split over two levels.
+static int irradiance_one_lookup(int w, int h, int theta, const IrradianceLod& lod) {
+  return fold_grid(w, h, theta, lod).ok || blend_grid(w, h, lod).ok ? 1 : 0;
+}
+
+// The folded grid, then one block per orbit.
+static althea_status launch_irradiance_fold(const float* pyr, const PyramidGeometry& g, const FoldGrid& fg,
+                                            const IrradianceLod& lod, int size, int theta_samples, int phi,
+                                            unsigned flags, float* cube, const float2* theta_tab,
+                                            const float4* phi_tab, float* grid, hipStream_t s) {
+  FoldGridParams q{};
+  q.src.w0 = fg.w0;
+  q.src.h0 = fg.h0;
+  q.src.off0 = g.off[lod.l0];
+  q.src.off1 = g.off[lod.l1];
+  q.src.delta = static_cast<double>(lod.delta);
+  q.blend = fg.blend;
+  q.cols = fg.cols;
+  q.rows = fg.rows;
+  hipLaunchKernelGGL(fold_grid_kernel, dim3(static_cast<unsigned>((8 * fg.nodes + 255) / 256)), dim3(256), 0, s,
+                     reinterpret_cast<const float4*>(pyr), q, grid);
+  const althea_status st = check_launch("fold_grid_kernel");
+  if (st != ALTHEA_OK) return st;
+  const LevelC c0 = make_level(fg.w0, fg.h0, 0);
+  FoldParams p{};
+  p.kx = c0.kx;
+  p.ky = -c0.ky;
+  p.cols = fg.cols;
+  p.rowbytes = static_cast<uint32_t>(kFoldNodeBytes * (fg.cols + 2));
+  p.size = size;
+  p.theta_samples = theta_samples;
+  p.phi_samples = phi;
+  p.theta_steps = (theta_samples + 7) / 8;
+  p.steps = p.theta_steps * ((phi + 7) / 8);
+  p.scale = M_PI / theta_samples / phi;
+  const int half = (size + 1) / 2;
+  const bool f64 = !(flags & ALTHEA_PRECOMPUTE_FP32_SUMS);
+  const size_t tables = sizeof(float4) * static_cast<size_t>(phi) + sizeof(float2) * static_cast<size_t>(theta_samples);
+  const bool lds = tables <= kFoldTableMax;
+  const int variant = (f64 ? 1 : 0) | (fg.blend ? 2 : 0) | (lds ? 4 : 0);
+  auto kernel = variant == 0   ? irradiance_fold_kernel<false, false, false>
+                : variant == 1 ? irradiance_fold_kernel<true, false, false>
+                : variant == 2 ? irradiance_fold_kernel<false, true, false>
+                : variant == 3 ? irradiance_fold_kernel<true, true, false>
+                : variant == 4 ? irradiance_fold_kernel<false, false, true>
+                : variant == 5 ? irradiance_fold_kernel<true, false, true>
+                : variant == 6 ? irradiance_fold_kernel<false, true, true>
+                               : irradiance_fold_kernel<true, true, true>;
+  hipLaunchKernelGGL(kernel, dim3(3 * half * half), dim3(64 * kFoldWaves), lds ? tables : 0, s,
+                     reinterpret_cast<const char*>(grid), theta_tab, phi_tab, p, reinterpret_cast<float4*>(cube));
+  return check_launch("irradiance_fold_kernel");
 }
 
 althea_status launch_irradiance(const float* pyr, int env_w, int env_h, int size, int theta_samples,
@@ -955,8 +1247,14 @@ althea_status launch_irradiance(const float* pyr, int env_w, int env_h, int size
   p.l0 = lod.l0;
   p.l1 = lod.l1;
   p.delta = lod.delta;
+  const int tab = std::max(theta_samples, phi);
+  hipLaunchKernelGGL(irradiance_tables_kernel, dim3((tab + 255) / 256), dim3(256), 0, s, theta_samples, phi, p.delta,
+                     irradiance_one_lookup(env_w, env_h, theta_samples, lod), theta_tab, phi_tab);
+  althea_status st = check_launch("irradiance_tables_kernel");
+  if (st != ALTHEA_OK) return st;
+  const FoldGrid fg = fold_grid(env_w, env_h, theta_samples, lod);
+  if (fg.ok) return launch_irradiance_fold(pyr, g, fg, lod, size, theta_samples, phi, flags, cube, theta_tab, phi_tab, gather, s);
   const BlendGrid bg = blend_grid(env_w, env_h, lod);
-  althea_status st = ALTHEA_OK;
   if (bg.ok) {
     BlendGridParams q{};
     q.w0 = bg.w0;
@@ -989,11 +1287,6 @@ althea_status launch_irradiance(const float* pyr, int env_w, int env_h, int size
     p.lv1 = split_level(env_w, env_h, gg, p.l1);
   }
   p.scale = M_PI / theta_samples / phi;
-  const int n = std::max(theta_samples, phi);
-  hipLaunchKernelGGL(irradiance_tables_kernel, dim3((n + 255) / 256), dim3(256), 0, s, theta_samples, phi, p.delta,
-                     p.blend, theta_tab, phi_tab);
-  st = check_launch("irradiance_tables_kernel");
-  if (st != ALTHEA_OK) return st;
   const dim3 grid((6 * size * size + 3) / 4);
   const char* g4 = reinterpret_cast<const char*>(gather);
   float4* cube4 = reinterpret_cast<float4*>(cube);

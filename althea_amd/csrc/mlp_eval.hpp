@@ -195,13 +195,6 @@ __device__ inline void mlp_stage_weights(MlpSmem& s, const MlpDeviceWeights& w, 
   }
 }
 
-// Orders this wave's LDS writes before its later LDS reads from other lanes.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Log-radiance of this lane's query (d, rough), evaluated for the wave as
 // four 16-sample MFMA tiles (lanes 16t .. 16t+15); a tile none of whose lanes
 // sets `want` is skipped and its lanes get 0.  Every lane of the wave must be

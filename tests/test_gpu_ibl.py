@@ -365,6 +365,29 @@ def test_irradiance_edge_shapes(torch, size, theta):
     assert err.max() < MAX_REL, summary(err)
 
 
+@pytest.mark.parametrize("w,h,size,theta,fp32", [(8, 4, 2, 2, False), (8, 4, 3, 8, False), (16, 8, 1, 6, True),
+                                                  (64, 32, 9, 30, False), (64, 32, 4, 64, True),
+                                                  (128, 512, 7, 20, False), (2048, 4, 4, 1500, False),
+                                                  (256, 128, 1, 2048, False), (256, 128, 1, 2050, False)])
+def test_irradiance_folded_matches_oracle(torch, w, h, size, theta, fp32):
+    """The folded irradiance (even azimuth counts): the smallest level it
+    takes, one level and two, odd and single-texel faces (texels that several
+    sign flips name), FP32 sums, azimuth and polar tables at both sides of
+    the 32 KB that LDS holds; and odd counts beside it on the general kernel,
+    every texel.  Tolerance: the contract (1e-3 for FP32 sums)."""
+    env = aa.synth.env(seed=SEED0 + 17 * w + h, width=w, height=h, sigma=0.5, suns=2, peak_min=10.0, peak_max=20.0,
+                       sun_sigma_deg=15.0)
+    pyr = aa.env_pyramid(torch.from_numpy(env).cuda())
+    ids = np.array([(0, f, x, y) for f in range(6) for y in range(size) for x in range(size)], np.int32)
+    oenv = ol.Env(env)
+    for t in (theta, theta + 1):
+        if int(np.float32(h) * np.float32(t) / np.float32(w)) < 1:
+            continue
+        got = aa.irradiance_cube(pyr, w, h, size, t, fp32_sums=fp32).cpu().numpy()[:, :3]
+        err = rel_err(got, oenv.irradiance_texels(size, ids[:, 1:], t), RADIANCE_FLOOR)
+        assert err.max() < (1e-3 if fp32 else MAX_REL), (t, summary(err))
+
+
 # ------------------------------------------------------------- IBL handle
 def test_ibl_handle_matches_low_level_calls(torch):
     env = _env("config0")
