@@ -1,11 +1,11 @@
 // Batched GGX prefilter: many environment maps of uneven resolution in one
 // persistent launch.  The reference prefilters one map with five sequential
-// dispatches (Src/ImageBasedLighting.cpp:352-402); here every (map, mip,
-// face, tile) of every map is one work item in a list sorted by estimated
-// cost (largest first), and waves of a grid sized to the machine pull items
+// dispatches (Src/ImageBasedLighting.cpp:352-402); here every block of
+// tiles of every mip of every map is one work item in a list sorted by estimated
+// cost (largest first), and blocks of a grid sized to the machine pull items
 // from an atomic counter until the list is exhausted (greedy list scheduling
-// of the longest items first).  Every texel runs prefilter_texel, the same
-// function as the single-map kernel, so batched and single results are
+// of the longest items first).  Every texel runs the single-map
+// kernel's sums (prefilter_pair_sums), so batched and single results are
 // bit-identical.
 //
 // A run replays one hipGraph: the pyramid chains of all maps, the sample
@@ -28,74 +28,43 @@
 
 namespace althea {
 
-struct BatchMap {
-  const char* pyr;   // source pyramid (bytes)
-  const char* gpyr;  // its gather copy (bytes)
-  float4* cube;      // output cube, [mip][face][y][x]
-  int size;          // face size at mip 0
-  int table_set;     // sample-table set of this map's source extent
-  int level_base;    // first LevelC / GatherLevel of this map
-  int chunk;         // table entries per partial sum, as the single-map kernel cuts this map's sums
-};
+// Blocks pull items (x map, y mip, z block of the mip) from a counter; a block
+// stages a map's levels in LDS when its map changes or its partial sums have
+// taken their place.  Blocks of 8 waves: two a CU at the default 16 waves (four
+// a SIMD, both levels of a sample in flight), so one stages or combines beside
+// another's samples.  12 maps of 1024, 512 and 256 texels width in one run: 2.91
+// ms gathering from global memory, 2.05 here; blocks of 16 waves 2.22, of 4 with
+// a whole tile to a wave 2.63; a level at a time at six waves a SIMD 2.27.
+constexpr int kBatchWaves = 8;
 
-// Work item: map, mip, face, tile index within the face.
-struct BatchParams {
-  int num_tiles;
-  int samples;
-  int mips;
-  int tile_w, tile_h;
-};
+template <bool kF64Sums, int kTW, int kTH>
+__global__ __launch_bounds__(64 * kBatchWaves) __attribute__((amdgpu_waves_per_eu(4))) void prefilter_batch_kernel(
+    const PrefilterMap* __restrict__ maps, const int4* __restrict__ work, int* counter, int items) {
+  extern __shared__ float s_levels[];
+  __shared__ int s_item;
+  char* lds = reinterpret_cast<char*>(s_levels);
+  int staged = -1;
+  for (;;) {
+    __syncthreads();  // the last item's reads of s_item and of LDS are done
+    if (threadIdx.x == 0) s_item = atomicAdd(counter, 1);
+    __syncthreads();
+    const int item = __builtin_amdgcn_readfirstlane(s_item);
+    if (item >= items) break;  // every block reaches this once the list is drained
+    const int4 w = work[item];
+    const PrefilterMap& p = maps[w.x];
+    const bool rough = w.y > 0 && p.mips > 1;
+    if (rough && staged != w.x) {
+      prefilter_stage<kBatchWaves>(p, lds);
+      __syncthreads();
+      staged = w.x;
+    }
+    prefilter_block<kF64Sums, kTW, kTH, kBatchWaves, true, true>(p, w.y, w.z, lds);
+    if (rough && p.split > 1) staged = -1;
+  }
+}
 
 __global__ void batch_reset_kernel(int* counter) {
   if (threadIdx.x == 0) counter[0] = 0;
-}
-
-template <bool kF64Sums, int kTW, int kTH>
-__global__ __launch_bounds__(256) void prefilter_batch_kernel(const BatchMap* __restrict__ maps,
-                                                              const LevelC* __restrict__ levels,
-                                                              const GatherLevel* __restrict__ glevels,
-                                                              const GgxEntry* __restrict__ tables,
-                                                              const int* __restrict__ counts,
-                                                              const double* __restrict__ wsum,
-                                                              const int4* __restrict__ work, int* counter,
-                                                              const BatchParams p) {
-  static_assert(kTW * kTH == 64, "one wave per tile");
-  const int lane = threadIdx.x & 63;
-  for (;;) {
-    int item = 0;
-    if (lane == 0) item = atomicAdd(counter, 1);
-    item = __builtin_amdgcn_readfirstlane(item);
-    if (item >= p.num_tiles) break;  // every wave reaches this once the list is drained
-    const int4 w = work[item];
-    const BatchMap mp = maps[w.x];
-    const int m = w.y, face = w.z, t = w.w;
-    const int S = max(1, mp.size >> m);
-    const int tpr = (S + kTW - 1) / kTW;
-    const int x = (t % tpr) * kTW + (lane % kTW);
-    const int y = (t / tpr) * kTH + (lane / kTW);
-    const bool active = x < S && y < S;
-    const int set_mip = mp.table_set * p.mips + m;
-    const LevelC* lv = levels + mp.level_base;
-    const auto level = [&](int l) -> const LevelC& { return lv[l]; };
-    float4 out;
-    if (m == 0 || p.mips == 1) {
-      // roughness 0: the mirror lookup, as the single-map kernel
-      out = prefilter_texel_mirror(mp.pyr, level, face, min(x, S - 1), min(y, S - 1), S);
-    } else {
-      const Frame fr = local_to_world(cube_texel_raw_dir(face, min(x, S - 1), min(y, S - 1), S));
-      out = prefilter_texel<kF64Sums>(GatherAcc{mp.gpyr, glevels + mp.level_base},
-                                      tables + static_cast<size_t>(set_mip) * p.samples, counts[set_mip],
-                                      wsum[set_mip], fr, mp.chunk);
-    }
-    if (active) {
-      size_t off = 0;
-      for (int k = 0; k < m; ++k) {
-        const size_t s = static_cast<size_t>(max(1, mp.size >> k));
-        off += 6 * s * s;
-      }
-      mp.cube[off + (static_cast<size_t>(face) * S + y) * S + x] = out;
-    }
-  }
 }
 
 // Source-independent count of kept samples (NdotL > 0) at roughness r: the
@@ -133,12 +102,13 @@ struct althea_prefilter_batch {
   std::vector<int> sizes;
   // Device state.
   std::vector<float*> pyramids;
-  std::vector<float*> gathers;  // gather copies of the pyramids, owned by the batch
   std::vector<float*> cubes;
   bool owns_buffers = true;  // false when the pyramids and cubes belong to IBL handles
-  BatchMap* d_maps = nullptr;
+  PrefilterMap* d_maps = nullptr;
   LevelC* d_levels = nullptr;
-  GatherLevel* d_glevels = nullptr;
+  StagedLevel* d_slevels = nullptr;
+  std::vector<int> waves;  // per map: waves per tile of a rough mip
+  size_t lds_bytes = 0;
   GgxEntry* d_tables = nullptr;
   int* d_counts = nullptr;
   double* d_wsum = nullptr;
@@ -183,10 +153,11 @@ std::vector<int4> build_work(const althea_prefilter_batch* b, int tw, int th, si
   for (int i = 0; i < b->count; ++i)
     for (int m = 0; m < b->mips; ++m) {
       const int S = std::max(1, b->sizes[i] >> m);
-      const int tpr = (S + tw - 1) / tw, tpc = (S + th - 1) / th;
+      const bool mirror = m == 0 || b->mips == 1;
       const int active = std::min(S, tw) * std::min(S, th);
-      for (int f = 0; f < 6; ++f)
-        for (int t = 0; t < tpr * tpc; ++t) items.push_back({mip_cost[m] * active, make_int4(i, m, f, t)});
+      const double cost = mip_cost[m] * active * (mirror ? kBatchWaves : 2.0 * kBatchWaves / b->waves[i]);
+      const int blocks = prefilter_blocks(b->sizes[i], b->mips, m, b->waves[i], tw, th, kBatchWaves);
+      for (int k = 0; k < blocks; ++k) items.push_back({cost, make_int4(i, m, k, 0)});
       tex += 6ull * S * S;
     }
   std::stable_sort(items.begin(), items.end(), [](const Item& a, const Item& c) { return a.cost > c.cost; });
@@ -207,23 +178,13 @@ althea_status upload_work(althea_prefilter_batch* b) {
 }
 
 template <bool kF64>
-void launch_persistent_t(const althea_prefilter_batch* b, int shape, int blocks, const int4* work, int tiles,
+void launch_persistent_t(const althea_prefilter_batch* b, int shape, int blocks, const int4* work, int items,
                          hipStream_t s) {
-  BatchParams p{tiles, b->samples, b->mips, kShapes[shape].w, kShapes[shape].h};
-  switch (shape) {
-    case 0:
-      hipLaunchKernelGGL((prefilter_batch_kernel<kF64, 8, 8>), dim3(blocks), dim3(256), 0, s, b->d_maps, b->d_levels,
-                         b->d_glevels, b->d_tables, b->d_counts, b->d_wsum, work, b->d_counter, p);
-      break;
-    case 1:
-      hipLaunchKernelGGL((prefilter_batch_kernel<kF64, 16, 4>), dim3(blocks), dim3(256), 0, s, b->d_maps,
-                         b->d_levels, b->d_glevels, b->d_tables, b->d_counts, b->d_wsum, work, b->d_counter, p);
-      break;
-    default:
-      hipLaunchKernelGGL((prefilter_batch_kernel<kF64, 4, 16>), dim3(blocks), dim3(256), 0, s, b->d_maps,
-                         b->d_levels, b->d_glevels, b->d_tables, b->d_counts, b->d_wsum, work, b->d_counter, p);
-      break;
-  }
+  auto kernel = shape == 0   ? prefilter_batch_kernel<kF64, 8, 8>
+                : shape == 1 ? prefilter_batch_kernel<kF64, 16, 4>
+                             : prefilter_batch_kernel<kF64, 4, 16>;
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kBatchWaves), b->lds_bytes, s, b->d_maps, work, b->d_counter,
+                     items);
 }
 
 // Counter reset + persistent kernel over `tiles` items of `work`.
@@ -232,7 +193,7 @@ althea_status launch_persistent(const althea_prefilter_batch* b, int shape, int 
   hipLaunchKernelGGL(batch_reset_kernel, dim3(1), dim3(64), 0, s, b->d_counter);
   althea_status st = check_launch("batch_reset_kernel");
   if (st != ALTHEA_OK) return st;
-  const int blocks = std::max(1, b->cus * waves_per_cu / 4);
+  const int blocks = std::max(1, b->cus * waves_per_cu / kBatchWaves);
   if (b->flags & ALTHEA_PRECOMPUTE_FP32_SUMS)
     launch_persistent_t<false>(b, shape, blocks, work, tiles, s);
   else
@@ -240,14 +201,11 @@ althea_status launch_persistent(const althea_prefilter_batch* b, int shape, int 
   return check_launch("prefilter_batch_kernel");
 }
 
-// Pyramids of all maps with their gather copies, and the sample tables of
-// every source extent.
+// Pyramids of all maps and the sample tables of every source extent.
 althea_status launch_prep(const althea_prefilter_batch* b, hipStream_t s) {
   for (int i = 0; i < b->count; ++i) {
     const int w = b->envs[i].width, h = b->envs[i].height;
     althea_status st = launch_pyramid(b->envs[i].rgba, w, h, b->pyramids[i], s);
-    if (st != ALTHEA_OK) return st;
-    st = launch_gather(b->pyramids[i], w, h, gather_geometry(w, h, 0, althea_env_levels(w, h) - 1), b->gathers[i], s);
     if (st != ALTHEA_OK) return st;
   }
   for (size_t k = 0; k < b->extents.size(); ++k) {
@@ -324,12 +282,14 @@ static althea_status batch_create(const althea_env_view* envs, int count, const 
     return fail(ALTHEA_ERROR_HIP);
   }
   std::map<std::pair<int, int>, int> set_of;
-  std::vector<BatchMap> maps(count);
+  std::vector<int> sets_of(count);
+
+  std::vector<PrefilterMap> maps(count);
   std::vector<LevelC> levels(static_cast<size_t>(count) * kMaxLevels);
-  std::vector<GatherLevel> glevels(static_cast<size_t>(count) * kMaxLevels);
+  std::vector<StagedLevel> slevels(static_cast<size_t>(count) * kMaxLevels);
   b->pyramids.assign(count, nullptr);
-  b->gathers.assign(count, nullptr);
   b->cubes.assign(count, nullptr);
+  b->waves.assign(count, 1);
   b->owns_buffers = ext_pyramids == nullptr;
   for (int i = 0; i < count; ++i) {
     const auto ext = std::make_pair(envs[i].width, envs[i].height);
@@ -347,22 +307,26 @@ static althea_status batch_create(const althea_env_view* envs, int count, const 
       set_error("prefilter_batch_create: out of device memory at map %d", i);
       return fail(ALTHEA_ERROR_OUT_OF_MEMORY);
     }
+    sets_of[i] = it->second;
     const int w = envs[i].width, h = envs[i].height;
-    const GatherGeometry gg = gather_geometry(w, h, 0, althea_env_levels(w, h) - 1);
-    if (hipMalloc(&b->gathers[i], 16 * gg.texels) != hipSuccess) {
-      set_error("prefilter_batch_create: out of device memory at map %d", i);
-      return fail(ALTHEA_ERROR_OUT_OF_MEMORY);
-    }
+    PrefilterMap& p = maps[i];
+    size_t staged = 0;
     pyramid_levels(w, h, &levels[static_cast<size_t>(i) * kMaxLevels]);
-    gather_levels(w, h, gg, &glevels[static_cast<size_t>(i) * kMaxLevels]);
-    maps[i] = BatchMap{reinterpret_cast<const char*>(b->pyramids[i]), reinterpret_cast<const char*>(b->gathers[i]),
-                       reinterpret_cast<float4*>(b->cubes[i]), face_sizes[i], it->second, i * kMaxLevels, 0};
-    prefilter_split(face_sizes[i], mips, samples, maps[i].chunk);
+    p.first = staged_levels(w, h, mips, samples, &slevels[static_cast<size_t>(i) * kMaxLevels], &staged);
+    p.levels = althea_env_levels(w, h);
+    p.pyr = reinterpret_cast<const char*>(b->pyramids[i]);
+    p.cube = reinterpret_cast<float4*>(b->cubes[i]);
+    p.size = face_sizes[i];
+    p.mips = mips;
+    p.samples = samples;
+    p.split = prefilter_split(face_sizes[i], mips, samples, p.chunk);
+    p.waves = b->waves[i] = std::min(p.split, kBatchWaves);
+    if (mips > 1) b->lds_bytes = std::max(b->lds_bytes, prefilter_lds_bytes(staged, p.split, p.waves, kBatchWaves));
   }
   const size_t sets = b->extents.size() * mips;
-  if (hipMalloc(&b->d_maps, sizeof(BatchMap) * count) != hipSuccess ||
+  if (hipMalloc(&b->d_maps, sizeof(PrefilterMap) * count) != hipSuccess ||
       hipMalloc(&b->d_levels, sizeof(LevelC) * levels.size()) != hipSuccess ||
-      hipMalloc(&b->d_glevels, sizeof(GatherLevel) * glevels.size()) != hipSuccess ||
+      hipMalloc(&b->d_slevels, sizeof(StagedLevel) * slevels.size()) != hipSuccess ||
       hipMalloc(&b->d_tables, sizeof(GgxEntry) * sets * samples) != hipSuccess ||
       hipMalloc(&b->d_counts, sizeof(int) * sets) != hipSuccess ||
       hipMalloc(&b->d_wsum, sizeof(double) * sets) != hipSuccess ||
@@ -371,9 +335,17 @@ static althea_status batch_create(const althea_env_view* envs, int count, const 
     set_error("prefilter_batch_create: out of device memory");
     return fail(ALTHEA_ERROR_OUT_OF_MEMORY);
   }
-  if (hipMemcpy(b->d_maps, maps.data(), sizeof(BatchMap) * count, hipMemcpyHostToDevice) != hipSuccess ||
+  for (int i = 0; i < count; ++i) {
+    const size_t set = static_cast<size_t>(sets_of[i]) * mips;
+    maps[i].tables = b->d_tables + set * samples;
+    maps[i].counts = b->d_counts + set;
+    maps[i].wsum = b->d_wsum + set;
+    maps[i].lv = b->d_levels + static_cast<size_t>(i) * kMaxLevels;
+    maps[i].slv = b->d_slevels + static_cast<size_t>(i) * kMaxLevels;
+  }
+  if (hipMemcpy(b->d_maps, maps.data(), sizeof(PrefilterMap) * count, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(b->d_levels, levels.data(), sizeof(LevelC) * levels.size(), hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(b->d_glevels, glevels.data(), sizeof(GatherLevel) * glevels.size(), hipMemcpyHostToDevice) !=
+      hipMemcpy(b->d_slevels, slevels.data(), sizeof(StagedLevel) * slevels.size(), hipMemcpyHostToDevice) !=
           hipSuccess ||
       hipStreamCreateWithFlags(&b->capture, hipStreamNonBlocking) != hipSuccess) {
     set_error("prefilter_batch_create: upload failed");
@@ -400,10 +372,9 @@ althea_status althea_prefilter_batch_destroy(althea_prefilter_batch* b) {
     for (float* p : b->pyramids) (void)hipFree(p);
     for (float* p : b->cubes) (void)hipFree(p);
   }
-  for (float* p : b->gathers) (void)hipFree(p);
   (void)hipFree(b->d_maps);
   (void)hipFree(b->d_levels);
-  (void)hipFree(b->d_glevels);
+  (void)hipFree(b->d_slevels);
   (void)hipFree(b->d_tables);
   (void)hipFree(b->d_counts);
   (void)hipFree(b->d_wsum);

@@ -156,31 +156,50 @@ __device__ __forceinline__ int cvt_floor(float x) {
   return r;
 }
 
-// The four REPEAT texels around (yaw, pitch) on a level (the FP32 texel
-// coordinate is one FMA from the angle) and the bilinear fractions.  Rows
-// wrap through the level's texel mask: the row after the last is row 0.
+// Texel coordinate of (yaw, pitch) on a level, one FMA per axis from the
+// angle: the lower texel and the bilinear fractions.
+struct TexelCoord {
+  int ix, iy;
+  float ax, ay;
+};
+template <class Level>
+__device__ __forceinline__ TexelCoord texel_coord(const Level& c, float yaw, float pitch) {
+  const float x = fmaf(yaw, c.kx, c.cx), y = fmaf(pitch, c.ky, c.cy);
+  return {cvt_floor(x), cvt_floor(y), __builtin_amdgcn_fractf(x), __builtin_amdgcn_fractf(y)};
+}
+
+// The four REPEAT texels around a coordinate and the bilinear fractions.
+// Rows wrap through the level's texel mask: the row after the last is row 0.
 struct LevelTaps {
   f3 t00, t10, t01, t11;
   float ax, ay;
 };
-__device__ __forceinline__ LevelTaps level_taps(const char* __restrict__ pyr_bytes, const LevelC& c, float yaw,
-                                                float pitch) {
-  const float x = fmaf(yaw, c.kx, c.cx), y = fmaf(pitch, c.ky, c.cy);
-  LevelTaps t;
-  t.ax = __builtin_amdgcn_fractf(x);
-  t.ay = __builtin_amdgcn_fractf(y);
-  const int ix = cvt_floor(x), iy = cvt_floor(y);
+__device__ __forceinline__ void level_texels(const char* __restrict__ pyr_bytes, const LevelC& c, int ix, int iy,
+                                             LevelTaps& t) {
   const uint32_t x0 = static_cast<uint32_t>(ix) & c.wmask, x1 = static_cast<uint32_t>(ix + 1) & c.wmask;
   const uint32_t lmask = ((c.hmask + 1u) << c.wshift) - 1u;  // texels of the level - 1 (wave-uniform)
   const uint32_t r0 = (static_cast<uint32_t>(iy) << c.wshift) & lmask;
   const uint32_t r1 = (r0 + c.wmask + 1u) & lmask;
   // The level offset goes into the (wave-uniform, scalar) base address.
   const char* lvl = pyr_bytes + (static_cast<size_t>(c.off) << 4);
-  auto ld = [&](uint32_t i) { return xyz(*reinterpret_cast<const float4*>(lvl + (i << 4))); };
+  typedef const __attribute__((address_space(1))) char gchar;
+  typedef const __attribute__((address_space(1))) float gfloat;
+  auto ld = [&](uint32_t i) {
+    gfloat* q = (gfloat*)((gchar*)lvl + (i << 4));
+    return mk(q[0], q[1], q[2]);
+  };
   t.t00 = ld(r0 + x0);
   t.t10 = ld(r0 + x1);
   t.t01 = ld(r1 + x0);
   t.t11 = ld(r1 + x1);
+}
+__device__ __forceinline__ LevelTaps level_taps(const char* __restrict__ pyr_bytes, const LevelC& c, float yaw,
+                                                float pitch) {
+  const TexelCoord q = texel_coord(c, yaw, pitch);
+  LevelTaps t;
+  t.ax = q.ax;
+  t.ay = q.ay;
+  level_texels(pyr_bytes, c, q.ix, q.iy, t);
   return t;
 }
 
@@ -192,72 +211,68 @@ __device__ __forceinline__ f3 level_bilinear(const char* __restrict__ pyr_bytes,
   return lerp3(top, bot, t.ay);
 }
 
-// Gather copy of a pyramid level, read by the precompute's sample loops:
-// the level with its REPEAT neighbours around it, (w + 2) x (h + 2) texels,
-// padded (r, c) = level((r - 1) mod h, (c - 1) mod w).  The texel coordinate
-// is formed exactly as level_taps forms it; with the wrap stored, a tap pair
-// sits at one byte offset and offset + 16, the next row at + rowbytes.
-struct GatherLevel {
+// A pyramid level staged in LDS: its texels' RGB, 12 bytes each, with their
+// REPEAT neighbours around them ((w + 2) x (h + 2), padded (r, c) =
+// level((r - 1) mod h, (c - 1) mod w)), so a cell's two rows are two offsets
+// and a row's tap pair 24 contiguous bytes (three ds_read2_b32).
+struct StagedLevel {
   float kx, cx, ky, cy;  // x = yaw kx + cx, y = pitch ky + cy (as LevelC)
-  uint32_t rowbytes;     // (w + 2) * 16
-  uint32_t off;          // first texel of the padded level, float4 units
-  uint32_t pad0, pad1;
+  uint32_t rowbytes;     // (w + 2) * 12
+  uint32_t off;          // byte offset of the level in LDS
+  uint32_t half;         // bytes of half a turn, (w / 2) * 12
+  uint32_t mirror;       // 2 off + h rowbytes + 12 w: cell (ix, iy) at o has its image
+                         // under (yaw, pitch) -> (-yaw, -pitch) at mirror - o
 };
 
-__host__ inline GatherLevel make_gather_level(int w, int h, uint32_t off) {
+__host__ inline StagedLevel make_staged_level(int w, int h, uint32_t off) {
   const LevelC c = make_level(w, h, 0);
-  GatherLevel g{};
+  StagedLevel g{};
   g.kx = c.kx;
   g.cx = c.cx;
   g.ky = c.ky;
   g.cy = c.cy;
-  g.rowbytes = static_cast<uint32_t>(w + 2) * 16u;
+  g.rowbytes = static_cast<uint32_t>(w + 2) * 12u;
   g.off = off;
+  g.half = static_cast<uint32_t>(w / 2) * 12u;
+  g.mirror = 2u * off + static_cast<uint32_t>(h) * g.rowbytes + 12u * static_cast<uint32_t>(w);
   return g;
 }
 
-// level_taps on a gather level: the same four texels and fractions.  The
-// angles are those of equirect_angles, |yaw| <= float(pi) and |pitch| <=
-// float(pi) / 2, so x lies in [-0.5, w - 0.5] and y in [-0.5, h - 0.5] up to
-// a rounding of w * 5e-8 texel: floor(x) + 1 is in [0, w] and floor(y) + 1
-// in [0, h], inside the padded level (levels are at most 2^15 wide; a NaN
-// angle converts to index 0).
-__device__ __forceinline__ LevelTaps gather_taps(const char* __restrict__ gpyr_bytes, const GatherLevel& g, float yaw,
-                                                 float pitch) {
-  const float x = fmaf(yaw, g.kx, g.cx), y = fmaf(pitch, g.ky, g.cy);
-  LevelTaps t;
-  t.ax = __builtin_amdgcn_fractf(x);
-  t.ay = __builtin_amdgcn_fractf(y);
-  const int ix = cvt_floor(x), iy = cvt_floor(y);
-  // (iy + 1) rowbytes + (ix + 1) 16 as iy * rowbytes + (16 ix + rowbytes + 16):
-  // one shift-add and one signed 24-bit multiply-add (iy >= -1, rowbytes < 2^20).
+// Byte offset of cell (ix, iy).  The angles are those of equirect_angles,
+// |yaw| <= float(pi) and |pitch| <= float(pi) / 2, so x lies in [-0.5, w - 0.5]
+// and y in [-0.5, h - 0.5] up to a rounding of w * 5e-8 texel: ix is in
+// [-1, w - 1] and iy in [-1, h - 1], inside the padded level (a NaN angle
+// converts to index 0).
+__device__ __forceinline__ uint32_t staged_offset(const StagedLevel& g, int ix, int iy) {
+  // off + iy rowbytes + (12 ix + rowbytes + 12): two signed 24-bit multiply-adds.
   const int rb = static_cast<int>(g.rowbytes);
   int col, o;
-  asm("v_lshl_add_u32 %0, %1, 4, %2" : "=v"(col) : "v"(ix), "s"(rb + 16));
+  asm("v_mad_i32_i24 %0, %1, 12, %2" : "=v"(col) : "v"(ix), "s"(rb + 12 + static_cast<int>(g.off)));
   asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(o) : "v"(iy), "s"(rb), "v"(col));
-  const uint32_t o0 = static_cast<uint32_t>(o);
-  const uint32_t o1 = o0 + g.rowbytes;
-  // Global address space: the loads take the scalar base plus a 32-bit lane
-  // offset and the immediate +16, also where the base comes from memory.
-  typedef const __attribute__((address_space(1))) char gchar;
-  typedef const __attribute__((address_space(1))) float gfloat;
-  gchar* lvl = (gchar*)gpyr_bytes + (static_cast<size_t>(g.off) << 4);
-  gfloat* r0 = (gfloat*)(lvl + o0);
-  gfloat* r1 = (gfloat*)(lvl + o1);
-  t.t00 = mk(r0[0], r0[1], r0[2]);
-  t.t10 = mk(r0[4], r0[5], r0[6]);
-  t.t01 = mk(r1[0], r1[1], r1[2]);
-  t.t11 = mk(r1[4], r1[5], r1[6]);
-  return t;
+  return static_cast<uint32_t>(o);
 }
 
-// Split gather copy: the padded texels of a gather level as an RG plane
+__device__ __forceinline__ void staged_texels(const char* lds, const StagedLevel& g, uint32_t o, LevelTaps& t) {
+  // Explicit address space: beside a branch that reads global memory the
+  // loads would otherwise be merged into flat ones.
+  typedef const __attribute__((address_space(3))) char lchar;
+  typedef const __attribute__((address_space(3))) float lfloat;
+  lfloat* r0 = (lfloat*)((lchar*)lds + o);
+  lfloat* r1 = (lfloat*)((lchar*)lds + (o + g.rowbytes));
+  t.t00 = mk(r0[0], r0[1], r0[2]);
+  t.t10 = mk(r0[3], r0[4], r0[5]);
+  t.t01 = mk(r1[0], r1[1], r1[2]);
+  t.t11 = mk(r1[3], r1[4], r1[5]);
+}
+
+// Split gather copy: the texels of a level with its REPEAT neighbours around
+// it, (w + 2) x (h + 2), padded (r, c) = level((r - 1) mod h, (c - 1) mod w), as an RG plane
 // (float2 per texel) and a B plane (float per texel).  A tap pair's red and
 // green are one 16-byte load and its blue one 8-byte load, so a wave whose
 // lanes read a patch of neighbouring texels touches about half the cache
 // lines that the float4 copy's two 12-byte loads per pair touch.
 struct SplitLevel {
-  float kx, cx, ky, cy;  // as GatherLevel
+  float kx, cx, ky, cy;  // as LevelC
   uint32_t rowbytes;     // (w + 2) * 8, one row of the RG plane
   uint32_t rg;           // byte offset of the level's RG plane
   uint32_t b;            // byte offset of the level's B plane
@@ -293,7 +308,7 @@ __device__ __forceinline__ LevelTaps split_taps_at(const char* __restrict__ base
   return t;
 }
 
-// gather_taps on a split level: the same four texels and fractions.
+// level_taps on a split level: the same four texels and fractions.
 __device__ __forceinline__ LevelTaps split_taps(const char* __restrict__ base, const SplitLevel& g, float yaw,
                                                 float pitch) {
   const float x = fmaf(yaw, g.kx, g.cx), y = fmaf(pitch, g.ky, g.cy);
@@ -325,33 +340,29 @@ __device__ __forceinline__ int blend_cell(float x0, float& t) {
 // acc += w * bilinear in weight form: the four texel weights carry w, so a
 // sample's two source levels (w = its weight times 1 - delta and times
 // delta) add straight into the running sums.  w (1 - a) is one FMA.
+struct TapWeights {
+  float w00, w10, w01, w11;
+};
+__device__ __forceinline__ TapWeights tap_weights(float ax, float ay, float w) {
+  const float wy1 = ay * w, wy0 = fmaf(-ay, w, w);
+  return {fmaf(-ax, wy0, wy0), ax * wy0, fmaf(-ax, wy1, wy1), ax * wy1};
+}
+__device__ __forceinline__ void taps_acc(const LevelTaps& t, const TapWeights& w, float& ar, float& ag, float& ab) {
+  ar = fmaf(t.t00.x, w.w00, ar);
+  ag = fmaf(t.t00.y, w.w00, ag);
+  ab = fmaf(t.t00.z, w.w00, ab);
+  ar = fmaf(t.t10.x, w.w10, ar);
+  ag = fmaf(t.t10.y, w.w10, ag);
+  ab = fmaf(t.t10.z, w.w10, ab);
+  ar = fmaf(t.t01.x, w.w01, ar);
+  ag = fmaf(t.t01.y, w.w01, ag);
+  ab = fmaf(t.t01.z, w.w01, ab);
+  ar = fmaf(t.t11.x, w.w11, ar);
+  ag = fmaf(t.t11.y, w.w11, ag);
+  ab = fmaf(t.t11.z, w.w11, ab);
+}
 __device__ __forceinline__ void taps_acc(const LevelTaps& t, float w, float& ar, float& ag, float& ab) {
-  const float wy1 = t.ay * w, wy0 = fmaf(-t.ay, w, w);
-  const float w10 = t.ax * wy0, w00 = fmaf(-t.ax, wy0, wy0);
-  const float w11 = t.ax * wy1, w01 = fmaf(-t.ax, wy1, wy1);
-  ar = fmaf(t.t00.x, w00, ar);
-  ag = fmaf(t.t00.y, w00, ag);
-  ab = fmaf(t.t00.z, w00, ab);
-  ar = fmaf(t.t10.x, w10, ar);
-  ag = fmaf(t.t10.y, w10, ag);
-  ab = fmaf(t.t10.z, w10, ab);
-  ar = fmaf(t.t01.x, w01, ar);
-  ag = fmaf(t.t01.y, w01, ag);
-  ab = fmaf(t.t01.z, w01, ab);
-  ar = fmaf(t.t11.x, w11, ar);
-  ag = fmaf(t.t11.y, w11, ag);
-  ab = fmaf(t.t11.z, w11, ab);
-}
-
-__device__ __forceinline__ void level_bilinear_acc(const char* __restrict__ pyr_bytes, const LevelC& c, float yaw,
-                                                   float pitch, float w, float& ar, float& ag, float& ab) {
-  taps_acc(level_taps(pyr_bytes, c, yaw, pitch), w, ar, ag, ab);
-}
-
-__device__ __forceinline__ void gather_bilinear_acc(const char* __restrict__ gpyr_bytes, const GatherLevel& g,
-                                                    float yaw, float pitch, float w, float& ar, float& ag,
-                                                    float& ab) {
-  taps_acc(gather_taps(gpyr_bytes, g, yaw, pitch), w, ar, ag, ab);
+  taps_acc(t, tap_weights(t.ax, t.ay, w), ar, ag, ab);
 }
 
 __device__ __forceinline__ void split_bilinear_acc(const char* __restrict__ base, const SplitLevel& g, float yaw,

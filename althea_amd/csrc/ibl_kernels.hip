@@ -214,120 +214,67 @@ __global__ __launch_bounds__(kTableThreads) void ggx_table_kernel(TableParams p,
 
 // ------------------------------------------------------------ prefilter
 struct PrefilterParams {
-  LevelC lv[kMaxLevels];        // source pyramid levels
-  GatherLevel glv[kMaxLevels];  // the same levels in the gather copy
-  CubeMips cube;
-  int samples;
-  int chunk;                        // table entries per partial sum (prefilter_sums)
+  LevelC lv[kMaxLevels];
+  StagedLevel slv[kMaxLevels];
+  PrefilterMap map;  // lv and slv set by the kernel
   int block_start[kMaxLevels + 1];  // blocks before each mip
 };
 
 constexpr int kPrefilterTile = 8;
 
-// kGather: the sample loop reads the padded gather copy `gpyr`; otherwise the
-// pyramid (bit-identical sums, more address arithmetic per lookup).
-// kSplit waves per block.  A rough mip's block is one 8x8 tile whose table
-// is cut into chunks of p.chunk entries, wave k summing chunk k; wave 0 adds
-// the partials in chunk order (prefilter_sums: the bits of one pass).  A
-// roughness-0 block holds kSplit tiles, one per wave.  kSplit > 1 fills the
-// GPU when the rough mips have few tiles (a 128^2 cube: 510 tiles, half a
-// wave per SIMD).
-template <bool kF64Sums, bool kGather, int kSplit>
-__global__ __launch_bounds__(64 * kSplit) void prefilter_cube_kernel(const char* __restrict__ pyr,
-                                                                     const char* __restrict__ gpyr,
-                                                                     const GgxEntry* __restrict__ tables,
-                                                                     const int* __restrict__ counts,
-                                                                     const double* __restrict__ wsum,
-                                                                     const PrefilterParams p,
-                                                                     float4* __restrict__ cube) {
+// 16 waves a block where a tile's table is cut into 16 chunks (few tiles: one
+// block a CU, four waves a SIMD), else 8, held to six waves a SIMD (three
+// blocks of at most 52 KB of LDS a CU, so one block's staging and last waves
+// run beside another's samples): 512^2 x 6 cube 0.95 ms, against 1.09 at four
+// waves a SIMD.
+constexpr int kPrefilterWide = 16, kPrefilterNarrow = 8;
+
+template <bool kF64Sums, int kWaves>
+__device__ __forceinline__ void prefilter_cube(const PrefilterParams& p, float* s_levels) {
   const int b = blockIdx.x;
   int m = 0;
-  while (m + 1 < p.cube.mips && b >= p.block_start[m + 1]) ++m;
-  const int S = max(1, p.cube.size >> m);
-  const int tpf = (S + kPrefilterTile - 1) / kPrefilterTile;
-  const auto level = [&](int l) -> const LevelC& { return p.lv[l]; };
-  const bool mirror = m == 0 || p.cube.mips == 1;  // roughness m / (mips - 1) == 0 (block-uniform)
-  if (kSplit == 1) {
-    const int local = b - p.block_start[m];
-    const int face = local / (tpf * tpf);
-    const int t = local - face * tpf * tpf;
-    const int x = (t % tpf) * kPrefilterTile + (threadIdx.x & 7);
-    const int y = (t / tpf) * kPrefilterTile + (threadIdx.x >> 3);
-    const bool active = x < S && y < S;
-    float4 out;
-    if (mirror) {
-      // the mirror lookup
-      out = prefilter_texel_mirror(pyr, level, face, min(x, S - 1), min(y, S - 1), S);
-    } else {
-      const Frame fr = local_to_world(cube_texel_raw_dir(face, min(x, S - 1), min(y, S - 1), S));
-      const GgxEntry* __restrict__ tab = tables + static_cast<size_t>(m) * p.samples;
-      if (kGather)
-        out = prefilter_value<kF64Sums>(prefilter_sums_whole<kF64Sums>(GatherAcc{gpyr, p.glv}, tab, 0, counts[m], fr),
-                                        wsum[m]);
-      else
-        out = prefilter_value<kF64Sums>(prefilter_sums_whole<kF64Sums>(PyramidAcc{pyr, p.lv}, tab, 0, counts[m], fr),
-                                        wsum[m]);
-    }
-    if (active) cube[p.cube.off[m] + (static_cast<size_t>(face) * S + y) * S + x] = out;
-    return;
+  while (m + 1 < p.map.mips && b >= p.block_start[m + 1]) ++m;
+  PrefilterMap map = p.map;
+  map.lv = p.lv;
+  map.slv = p.slv;
+  char* lds = reinterpret_cast<char*>(s_levels);
+  if (m > 0) {
+    prefilter_stage<kWaves>(map, lds);
+    __syncthreads();
   }
-  using T = typename PrefilterSums<kF64Sums>::T;
-  __shared__ T s_part[kSplit][4][64];
-  const int tiles = 6 * tpf * tpf;
-  const int wave = static_cast<int>(threadIdx.x >> 6), lane = static_cast<int>(threadIdx.x & 63);
-  const int local = mirror ? (b - p.block_start[m]) * kSplit + wave : b - p.block_start[m];
-  const int lt = min(local, tiles - 1);
-  const int face = lt / (tpf * tpf);
-  const int t = lt - face * tpf * tpf;
-  const int x = (t % tpf) * kPrefilterTile + (lane & 7);
-  const int y = (t / tpf) * kPrefilterTile + (lane >> 3);
-  const bool active = local < tiles && x < S && y < S;
-  const size_t dst = p.cube.off[m] + (static_cast<size_t>(face) * S + min(y, S - 1)) * S + min(x, S - 1);
-  if (mirror) {
-    const float4 out = prefilter_texel_mirror(pyr, level, face, min(x, S - 1), min(y, S - 1), S);
-    if (active) cube[dst] = out;
-    return;
-  }
-  const Frame fr = local_to_world(cube_texel_raw_dir(face, min(x, S - 1), min(y, S - 1), S));
-  const GgxEntry* __restrict__ tab = tables + static_cast<size_t>(m) * p.samples;
-  const int count = counts[m];
-  const int lo = min(count, wave * p.chunk), hi = min(count, lo + p.chunk);
-  // A wave's range lies inside one chunk: its sums are one pass.
-  const PrefilterSums<kF64Sums> part =
-      kGather ? prefilter_sums_whole<kF64Sums>(GatherAcc{gpyr, p.glv}, tab, lo, hi, fr)
-              : prefilter_sums_whole<kF64Sums>(PyramidAcc{pyr, p.lv}, tab, lo, hi, fr);
-  s_part[wave][0][lane] = part.r;
-  s_part[wave][1][lane] = part.g;
-  s_part[wave][2][lane] = part.b;
-  s_part[wave][3][lane] = static_cast<T>(part.w);
-  __syncthreads();
-  if (wave == 0) {
-    PrefilterSums<kF64Sums> tot;
-    for (int k = 0; k < kSplit; ++k) {
-      tot.r += s_part[k][0][lane];
-      tot.g += s_part[k][1][lane];
-      tot.b += s_part[k][2][lane];
-      tot.w += static_cast<float>(s_part[k][3][lane]);
-    }
-    if (active) cube[dst] = prefilter_value<kF64Sums>(tot, wsum[m]);
-  }
+  prefilter_block<kF64Sums, kPrefilterTile, kPrefilterTile, kWaves, kWaves == kPrefilterWide, false>(
+      map, m, b - p.block_start[m], lds);
 }
 
-// Waves per block of the single-map prefilter and the table entries per
-// partial sum: the rough mips' tiles times the waves reach 4096 (four waves
-// per SIMD) with at most 8 waves and 64 entries per chunk; chunks are
-// multiples of the 32-entry FP32 blocks.  One wave: a chunk longer than any
-// table.  The batched kernel cuts each map's sums the same way.
+template <bool kF64Sums>
+__global__ __launch_bounds__(64 * kPrefilterWide) void prefilter_wide_kernel(const PrefilterParams p) {
+  extern __shared__ float s_levels[];
+  prefilter_cube<kF64Sums, kPrefilterWide>(p, s_levels);
+}
+
+template <bool kF64Sums>
+__global__ __launch_bounds__(64 * kPrefilterNarrow) __attribute__((amdgpu_waves_per_eu(6))) void prefilter_cube_kernel(
+    const PrefilterParams p) {
+  extern __shared__ float s_levels[];
+  prefilter_cube<kF64Sums, kPrefilterNarrow>(p, s_levels);
+}
+
+// Chunks of a rough mip's table: doubled while the pairs of tiles times the
+// chunks stay under 4096 waves (to 16), or to 8 while they stay under 32 768
+// (finer blocks level the last round, the roughest tiles having half the kept
+// samples of the smoothest), as long as a chunk keeps 32 entries.  Chunks are
+// multiples of the 32-entry FP32 blocks; one chunk is longer than any table.
+// The batched kernel cuts each map's sums the same way.
 int prefilter_split(int size, int mips, int samples, int& chunk) {
   long long rough = 0;
   for (int m = 1; m < mips; ++m) {
     const int S = std::max(1, size >> m);
     const int tpf = (S + kPrefilterTile - 1) / kPrefilterTile;
-    rough += 6ll * tpf * tpf;
+    rough += 3ll * tpf * tpf;
   }
   int k = 1;
-  while (k < 8 && rough > 0 && rough * k < 4096 && samples / (2 * k) >= 64) k *= 2;
-  chunk = k == 1 ? (1 << 30) : ((samples + k - 1) / k + 31) / 32 * 32;
+  while (k < kPrefilterMaxSplit && rough > 0 && rough * k < (k < 8 ? 32768 : 4096) && samples / (2 * k) >= kBlockSums) k *= 2;
+  chunk = k == 1 ? (1 << 30) : ((samples + k - 1) / k + kBlockSums - 1) / kBlockSums * kBlockSums;
   return k;
 }
 
@@ -338,10 +285,56 @@ void pyramid_levels(int w, int h, LevelC* out) {
   for (int l = 0; l < g.levels; ++l) out[l] = make_level(g.w[l], g.h[l], g.off[l]);
 }
 
-// ------------------------------------------------------------ gather copy
+// ------------------------------------------------------------ staged levels
+// The lowest source level the sample tables name: the source LOD grows with
+// roughness and away from the lobe's centre, so it is that of sample 0 (the
+// half vector N) at the lowest sampled roughness, 1 / (mips - 1); a margin of
+// 1e-4 level covers the device's rounding.
+static int prefilter_first_level(int w, int h, int mips, int samples) {
+  const double rough = mips > 1 ? 1.0 / (mips - 1) : 1.0, a2 = rough * rough;
+  const double pdf = 1.0 / (M_PI * a2 * (4.0 + 0.00001));
+  const double sa_texel = 4.0 * M_PI / (6.0 * static_cast<double>(w) * h);
+  const double lod = 0.5 * std::log2(1.0 / (samples * pdf + 0.0001) / sa_texel);
+  return std::min(std::max(static_cast<int>(std::floor(lod - 1e-4)), 0), althea_env_levels(w, h) - 1);
+}
+
+// The levels of a map that a prefilter block stages in LDS: the coarsest ones,
+// as many as the tables name and kStagedMaxBytes holds (from 64 x 32 on for a
+// 2:1 source, 38 KB; three blocks a CU).  At 1024 samples the lobes of roughness
+// 1/4 and up read finer levels for a seventh of their samples or less, whatever
+// the source's extent; staging 128 x 64 too (140 KB, one block a CU) measured
+// 1.21 ms against 0.95 on the 512^2 x 6 cube.
+constexpr size_t kStagedMaxBytes = 52 * 1024;
+
+int staged_levels(int w, int h, int mips, int samples, StagedLevel* out, size_t* bytes) {
+  const PyramidGeometry g = pyramid_geometry(w, h);
+  size_t total = 0;
+  int first = g.levels;
+  const int lowest = prefilter_first_level(w, h, mips, samples);
+  while (first > lowest) {
+    const size_t level = 12 * static_cast<size_t>(g.w[first - 1] + 2) * (g.h[first - 1] + 2);
+    if (total + level > kStagedMaxBytes) break;
+    --first;
+    out[first] = make_staged_level(g.w[first], g.h[first], static_cast<uint32_t>(total));
+    total += level;
+  }
+  *bytes = total;
+  return first;
+}
+
+size_t prefilter_lds_bytes(size_t staged, int split, int waves, int block_waves) {
+  return std::max(staged, split > 1 ? sizeof(double) * kPrefilterPart * split * (block_waves / waves) : size_t{0});
+}
+
+// ------------------------------------------------------ split gather copy
 // Levels first..last of a pyramid, each padded with its REPEAT neighbours
-// ((w + 2) x (h + 2) texels, GatherLevel), concatenated from texel 0.
-GatherGeometry gather_geometry(int w, int h, int first, int last) {
+// ((w + 2) x (h + 2) texels, SplitLevel), concatenated from texel 0.
+struct GatherGeometry {
+  int first, last;
+  uint32_t off[kMaxLevels];
+  size_t texels;
+};
+static GatherGeometry gather_geometry(int w, int h, int first, int last) {
   const PyramidGeometry g = pyramid_geometry(w, h);
   GatherGeometry out{};
   out.first = first;
@@ -353,16 +346,6 @@ GatherGeometry gather_geometry(int w, int h, int first, int last) {
   }
   out.texels = total;
   return out;
-}
-
-size_t gather_bytes(int w, int h, int first, int last) {
-  if (w <= 0 || h <= 0) return 0;
-  return align256(16 * gather_geometry(w, h, first, last).texels);
-}
-
-void gather_levels(int w, int h, const GatherGeometry& gg, GatherLevel* out) {
-  const PyramidGeometry g = pyramid_geometry(w, h);
-  for (int l = gg.first; l <= gg.last; ++l) out[l] = make_gather_level(g.w[l], g.h[l], gg.off[l]);
 }
 
 struct PadParams {
@@ -377,12 +360,12 @@ struct PadParams {
 // aligned.
 static size_t split_plane_texels(const GatherGeometry& gg) { return (gg.texels + 63) & ~static_cast<size_t>(63); }
 
-size_t split_gather_bytes(int w, int h, int first, int last) {
+static size_t split_gather_bytes(int w, int h, int first, int last) {
   if (w <= 0 || h <= 0) return 0;
   return 12 * split_plane_texels(gather_geometry(w, h, first, last));
 }
 
-SplitLevel split_level(int w, int h, const GatherGeometry& gg, int l) {
+static SplitLevel split_level(int w, int h, const GatherGeometry& gg, int l) {
   const PyramidGeometry g = pyramid_geometry(w, h);
   const LevelC c = make_level(g.w[l], g.h[l], 0);
   SplitLevel s{};
@@ -396,12 +379,10 @@ SplitLevel split_level(int w, int h, const GatherGeometry& gg, int l) {
   return s;
 }
 
-// One thread per gather texel: padded (r, c) of level l is the pyramid texel
-// ((r - 1) mod h, (c - 1) mod w).  kSplit writes it as the split copy's RG
-// and B planes (plane_texels apart) instead of one float4.
-template <bool kSplit>
+// One thread per padded texel: padded (r, c) of level l is the pyramid texel
+// ((r - 1) mod h, (c - 1) mod w), into the RG and B planes (plane_texels apart).
 __global__ __launch_bounds__(256) void gather_pad_kernel(const float4* __restrict__ pyr, const PadParams p,
-                                                         float4* __restrict__ gpyr, size_t plane_texels) {
+                                                         float2* __restrict__ rg, size_t plane_texels) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
   if (i >= p.dst[p.last + 1]) return;
   int l = p.first;
@@ -413,16 +394,12 @@ __global__ __launch_bounds__(256) void gather_pad_kernel(const float4* __restric
   const int sr = r == 0 ? h - 1 : (r == h + 1 ? 0 : r - 1);
   const int sc = c == 0 ? w - 1 : (c == w + 1 ? 0 : c - 1);
   const float4 v = pyr[p.src[l] + static_cast<size_t>(sr) * w + sc];
-  if (kSplit) {
-    reinterpret_cast<float2*>(gpyr)[i] = make_float2(v.x, v.y);
-    reinterpret_cast<float*>(reinterpret_cast<float2*>(gpyr) + plane_texels)[i] = v.z;
-  } else {
-    gpyr[i] = v;
-  }
+  rg[i] = make_float2(v.x, v.y);
+  reinterpret_cast<float*>(rg + plane_texels)[i] = v.z;
 }
 
-static althea_status launch_gather_as(const float* pyr, int w, int h, const GatherGeometry& gg, float* gpyr,
-                                      bool split, hipStream_t s) {
+static althea_status launch_split_gather(const float* pyr, int w, int h, const GatherGeometry& gg, float* gpyr,
+                                         hipStream_t s) {
   const PyramidGeometry g = pyramid_geometry(w, h);
   PadParams p{};
   p.first = gg.first;
@@ -435,22 +412,9 @@ static althea_status launch_gather_as(const float* pyr, int w, int h, const Gath
   }
   p.dst[gg.last + 1] = static_cast<uint32_t>(gg.texels);
   const uint32_t blocks = static_cast<uint32_t>((gg.texels + 255) / 256);
-  if (split)
-    hipLaunchKernelGGL(gather_pad_kernel<true>, dim3(blocks), dim3(256), 0, s, reinterpret_cast<const float4*>(pyr),
-                       p, reinterpret_cast<float4*>(gpyr), split_plane_texels(gg));
-  else
-    hipLaunchKernelGGL(gather_pad_kernel<false>, dim3(blocks), dim3(256), 0, s, reinterpret_cast<const float4*>(pyr),
-                       p, reinterpret_cast<float4*>(gpyr), size_t{0});
+  hipLaunchKernelGGL(gather_pad_kernel, dim3(blocks), dim3(256), 0, s, reinterpret_cast<const float4*>(pyr), p,
+                     reinterpret_cast<float2*>(gpyr), split_plane_texels(gg));
   return check_launch("gather_pad_kernel");
-}
-
-althea_status launch_gather(const float* pyr, int w, int h, const GatherGeometry& gg, float* gpyr, hipStream_t s) {
-  return launch_gather_as(pyr, w, h, gg, gpyr, false, s);
-}
-
-althea_status launch_split_gather(const float* pyr, int w, int h, const GatherGeometry& gg, float* gpyr,
-                                  hipStream_t s) {
-  return launch_gather_as(pyr, w, h, gg, gpyr, true, s);
 }
 
 static CubeMips cube_mips_of(int size, int mips) {
@@ -478,10 +442,8 @@ size_t prefilter_table_bytes(int mips, int samples) {
          align256(sizeof(double) * mips) + align256(sizeof(float) * mips);
 }
 
-// The sample tables, then the gather copy of every level.
-size_t prefilter_workspace_bytes(int env_w, int env_h, int, int mips, int samples) {
-  return prefilter_table_bytes(mips, samples) + gather_bytes(env_w, env_h, 0, althea_env_levels(env_w, env_h) - 1);
-}
+// The sample tables.
+size_t prefilter_workspace_bytes(int, int, int, int mips, int samples) { return prefilter_table_bytes(mips, samples); }
 
 // ------------------------------------------- allocation-free prefilter
 // The sample tables of althea_prefilter_cube_noalloc: a fixed device array,
@@ -518,23 +480,16 @@ static althea_status prefilter_scratch(void** out) {
 // Every table entry, count and weight sum the prefilter reads is written by
 // the table kernel of the same call before the texel kernel runs, so nothing
 // left in the array by an earlier call is read and nothing needs clearing.
-static althea_status prefilter_cube_tables_in(const float* pyr, int env_w, int env_h, int size, int mips,
-                                              int samples, unsigned flags, float* cube, void* workspace,
-                                              float* gather, hipStream_t s);
-
 althea_status launch_prefilter_cube_noalloc(const float* pyr, int env_w, int env_h, int size, int mips,
                                             int samples, unsigned flags, float* cube, hipStream_t s) {
   void* ws = nullptr;
   althea_status st = prefilter_scratch(&ws);
   if (st != ALTHEA_OK) return st;
-  return prefilter_cube_tables_in(pyr, env_w, env_h, size, mips, samples, flags, cube, ws, nullptr, s);
+  return launch_prefilter_cube(pyr, env_w, env_h, size, mips, samples, flags, cube, ws, s);
 }
 
-// Tables in `workspace`; the sample loop reads the gather copy `gather` when
-// one is given (written here first), else the pyramid.
-static althea_status prefilter_cube_tables_in(const float* pyr, int env_w, int env_h, int size, int mips,
-                                              int samples, unsigned flags, float* cube, void* workspace,
-                                              float* gather, hipStream_t s) {
+althea_status launch_prefilter_cube(const float* pyr, int env_w, int env_h, int size, int mips, int samples,
+                                    unsigned flags, float* cube, void* workspace, hipStream_t s) {
   char* ws = static_cast<char*>(workspace);
   GgxEntry* tables = reinterpret_cast<GgxEntry*>(ws);
   ws += align256(sizeof(GgxEntry) * static_cast<size_t>(mips) * samples);
@@ -549,54 +504,29 @@ static althea_status prefilter_cube_tables_in(const float* pyr, int env_w, int e
 
   PrefilterParams p{};
   pyramid_levels(env_w, env_h, p.lv);
-  if (gather) {
-    const GatherGeometry gg = gather_geometry(env_w, env_h, 0, althea_env_levels(env_w, env_h) - 1);
-    st = launch_gather(pyr, env_w, env_h, gg, gather, s);
-    if (st != ALTHEA_OK) return st;
-    gather_levels(env_w, env_h, gg, p.glv);
-  }
-  p.cube = cube_mips_of(size, mips);
-  p.samples = samples;
-  const int split = prefilter_split(size, mips, samples, p.chunk);
-  int blocks = 0;
-  for (int m = 0; m < mips; ++m) {
-    p.block_start[m] = blocks;
-    int S = std::max(1, size >> m);
-    int tpf = (S + kPrefilterTile - 1) / kPrefilterTile;
-    const int tiles = 6 * tpf * tpf;
-    blocks += (m == 0 || mips == 1) ? (tiles + split - 1) / split : tiles;
-  }
-  p.block_start[mips] = blocks;
-  const char* pyr_b = reinterpret_cast<const char*>(pyr);
-  const char* g_b = reinterpret_cast<const char*>(gather);
-  float4* cube4 = reinterpret_cast<float4*>(cube);
+  size_t staged = 0;
+  p.map.first = staged_levels(env_w, env_h, mips, samples, p.slv, &staged);
+  p.map.levels = althea_env_levels(env_w, env_h);
+  p.map.pyr = reinterpret_cast<const char*>(pyr);
+  p.map.cube = reinterpret_cast<float4*>(cube);
+  p.map.tables = tables;
+  p.map.counts = counts;
+  p.map.wsum = wsum;
+  p.map.size = size;
+  p.map.mips = mips;
+  p.map.samples = samples;
+  p.map.split = p.map.waves = prefilter_split(size, mips, samples, p.map.chunk);
+  const bool wide = p.map.waves > kPrefilterNarrow;
+  const int waves = wide ? kPrefilterWide : kPrefilterNarrow;
+  for (int m = 0; m < mips; ++m)
+    p.block_start[m + 1] = p.block_start[m] + prefilter_blocks(size, mips, m, p.map.waves, kPrefilterTile,
+                                                               kPrefilterTile, waves);
   const bool f64 = !(flags & ALTHEA_PRECOMPUTE_FP32_SUMS);
-  const int variant = (f64 ? 1 : 0) | (gather ? 2 : 0);
-  switch (split) {
-#define ALTHEA_PREFILTER_LAUNCH(k)                                                                                   \
-  case k: {                                                                                                          \
-    auto kernel = variant == 3   ? prefilter_cube_kernel<true, true, k>                                              \
-                  : variant == 1 ? prefilter_cube_kernel<true, false, k>                                             \
-                  : variant == 2 ? prefilter_cube_kernel<false, true, k>                                             \
-                                 : prefilter_cube_kernel<false, false, k>;                                           \
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * k), 0, s, pyr_b, g_b, tables, counts, wsum, p, cube4);        \
-    break;                                                                                                           \
-  }
-    ALTHEA_PREFILTER_LAUNCH(1)
-    ALTHEA_PREFILTER_LAUNCH(2)
-    ALTHEA_PREFILTER_LAUNCH(4)
-    ALTHEA_PREFILTER_LAUNCH(8)
-#undef ALTHEA_PREFILTER_LAUNCH
-    default:
-      break;
-  }
+  auto kernel = wide ? (f64 ? prefilter_wide_kernel<true> : prefilter_wide_kernel<false>)
+                     : (f64 ? prefilter_cube_kernel<true> : prefilter_cube_kernel<false>);
+  hipLaunchKernelGGL(kernel, dim3(p.block_start[mips]), dim3(64 * waves),
+                     mips > 1 ? prefilter_lds_bytes(staged, p.map.split, p.map.waves, waves) : 0, s, p);
   return check_launch("prefilter_cube_kernel");
-}
-
-althea_status launch_prefilter_cube(const float* pyr, int env_w, int env_h, int size, int mips, int samples,
-                                    unsigned flags, float* cube, void* workspace, hipStream_t s) {
-  float* gather = reinterpret_cast<float*>(static_cast<char*>(workspace) + prefilter_table_bytes(mips, samples));
-  return prefilter_cube_tables_in(pyr, env_w, env_h, size, mips, samples, flags, cube, workspace, gather, s);
 }
 
 // -------------------------------------------------------- point prefilter
@@ -1071,7 +1001,7 @@ __global__ __launch_bounds__(64 * kFoldWaves) void irradiance_fold_kernel(const 
                                                                           const float4* __restrict__ phi_glob,
                                                                           const FoldParams p,
                                                                           float4* __restrict__ cube) {
-  using T = typename PrefilterSums<kF64Sums>::T;
+  using T = typename std::conditional<kF64Sums, double, float>::type;
   typedef const __attribute__((address_space(1))) char gchar;
   typedef const __attribute__((address_space(1))) float gfloat;
   extern __shared__ float4 s_tab[];  // the polar rows, then the azimuth rows (kLds)

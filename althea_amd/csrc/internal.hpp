@@ -56,32 +56,17 @@ althea_status launch_cube_border(const float* cube, int size, int mips, float* b
 
 struct GgxEntry;
 struct LevelC;
-struct GatherLevel;
+struct StagedLevel;
 
-// Gather copy of pyramid levels first..last (each padded with its REPEAT
-// neighbours, (w + 2) x (h + 2) texels, concatenated): texel offset of each
-// level and the total.
-struct GatherGeometry {
-  int first, last;
-  uint32_t off[16];
-  size_t texels;
-};
-GatherGeometry gather_geometry(int w, int h, int first, int last);
-size_t gather_bytes(int w, int h, int first, int last);
-void gather_levels(int w, int h, const GatherGeometry& gg, GatherLevel* out);
-althea_status launch_gather(const float* pyr, int w, int h, const GatherGeometry& gg, float* gpyr, hipStream_t s);
-// The split form (SplitLevel): the same padded texels as an RG plane of
-// float2 followed by a B plane of floats.
-struct SplitLevel;
-size_t split_gather_bytes(int w, int h, int first, int last);
-SplitLevel split_level(int w, int h, const GatherGeometry& gg, int l);
-althea_status launch_split_gather(const float* pyr, int w, int h, const GatherGeometry& gg, float* gpyr,
-                                  hipStream_t s);
+// The pyramid levels a prefilter block stages in LDS: their layouts, the first
+// of them and their bytes; and the LDS of a block of `block_waves` waves with
+// `waves` waves per tile, its table cut into `split` chunks.
+int staged_levels(int w, int h, int mips, int samples, StagedLevel* out, size_t* bytes);
+size_t prefilter_lds_bytes(size_t staged, int split, int waves, int block_waves);
 // Sample tables of a prefilter (the part of its workspace the allocation-free
 // entry point keeps in the library's fixed array).
 size_t prefilter_table_bytes(int mips, int samples);
-// Waves per block of the single-map prefilter for a cube and the table
-// entries per partial sum (`chunk`), which the batched kernel uses too.
+// Chunks that a cube's rough mips cut their tables into, and entries per chunk.
 int prefilter_split(int size, int mips, int samples, int& chunk);
 
 // Kernel launchers (ibl_kernels.hip).

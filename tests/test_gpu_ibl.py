@@ -231,12 +231,12 @@ def test_prefilter_edge_shapes(torch, size, mips, samples):
 
 @pytest.mark.parametrize("size,mips,samples", [(64, 5, 128), (256, 5, 1024), (128, 5, 1000), (64, 4, 100)])
 def test_prefilter_sample_split_shapes(torch, size, mips, samples):
-    """Cubes whose rough mips have few 8x8 tiles split each tile's sample
-    table over a block of waves (chunks of a multiple of 32 entries, FP64
-    partials added in order), as long as every chunk keeps 64 entries.
-    These shapes take 2 (132 rough tiles, 128 samples), 4 (2 040 tiles),
-    8 (510 tiles; 1 000 samples, so the last chunk is short) and 1 wave
-    (100 samples) per tile."""
+    """Cubes whose rough mips have few pairs of 8x8 tiles split each pair's
+    sample table over a block of waves (chunks of a multiple of 32 entries,
+    FP64 partials added in order), as long as every chunk keeps 32 entries.
+    These shapes take 4 (66 pairs of tiles, 128 samples), 8 (1 020 pairs), 16
+    (255 pairs; 1 000 samples, so the last chunk is short) and 2 waves (100
+    samples) per pair."""
     env = _env("smooth")
     pyr = aa.env_pyramid(torch.from_numpy(env).cuda())
     cube = aa.prefilter_cube(pyr, 512, 256, size, mips, samples).cpu().numpy()
@@ -252,6 +252,32 @@ def test_prefilter_sample_split_shapes(torch, size, mips, samples):
     assert st == _lib.ALTHEA_OK, aa.lib().althea_last_error()
     torch.cuda.synchronize()
     np.testing.assert_array_equal(again.cpu().numpy().view(np.uint32), cube.view(np.uint32))
+
+
+@pytest.mark.parametrize("w,h,size,mips,samples", [(64, 32, 1, 1, 32), (64, 32, 2, 2, 64), (128, 64, 4, 3, 256),
+                                                    (16, 128, 8, 4, 512), (1024, 512, 16, 5, 20000),
+                                                    (512, 512, 8, 3, 4096), (2, 1, 4, 3, 64)])
+def test_prefilter_pairs_match_oracle(torch, w, h, size, mips, samples):
+    """Every texel of small cubes: a texel and its partner on the opposite face
+    share their samples (single-texel faces, tiles on the Z faces' diagonals),
+    from levels staged in LDS and, at many samples or a square source, from
+    finer levels in the pyramid.  The batch's 8-wave blocks (two chunks of a
+    16-chunk table to a wave) write the single map's bits."""
+    from althea_amd.batch import PrefilterBatch
+
+    env = aa.synth.env(seed=SEED0 + 3 * w + h, width=w, height=h, sigma=0.5, suns=2, peak_min=10.0, peak_max=20.0,
+                       sun_sigma_deg=15.0)
+    dev = torch.from_numpy(env).cuda()
+    cube = aa.prefilter_cube(aa.env_pyramid(dev), w, h, size, mips, samples).cpu().numpy()
+    ids = np.array([(m, f, x, y) for m in range(mips) for f in range(6) for y in range(size >> m)
+                    for x in range(size >> m)], np.int32)
+    err = rel_err(cube_gather(cube, size, ids), ol.Env(env).prefilter_texels(size, mips, samples, ids)[:, :3],
+                  RADIANCE_FLOOR)
+    assert err.max() < MAX_REL, summary(err)
+    b = PrefilterBatch([dev, dev], [size, size], mips=mips, samples=samples)
+    b.run()
+    for k in range(2):
+        np.testing.assert_array_equal(b.cube(k).cpu().numpy().view(np.uint32), cube.view(np.uint32))
 
 
 def test_prefilter_points_match_oracle(env_case, torch):
@@ -285,9 +311,9 @@ def test_prefilter_points_agree_with_cube_texels(torch):
 @pytest.mark.parametrize("w,h", [(1, 1), (2, 1), (1, 4), (4, 16), (16, 4), (64, 8)])
 def test_gather_copy_edge_sources(torch, w, h):
     """Sources down to one texel and of either aspect.  The prefilter and the
-    irradiance read a padded copy of each level (its REPEAT neighbours stored
-    around it); both match the oracle, and the allocation-free prefilter, which
-    reads the pyramid itself, writes the same bits."""
+    irradiance read padded copies of the levels (their REPEAT neighbours stored
+    around them); both match the oracle, and the allocation-free prefilter
+    writes the same bits."""
     env = aa.synth.env(seed=SEED0 + 131 * w + h, width=w, height=h, sigma=0.5, suns=1, peak_min=10.0,
                        peak_max=10.0, sun_sigma_deg=20.0)
     pyr = aa.env_pyramid(torch.from_numpy(env).cuda())
