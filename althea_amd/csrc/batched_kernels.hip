@@ -54,7 +54,7 @@ __global__ __launch_bounds__(64 * kBatchWaves) __attribute__((amdgpu_waves_per_e
     const PrefilterMap& p = maps[w.x];
     const bool rough = w.y > 0 && p.mips > 1;
     if (rough && staged != w.x) {
-      prefilter_stage<kBatchWaves>(p, lds);
+      stage_levels<kBatchWaves>(p.pyr, p.lv, p.slv, p.first, p.levels, lds);
       __syncthreads();
       staged = w.x;
     }
@@ -312,7 +312,8 @@ static althea_status batch_create(const althea_env_view* envs, int count, const 
     PrefilterMap& p = maps[i];
     size_t staged = 0;
     pyramid_levels(w, h, &levels[static_cast<size_t>(i) * kMaxLevels]);
-    p.first = staged_levels(w, h, mips, samples, &slevels[static_cast<size_t>(i) * kMaxLevels], &staged);
+    p.first = staged_levels(w, h, prefilter_first_level(w, h, mips, samples),
+                           &slevels[static_cast<size_t>(i) * kMaxLevels], &staged);
     p.levels = althea_env_levels(w, h);
     p.pyr = reinterpret_cast<const char*>(b->pyramids[i]);
     p.cube = reinterpret_cast<float4*>(b->cubes[i]);

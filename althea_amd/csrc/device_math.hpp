@@ -193,24 +193,6 @@ __device__ __forceinline__ void level_texels(const char* __restrict__ pyr_bytes,
   t.t01 = ld(r1 + x0);
   t.t11 = ld(r1 + x1);
 }
-__device__ __forceinline__ LevelTaps level_taps(const char* __restrict__ pyr_bytes, const LevelC& c, float yaw,
-                                                float pitch) {
-  const TexelCoord q = texel_coord(c, yaw, pitch);
-  LevelTaps t;
-  t.ax = q.ax;
-  t.ay = q.ay;
-  level_texels(pyr_bytes, c, q.ix, q.iy, t);
-  return t;
-}
-
-// Bilinear REPEAT fetch of (yaw, pitch) from a level.
-__device__ __forceinline__ f3 level_bilinear(const char* __restrict__ pyr_bytes, const LevelC& c, float yaw,
-                                             float pitch) {
-  const LevelTaps t = level_taps(pyr_bytes, c, yaw, pitch);
-  const f3 top = lerp3(t.t00, t.t10, t.ax), bot = lerp3(t.t01, t.t11, t.ax);
-  return lerp3(top, bot, t.ay);
-}
-
 // A pyramid level staged in LDS: its texels' RGB, 12 bytes each, with their
 // REPEAT neighbours around them ((w + 2) x (h + 2), padded (r, c) =
 // level((r - 1) mod h, (c - 1) mod w)), so a cell's two rows are two offsets
@@ -308,7 +290,7 @@ __device__ __forceinline__ LevelTaps split_taps_at(const char* __restrict__ base
   return t;
 }
 
-// level_taps on a split level: the same four texels and fractions.
+// The four texels of a split level around (yaw, pitch) and the fractions.
 __device__ __forceinline__ LevelTaps split_taps(const char* __restrict__ base, const SplitLevel& g, float yaw,
                                                 float pitch) {
   const float x = fmaf(yaw, g.kx, g.cx), y = fmaf(pitch, g.ky, g.cy);

@@ -239,7 +239,7 @@ __device__ __forceinline__ void prefilter_cube(const PrefilterParams& p, float* 
   map.slv = p.slv;
   char* lds = reinterpret_cast<char*>(s_levels);
   if (m > 0) {
-    prefilter_stage<kWaves>(map, lds);
+    stage_levels<kWaves>(map.pyr, map.lv, map.slv, map.first, map.levels, lds);
     __syncthreads();
   }
   prefilter_block<kF64Sums, kPrefilterTile, kPrefilterTile, kWaves, kWaves == kPrefilterWide, false>(
@@ -290,7 +290,7 @@ void pyramid_levels(int w, int h, LevelC* out) {
 // roughness and away from the lobe's centre, so it is that of sample 0 (the
 // half vector N) at the lowest sampled roughness, 1 / (mips - 1); a margin of
 // 1e-4 level covers the device's rounding.
-static int prefilter_first_level(int w, int h, int mips, int samples) {
+int prefilter_first_level(int w, int h, int mips, int samples) {
   const double rough = mips > 1 ? 1.0 / (mips - 1) : 1.0, a2 = rough * rough;
   const double pdf = 1.0 / (M_PI * a2 * (4.0 + 0.00001));
   const double sa_texel = 4.0 * M_PI / (6.0 * static_cast<double>(w) * h);
@@ -299,18 +299,17 @@ static int prefilter_first_level(int w, int h, int mips, int samples) {
 }
 
 // The levels of a map that a prefilter block stages in LDS: the coarsest ones,
-// as many as the tables name and kStagedMaxBytes holds (from 64 x 32 on for a
+// from `lowest` on, as many as kStagedMaxBytes holds (from 64 x 32 on for a
 // 2:1 source, 38 KB; three blocks a CU).  At 1024 samples the lobes of roughness
 // 1/4 and up read finer levels for a seventh of their samples or less, whatever
 // the source's extent; staging 128 x 64 too (140 KB, one block a CU) measured
 // 1.21 ms against 0.95 on the 512^2 x 6 cube.
 constexpr size_t kStagedMaxBytes = 52 * 1024;
 
-int staged_levels(int w, int h, int mips, int samples, StagedLevel* out, size_t* bytes) {
+int staged_levels(int w, int h, int lowest, StagedLevel* out, size_t* bytes) {
   const PyramidGeometry g = pyramid_geometry(w, h);
   size_t total = 0;
   int first = g.levels;
-  const int lowest = prefilter_first_level(w, h, mips, samples);
   while (first > lowest) {
     const size_t level = 12 * static_cast<size_t>(g.w[first - 1] + 2) * (g.h[first - 1] + 2);
     if (total + level > kStagedMaxBytes) break;
@@ -505,7 +504,7 @@ althea_status launch_prefilter_cube(const float* pyr, int env_w, int env_h, int 
   PrefilterParams p{};
   pyramid_levels(env_w, env_h, p.lv);
   size_t staged = 0;
-  p.map.first = staged_levels(env_w, env_h, mips, samples, p.slv, &staged);
+  p.map.first = staged_levels(env_w, env_h, prefilter_first_level(env_w, env_h, mips, samples), p.slv, &staged);
   p.map.levels = althea_env_levels(env_w, env_h);
   p.map.pyr = reinterpret_cast<const char*>(pyr);
   p.map.cube = reinterpret_cast<float4*>(cube);
@@ -530,83 +529,165 @@ althea_status launch_prefilter_cube(const float* pyr, int env_w, int env_h, int 
 }
 
 // -------------------------------------------------------- point prefilter
-// Same estimator at per-lane (direction, roughness): the sample quantities are
-// evaluated per lane in FP32 (sin^2 theta formed without cancellation), sums
-// in FP32 blocks flushed to FP64.
+// Same estimator at a query's (direction, roughness r).  A wave takes a query,
+// its lanes the samples; lane l takes samples l C + t, t = 0..C - 1 (C = n / 64
+// rounded up), so with C a power of two the lanes of a step have radical
+// inverses within 1 / C: nearly one source LOD, spread around a ring of the
+// lobe, and the steps outside the hemisphere are skipped whole.
+//
+// With x2 the radical inverse and den = 1 + (r^2 - 1) x2, the GGX half vector
+// has cos^2 = (1 - x2) / den and sin^2 = r^2 x2 / den, so L in the frame is
+//   (r q cos phi, r q sin phi, 1 - (1 + r^2) x2) / den, q = 2 sqrt(x2 (1 - x2)),
+// whose r-free parts are a table of the sample set, and D = den^2 / (pi r^2):
+// one reciprocal a sample, no square root.  pdf = D cos / (4 cos + 1e-5)
+// (PreFilterEnvMap.comp:155-161) takes D (1/4 - 1e-5 / (16 cos)) with 1 / cos =
+// 1.415 - 0.425 L.z on the kept range, 5e-8 of the pdf.
+//
+// Bound: VALU (about 140 a step).  One lane per query walked its samples alone,
+// 250 VALU each with IEEE roots and quotients, its lookups unrelated to its
+// neighbours': 2^18 queries of 1024 samples from 1024 x 512, 2.06 ms, here 0.91;
+// 1 394 queries of 605 samples, 598 us (a wave's latency of all samples), here
+// 18.  The error against 64 bits went from 2.1e-5 (sin and cos of theta by FP32
+// roots) to 4.8e-7.
 struct PointParams {
   LevelC lv[kMaxLevels];
-  int levels;
-  int samples;
+  StagedLevel slv[kMaxLevels];
+  const char* pyr;
+  int first, levels;
+  int samples, steps;  // steps = ceil(samples / 64)
   int count;
+  int level_off, table_off;  // byte offsets in LDS of the level records and the sample table
   float log2_sa_texel;
 };
 
-// Trilinear lookup with per-lane LOD: level constants from LDS.
-__device__ __forceinline__ f3 lds_trilinear(const char* __restrict__ pyr, const LevelC* s_lv, int levels, float yaw,
-                                            float pitch, float lod) {
-  const float d = fminf(fmaxf(lod, 0.0f), static_cast<float>(levels - 1));
-  const float fl = floorf(d);
-  const int l0 = static_cast<int>(fl);
-  const float delta = d - fl;
-  f3 v = level_bilinear(pyr, s_lv[l0], yaw, pitch);
-  if (delta != 0.0f) v = lerp3(v, level_bilinear(pyr, s_lv[min(l0 + 1, levels - 1)], yaw, pitch), delta);
-  return v;
+// A level's constants as a lane reads them from LDS (its levels are its own).
+struct PointLevel {
+  float kx, cx, ky, cy;
+  uint32_t rowbytes, off;          // staged
+  uint32_t wmask, hmask;
+  uint32_t wshift, src, pad0, pad1;  // pyramid texel offset
+};
+
+// Sample i of n: (q cos phi, q sin phi, x2); x2 = 2 beyond the set (never kept).
+__device__ __forceinline__ f3 point_sample(int i, int n) {
+  if (i >= n) return mk(0.0f, 0.0f, 2.0f);
+  float x1, x2, sp, cp;
+  hammersley(static_cast<uint32_t>(i), static_cast<uint32_t>(n), x1, x2);
+  sincospif(2.0f * x1, &sp, &cp);
+  const float q = 2.0f * sqrtf(x2 * (1.0f - x2));
+  return mk(q * cp, q * sp, x2);
 }
 
-__global__ __launch_bounds__(256) void prefilter_points_kernel(const char* __restrict__ pyr, const PointParams p,
-                                                               const float4* __restrict__ dir_rough,
-                                                               float4* __restrict__ out) {
-  __shared__ LevelC s_lv[kMaxLevels];
-  if (threadIdx.x < kMaxLevels) s_lv[threadIdx.x] = p.lv[threadIdx.x];
-  __syncthreads();
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= p.count) return;
-  const float4 q = dir_rough[i];
-  const Frame fr = local_to_world(mk(q.x, q.y, q.z));
-  const float rough = q.w;
-  const float a2 = rough * rough;
-  const float fn = static_cast<float>(p.samples);
-  const float max_lod = static_cast<float>(p.levels - 1);
-  double ar = 0.0, ag = 0.0, ab = 0.0, aw = 0.0;
-  float sr = 0.0f, sg = 0.0f, sb = 0.0f, sw = 0.0f;
-  for (int s = 0; s < p.samples; ++s) {
-    float x1, x2;
-    hammersley(static_cast<uint32_t>(s), static_cast<uint32_t>(p.samples), x1, x2);
-    const float den = fmaf(a2 - 1.0f, x2, 1.0f);
-    const float cos_t = sqrtf((1.0f - x2) / den);
-    const float sin_t = sqrtf(a2 * x2 / den);
-    float sp, cp;
-    sincospif(2.0f * x1, &sp, &cp);
-    const float hz = cos_t;
-    const float lz = fmaf(2.0f * hz, hz, -1.0f);
-    if (lz > 0.0f) {
-      const float lx = 2.0f * hz * (cp * sin_t), ly = 2.0f * hz * (sp * sin_t);
-      float lod = 0.0f;
-      if (rough != 0.0f) {
-        const float t = fmaf(hz * hz, a2 - 1.0f, 1.0f);
-        const float D = a2 / (kPi * t * t);
-        const float pdf = D * hz / fmaf(4.0f, hz, 0.00001f);
-        lod = 0.5f * (-log2f(fmaf(fn, pdf, 0.0001f)) - p.log2_sa_texel);
-      }
-      lod = fminf(fmaxf(lod, 0.0f), max_lod);
-      f3 L = fr.t * lx + fr.b * ly + fr.n * lz;
-      float yaw, pitch;
-      equirect_angles(L, yaw, pitch);
-      f3 v = lds_trilinear(pyr, s_lv, p.levels, yaw, pitch, lod);
-      sr = fmaf(v.x, lz, sr);
-      sg = fmaf(v.y, lz, sg);
-      sb = fmaf(v.z, lz, sb);
-      sw += lz;
-    }
-    if ((s & (kBlockSums - 1)) == kBlockSums - 1) {
-      ar += sr; ag += sg; ab += sb; aw += sw;
-      sr = sg = sb = sw = 0.0f;
+// Adds w times the bilinear value of level l at (yaw, pitch).
+__device__ __forceinline__ void point_lookup(const char* __restrict__ pyr, const char* lds, const PointLevel& g,
+                                             bool staged, float yaw, float pitch, float w, float s[3]) {
+  const TexelCoord q = texel_coord(g, yaw, pitch);
+  LevelTaps t;
+  if (staged) {
+    // off + (iy + 1) rowbytes + (ix + 1) 12
+    const uint32_t o = g.off + static_cast<uint32_t>(__mul24(q.iy + 1, static_cast<int>(g.rowbytes)) + 12 * (q.ix + 1));
+    StagedLevel sl{};
+    sl.rowbytes = g.rowbytes;
+    staged_texels(lds, sl, o, t);
+  } else {
+    LevelC c{};
+    c.wmask = g.wmask;
+    c.hmask = g.hmask;
+    c.wshift = g.wshift;
+    level_texels(pyr + (static_cast<size_t>(g.src) << 4), c, q.ix, q.iy, t);
+  }
+  taps_acc(t, tap_weights(q.ax, q.ay, w), s[0], s[1], s[2]);
+}
+
+constexpr int kPointWaves = 8;
+constexpr int kPointTableMax = 2048;  // samples whose table stays in LDS (24 KB)
+
+template <bool kTable>
+__global__ __launch_bounds__(64 * kPointWaves) void prefilter_points_kernel(const PointParams p,
+                                                                            const float4* __restrict__ dir_rough,
+                                                                            float* __restrict__ out) {
+  extern __shared__ float s_levels[];
+  char* lds = reinterpret_cast<char*>(s_levels);
+  PointLevel* levels = reinterpret_cast<PointLevel*>(lds + p.level_off);
+  float* table = reinterpret_cast<float*>(lds + p.table_off);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  stage_levels<kPointWaves>(p.pyr, p.lv, p.slv, p.first, p.levels, lds);
+  if (static_cast<int>(threadIdx.x) < p.levels) {
+    const LevelC& c = p.lv[threadIdx.x];
+    const StagedLevel& g = p.slv[threadIdx.x];
+    levels[threadIdx.x] = PointLevel{c.kx, c.cx, c.ky, c.cy, g.rowbytes, g.off, c.wmask, c.hmask, c.wshift, c.off, 0, 0};
+  }
+  if (kTable) {
+    // Step t's lanes side by side.
+    for (int i = threadIdx.x; i < 64 * p.steps; i += 64 * kPointWaves) {
+      const f3 v = point_sample((i & 63) * p.steps + (i >> 6), p.samples);
+      table[3 * i] = v.x, table[3 * i + 1] = v.y, table[3 * i + 2] = v.z;
     }
   }
-  ar += sr; ag += sg; ab += sb; aw += sw;
-  const double inv = 1.0 / aw;
-  out[i] = make_float4(static_cast<float>(ar * inv), static_cast<float>(ag * inv), static_cast<float>(ab * inv),
-                       1.0f);
+  __syncthreads();
+  const float max_lod = static_cast<float>(p.levels - 1);
+  const float half_sa = -0.5f * p.log2_sa_texel;
+  for (int query = static_cast<int>(blockIdx.x) * kPointWaves + wave; query < p.count;
+       query += static_cast<int>(gridDim.x) * kPointWaves) {
+    const float4 q = dir_rough[__builtin_amdgcn_readfirstlane(query)];
+    const Frame fr = local_to_world(mk(q.x, q.y, q.z));
+    const float rough = fabsf(q.w), a2 = rough * rough, a2m1 = a2 - 1.0f, a2p1 = a2 + 1.0f;
+    const float kd = static_cast<float>(p.samples) * kInvPi / a2;  // n D = kd den^2
+    double ar = 0.0, ag = 0.0, ab = 0.0, aw = 0.0;
+    float s[3] = {0.0f, 0.0f, 0.0f}, sw = 0.0f;
+    for (int t = 0; t < p.steps; ++t) {
+      f3 e;
+      if (kTable) {
+        const float* v = table + 3 * (64 * t + lane);
+        e = mk(v[0], v[1], v[2]);
+      } else {
+        e = point_sample(lane * p.steps + t, p.samples);
+      }
+      const float num = fmaf(-e.z, a2p1, 1.0f);
+      if (num > 0.0f) {
+        const float den = fmaf(e.z, a2m1, 1.0f);
+        const float rden = rcp_fast(den);
+        const float lz = num * rden, k = rough * rden;
+        const float lx = e.x * k, ly = e.y * k;
+        float lod = 0.0f;
+        if (rough != 0.0f) {
+          const float f = fmaf(lz, 2.65625e-7f, 0.249999116f);
+          lod = fmaf(__builtin_amdgcn_logf(fmaf(den * den * f, kd, 0.0001f)), -0.5f, half_sa);
+        }
+        lod = fminf(fmaxf(lod, 0.0f), max_lod);
+        const float fl = floorf(lod), delta = lod - fl;
+        const int l0 = static_cast<int>(fl);
+        const f3 L = mk(fmaf(fr.t.x, lx, fmaf(fr.b.x, ly, fr.n.x * lz)), fmaf(fr.t.y, lx, fmaf(fr.b.y, ly, fr.n.y * lz)),
+                        fmaf(fr.t.z, lx, fmaf(fr.b.z, ly, fr.n.z * lz)));
+        float yaw, pitch;
+        equirect_angles(L, yaw, pitch);
+        point_lookup(p.pyr, lds, levels[l0], l0 >= p.first, yaw, pitch, fmaf(-delta, lz, lz), s);
+        if (delta != 0.0f) {
+          const int l1 = min(l0 + 1, p.levels - 1);
+          point_lookup(p.pyr, lds, levels[l1], l1 >= p.first, yaw, pitch, delta * lz, s);
+        }
+        sw += lz;
+      }
+      if ((t & (kBlockSums - 1)) == kBlockSums - 1) {
+        ar += s[0], ag += s[1], ab += s[2], aw += sw;
+        s[0] = s[1] = s[2] = sw = 0.0f;
+      }
+    }
+    ar += s[0], ag += s[1], ab += s[2], aw += sw;
+    // Four sums over 64 lanes: halves exchange two sums, quarters one, then one
+    // value is summed over 16 lanes (lane 0: r, 16: g, 32: b, 48: w).
+    const bool hi = lane & 32, hi2 = lane & 16;
+    double k0 = hi ? ab : ar, k1 = hi ? aw : ag;
+    k0 += __shfl_xor(hi ? ar : ab, 32, 64);
+    k1 += __shfl_xor(hi ? ag : aw, 32, 64);
+    double v = hi2 ? k1 : k0;
+    v += __shfl_xor(hi2 ? k0 : k1, 16, 64);
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    const double w = __shfl(v, 48, 64);
+    if ((lane & 15) == 0)
+      out[4 * static_cast<size_t>(query) + (lane >> 4)] = lane == 48 ? 1.0f : static_cast<float>(v / w);
+  }
 }
 
 althea_status launch_prefilter_points(const float* pyr, int env_w, int env_h, int samples, const float* dir_rough,
@@ -614,13 +695,26 @@ althea_status launch_prefilter_points(const float* pyr, int env_w, int env_h, in
   if (count == 0) return ALTHEA_OK;
   PointParams p{};
   pyramid_levels(env_w, env_h, p.lv);
+  size_t staged = 0;
+  p.first = staged_levels(env_w, env_h, 0, p.slv, &staged);
   p.levels = althea_env_levels(env_w, env_h);
+  p.pyr = reinterpret_cast<const char*>(pyr);
   p.samples = samples;
+  p.steps = (samples + 63) / 64;
   p.count = count;
+  p.level_off = static_cast<int>((staged + 15) & ~size_t{15});
+  p.table_off = p.level_off + static_cast<int>(sizeof(PointLevel)) * kMaxLevels;
   p.log2_sa_texel = static_cast<float>(std::log2(4.0 * M_PI / (6.0 * static_cast<double>(env_w) * env_h)));
-  hipLaunchKernelGGL(prefilter_points_kernel, dim3((count + 255) / 256), dim3(256), 0, s,
-                     reinterpret_cast<const char*>(pyr), p, reinterpret_cast<const float4*>(dir_rough),
-                     reinterpret_cast<float4*>(out));
+  const bool table = samples <= kPointTableMax;
+  const size_t lds = p.table_off + (table ? sizeof(float) * 3 * 64 * p.steps : size_t{0});
+  // Three blocks a CU walk the queries; the staging and the table are per block.
+  int dev = 0, cus = 256;
+  ALTHEA_TRY_HIP(hipGetDevice(&dev));
+  ALTHEA_TRY_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  const int blocks = std::min((count + kPointWaves - 1) / kPointWaves, 3 * cus);
+  auto kernel = table ? prefilter_points_kernel<true> : prefilter_points_kernel<false>;
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kPointWaves), lds, s, p,
+                     reinterpret_cast<const float4*>(dir_rough), out);
   return check_launch("prefilter_points_kernel");
 }
 

@@ -58,10 +58,11 @@ struct GgxEntry;
 struct LevelC;
 struct StagedLevel;
 
-// The pyramid levels a prefilter block stages in LDS: their layouts, the first
-// of them and their bytes; and the LDS of a block of `block_waves` waves with
+// The lowest pyramid level a prefilter's tables name; the levels from `lowest` on
+// that a block stages in LDS: their layouts, the first of them and their bytes; and the LDS of a block of `block_waves` waves with
 // `waves` waves per tile, its table cut into `split` chunks.
-int staged_levels(int w, int h, int mips, int samples, StagedLevel* out, size_t* bytes);
+int prefilter_first_level(int w, int h, int mips, int samples);
+int staged_levels(int w, int h, int lowest, StagedLevel* out, size_t* bytes);
 size_t prefilter_lds_bytes(size_t staged, int split, int waves, int block_waves);
 // Sample tables of a prefilter (the part of its workspace the allocation-free
 // entry point keeps in the library's fixed array).

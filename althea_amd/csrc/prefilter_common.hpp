@@ -227,15 +227,16 @@ struct PrefilterMap {
 constexpr int kPrefilterMaxSplit = 16;
 constexpr int kPrefilterPart = 6 * 64 + 1;  // sums of a chunk: a tile's six, the weight
 
-// LDS texels of levels first..levels - 1 of the map, block-cooperative; the
-// caller synchronises the block.
+// LDS texels of levels first..levels - 1, block-cooperative; the caller
+// synchronises the block.
 template <int kWaves>
-__device__ __forceinline__ void prefilter_stage(const PrefilterMap& p, char* lds) {
-  for (int l = p.first; l < p.levels; ++l) {
-    const LevelC& c = p.lv[l];
+__device__ __forceinline__ void stage_levels(const char* __restrict__ pyr, const LevelC* __restrict__ lv,
+                                             const StagedLevel* __restrict__ slv, int first, int levels, char* lds) {
+  for (int l = first; l < levels; ++l) {
+    const LevelC& c = lv[l];
     const int w = static_cast<int>(c.wmask) + 1, h = static_cast<int>(c.hmask) + 1;
-    const float4* src = reinterpret_cast<const float4*>(p.pyr) + c.off;
-    float* dst = reinterpret_cast<float*>(lds + p.slv[l].off);
+    const float4* src = reinterpret_cast<const float4*>(pyr) + c.off;
+    float* dst = reinterpret_cast<float*>(lds + slv[l].off);
     const int n = (w + 2) * (h + 2);
     for (int i = threadIdx.x; i < n; i += 64 * kWaves) {
       const int r = i / (w + 2), col = i - r * (w + 2);

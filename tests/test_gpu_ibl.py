@@ -290,6 +290,24 @@ def test_prefilter_points_match_oracle(env_case, torch):
     assert s["max"] < (MAX_REL if name == "smooth" else 1e-3) and s["mean"] < 1e-5, s
 
 
+@pytest.mark.parametrize("w,h,count,samples", [(1, 1, 1, 1), (2, 1, 7, 63), (64, 32, 9, 64), (16, 64, 8, 65),
+                                               (512, 256, 33, 1000), (512, 256, 5, 2048), (256, 128, 17, 2049),
+                                               (2048, 1024, 40, 4160)])
+def test_prefilter_points_shapes(torch, w, h, count, samples):
+    """Queries of any roughness, 0 and 1 among them: sample counts at both sides
+    of a wave and of the table that LDS holds (2 048), query counts at both sides
+    of a block's eight waves, levels staged in LDS and finer ones."""
+    env = aa.synth.env(seed=SEED0 + w + h, width=w, height=h, sigma=0.2, suns=1, peak_min=5.0, peak_max=5.0,
+                       sun_sigma_deg=30.0)
+    q = aa.synth.dir_rough(seed=w + count, n=count, rmin=0.0, rmax=1.0)
+    q[0, 3] = 0.0
+    q[-1, 3] = 1.0
+    got = aa.prefilter_points(aa.env_pyramid(torch.from_numpy(env).cuda()), w, h, samples,
+                              torch.from_numpy(q).cuda()).cpu().numpy()
+    err = rel_err(got[:, :3], ol.Env(env).prefilter_points(samples, q), RADIANCE_FLOOR)
+    assert err.max() < MAX_REL and (got[:, 3] == 1.0).all(), summary(err)
+
+
 def test_prefilter_points_agree_with_cube_texels(torch):
     # The point kernel at a cube texel's direction and roughness m/(mips-1)
     # estimates the same quantity as the cube kernel (same samples).
