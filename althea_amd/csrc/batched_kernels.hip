@@ -112,7 +112,8 @@ struct althea_prefilter_batch {
   GgxEntry* d_tables = nullptr;
   int* d_counts = nullptr;
   double* d_wsum = nullptr;
-  float* d_wsum32 = nullptr;
+  PyramidJob* d_jobs = nullptr;
+  int pyramid_blocks[kPyramidPasses] = {};
   int* d_counter = nullptr;
   std::vector<std::pair<int, int>> extents;  // distinct (w, h), one table set each
   // Work list of the current tile shape.
@@ -203,16 +204,12 @@ althea_status launch_persistent(const althea_prefilter_batch* b, int shape, int 
 
 // Pyramids of all maps and the sample tables of every source extent.
 althea_status launch_prep(const althea_prefilter_batch* b, hipStream_t s) {
-  for (int i = 0; i < b->count; ++i) {
-    const int w = b->envs[i].width, h = b->envs[i].height;
-    althea_status st = launch_pyramid(b->envs[i].rgba, w, h, b->pyramids[i], s);
-    if (st != ALTHEA_OK) return st;
-  }
+  althea_status st = launch_pyramid_batch(b->d_jobs, b->count, b->pyramid_blocks, s);
+  if (st != ALTHEA_OK) return st;
   for (size_t k = 0; k < b->extents.size(); ++k) {
     const size_t set = k * b->mips;
-    althea_status st = launch_ggx_tables(b->samples, b->mips, b->extents[k].first, b->extents[k].second,
-                                         b->d_tables + set * b->samples, b->d_counts + set, b->d_wsum + set,
-                                         b->d_wsum32 + set, s);
+    st = launch_ggx_tables(b->samples, b->mips, b->extents[k].first, b->extents[k].second,
+                           b->d_tables + set * b->samples, b->d_counts + set, b->d_wsum + set, s);
     if (st != ALTHEA_OK) return st;
   }
   return ALTHEA_OK;
@@ -285,6 +282,7 @@ static althea_status batch_create(const althea_env_view* envs, int count, const 
   std::vector<int> sets_of(count);
 
   std::vector<PrefilterMap> maps(count);
+  std::vector<PyramidJob> jobs;
   std::vector<LevelC> levels(static_cast<size_t>(count) * kMaxLevels);
   std::vector<StagedLevel> slevels(static_cast<size_t>(count) * kMaxLevels);
   b->pyramids.assign(count, nullptr);
@@ -310,6 +308,7 @@ static althea_status batch_create(const althea_env_view* envs, int count, const 
     sets_of[i] = it->second;
     const int w = envs[i].width, h = envs[i].height;
     PrefilterMap& p = maps[i];
+    jobs.push_back(pyramid_job(envs[i].rgba, w, h, b->pyramids[i]));
     size_t staged = 0;
     pyramid_levels(w, h, &levels[static_cast<size_t>(i) * kMaxLevels]);
     p.first = staged_levels(w, h, prefilter_first_level(w, h, mips, samples),
@@ -331,7 +330,7 @@ static althea_status batch_create(const althea_env_view* envs, int count, const 
       hipMalloc(&b->d_tables, sizeof(GgxEntry) * sets * samples) != hipSuccess ||
       hipMalloc(&b->d_counts, sizeof(int) * sets) != hipSuccess ||
       hipMalloc(&b->d_wsum, sizeof(double) * sets) != hipSuccess ||
-      hipMalloc(&b->d_wsum32, sizeof(float) * sets) != hipSuccess ||
+      hipMalloc(&b->d_jobs, sizeof(PyramidJob) * count) != hipSuccess ||
       hipMalloc(&b->d_counter, 256) != hipSuccess) {
     set_error("prefilter_batch_create: out of device memory");
     return fail(ALTHEA_ERROR_OUT_OF_MEMORY);
@@ -344,7 +343,9 @@ static althea_status batch_create(const althea_env_view* envs, int count, const 
     maps[i].lv = b->d_levels + static_cast<size_t>(i) * kMaxLevels;
     maps[i].slv = b->d_slevels + static_cast<size_t>(i) * kMaxLevels;
   }
+  pyramid_schedule(jobs, b->pyramid_blocks);
   if (hipMemcpy(b->d_maps, maps.data(), sizeof(PrefilterMap) * count, hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemcpy(b->d_jobs, jobs.data(), sizeof(PyramidJob) * count, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(b->d_levels, levels.data(), sizeof(LevelC) * levels.size(), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(b->d_slevels, slevels.data(), sizeof(StagedLevel) * slevels.size(), hipMemcpyHostToDevice) !=
           hipSuccess ||
@@ -379,7 +380,7 @@ althea_status althea_prefilter_batch_destroy(althea_prefilter_batch* b) {
   (void)hipFree(b->d_tables);
   (void)hipFree(b->d_counts);
   (void)hipFree(b->d_wsum);
-  (void)hipFree(b->d_wsum32);
+  (void)hipFree(b->d_jobs);
   (void)hipFree(b->d_counter);
   (void)hipFree(b->d_work);
   delete b;

@@ -6,6 +6,7 @@
 #include <cstdarg>
 #include <cstddef>
 #include <cstdint>
+#include <vector>
 
 #include "althea/althea.h"
 
@@ -72,11 +73,25 @@ int prefilter_split(int size, int mips, int samples, int& chunk);
 
 // Kernel launchers (ibl_kernels.hip).
 althea_status launch_ggx_tables(int samples, int mips, int env_w, int env_h, GgxEntry* tables, int* counts,
-                                double* wsum, float* wsum32, hipStream_t s);
+                                double* wsum, hipStream_t s);
 void pyramid_levels(int w, int h, LevelC* out);
 althea_status launch_hammersley(uint32_t n, uint32_t first, uint32_t count, uint32_t* bits, float* xi,
                                 hipStream_t s);
 althea_status launch_pyramid(const float* level0, int w, int h, float* pyr, hipStream_t s);
+
+// Pyramids of many maps, five levels a pass over all of them.
+constexpr int kPyramidPasses = 4;  // 16 levels
+struct PyramidJob {
+  const float4* src;  // level 0, or pyr itself
+  float4* pyr;
+  int w, h, levels;
+  uint32_t off[16];  // texel offset of each level
+  int first_block[kPyramidPasses];
+};
+PyramidJob pyramid_job(const float* level0, int w, int h, float* pyr);
+void pyramid_schedule(std::vector<PyramidJob>& jobs, int blocks[kPyramidPasses]);
+althea_status launch_pyramid_batch(const PyramidJob* d_jobs, int count, const int blocks[kPyramidPasses],
+                                   hipStream_t s);
 althea_status launch_prefilter_cube(const float* pyr, int env_w, int env_h, int size, int mips, int samples,
                                     unsigned flags, float* cube, void* workspace, hipStream_t s);
 size_t prefilter_workspace_bytes(int env_w, int env_h, int size, int mips, int samples);

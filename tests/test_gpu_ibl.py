@@ -75,6 +75,26 @@ def test_pyramid_matches_oracle(env_case, torch):
     assert err.max() < 1e-6, summary(err)
 
 
+@pytest.mark.parametrize("w,h", [(1, 1), (2, 1), (1, 64), (32, 1), (64, 2), (32, 32), (16, 4096), (1024, 64)])
+def test_pyramid_is_the_box_chain(torch, w, h):
+    """Extents at and below the 32 x 32 tile, unit extents and several passes,
+    bit for bit: each level is ((a + b) + (c + d)) / 4 of the one above, or
+    (a + b) / 2 where one extent is 1."""
+    rng = np.random.default_rng(w + 7 * h)
+    lvl = rng.uniform(0.0, 100.0, (h, w, 4)).astype(np.float32)
+    ref = [lvl.reshape(-1, 4)]
+    got = aa.env_pyramid(torch.from_numpy(lvl).cuda()).cpu().numpy()
+    while max(lvl.shape[:2]) > 1:
+        if min(lvl.shape[:2]) > 1:
+            lvl = ((lvl[0::2, 0::2] + lvl[0::2, 1::2]) + (lvl[1::2, 0::2] + lvl[1::2, 1::2])) * np.float32(0.25)
+        elif lvl.shape[1] > 1:
+            lvl = (lvl[:, 0::2] + lvl[:, 1::2]) * np.float32(0.5)
+        else:
+            lvl = (lvl[0::2] + lvl[1::2]) * np.float32(0.5)
+        ref.append(lvl.reshape(-1, 4))
+    np.testing.assert_array_equal(got.view(np.uint32), np.concatenate(ref).view(np.uint32))
+
+
 def test_pyramid_4096_levels(torch):
     env = aa.synth.env(seed=SEED0 + 2, width=4096, height=2048, sigma=1.5, suns=8, peak_min=1e3, peak_max=1e4)
     pyr = aa.env_pyramid(torch.from_numpy(env).cuda()).cpu().numpy()
