@@ -100,7 +100,7 @@ __device__ __forceinline__ void encode_all(float dx, float dy, float dz, float r
 // -------------------------------------------- register-resident inference
 // The forward A operands of this lane (feature group g = lane / 16, row
 // n = lane % 16 of each 16-row block), 88 VGPRs, loaded once per wave; the
-// streaming inference layout of mlp_fwd_kernel.
+// streaming inference layout.
 struct MlpRegWeights {
   bf16x8 a1[4], a2[4][2], a3[4][2], a4[2];
 };
@@ -120,8 +120,8 @@ __device__ __forceinline__ void mlp_load_reg_weights(const MlpDeviceWeights& w, 
 
 // Log-radiance of one 16-query tile: lane (g, n) passes query n (every group
 // of the tile passes the same query n); the result for query n sits in lane
-// n of group 0 (rows 0..2 of y).  Arithmetic identical to mlp_fwd_kernel's
-// inference: same features, MFMA order, bias and SiLU.
+// n of group 0 (rows 0..2 of y).  The training forward takes the same
+// features, MFMA order, bias and SiLU.
 __device__ __forceinline__ f32x4 mlp_tile_eval(const MlpRegWeights& r, const MlpDeviceWeights& w, int g, float dx,
                                                float dy, float dz, float rough) {
   float f[32];

@@ -14,14 +14,13 @@
 // between layers.  The backward pass (dH = W^T dZ) uses the same trick with
 // transposed packed weights.
 //
-// Training per batch: mlp_fwd_bwd_kernel (forward, loss, backward-data,
-// feature-major bf16 copies of X, H1..H3, dY, dZ1..dZ3, per-block bias and
-// loss partials) -> mlp_wgrad_kernel (dW = dZ . H^T as split-K MFMA over
-// samples, per-block partials) -> mlp_adam_kernel (fixed-order reduction of
-// the partials, Adam on the FP32 master copy) -> mlp_pack_kernel (BF16
-// operand layouts).
+// Training per batch: mlp_train_kernel (forward, loss, backward-data, and the
+// weight and bias gradients as split-K MFMA over the block's samples, per-block
+// partials) -> mlp_adam_kernel (fixed-order reduction of the partials, Adam on
+// the FP32 master copy, the updated parameters' BF16 operands).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <new>
@@ -72,65 +71,115 @@ __global__ void mlp_pack_kernel(const float* __restrict__ p, MlpDeviceWeights w)
   if (t < 16) w.b4[t] = t < kMlpOut ? p[kOffB4 + t] : 0.0f;
 }
 
-// ------------------------------------------------- forward (+ backward-data)
+// --------------------------------------------------------------- inference
 struct FwdParams {
   MlpDeviceWeights w;
   const float4* dir_rough;
-  const float4* targets;  // training only
-  float4* out;            // inference only: rgb radiance = exp(y)
+  float4* out;  // rgb radiance = exp(y)
   int count;
-  float grad_scale;       // 2 / (3 * batch)
-  MlpActivations act;     // feature-major copies (training)
-  float* bias_partial;    // [gridDim.x][kMlpBiasPartial] (training: the loss column)
 };
 
-// One 16-sample tile per iteration per wave.  kTrain adds the loss, the
-// backward-data chain and the feature-major stores (the weight-gradient
-// kernel forms every weight and bias gradient from those).
-template <bool kTrain>
-__global__ __launch_bounds__(256) void mlp_fwd_kernel(const FwdParams p) {
+// One 16-sample tile per iteration per wave, the forward operands in registers.
+__global__ __launch_bounds__(256) void mlp_infer_kernel(const FwdParams p) {
   const int lane = threadIdx.x & 63;
   const int g = lane >> 4, n = lane & 15;
   const int wave = threadIdx.x >> 6;
-  const int waves_total = gridDim.x * 4;
-  const int tiles = kTrain ? 2 * ((p.count + 31) / 32) : (p.count + 15) / 16;
-
-  // Inference keeps the forward A operands in registers; training reloads
-  // them (L1/L2 resident) at each use to leave registers for the backward.
-  bf16x8 a1[4], a2[4][2], a3[4][2], a4[2];
-  if (!kTrain) {
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      a1[b] = load8(p.w.w1 + (16 * b + n) * 32 + 8 * g);
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        a2[b][kb] = load8(p.w.w2 + (16 * b + n) * 64 + 32 * kb + 8 * g);
-        a3[b][kb] = load8(p.w.w3 + (16 * b + n) * 64 + 32 * kb + 8 * g);
-      }
-    }
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) a4[kb] = load8(p.w.w4 + n * 64 + 32 * kb + 8 * g);
-  }
-  auto A1 = [&](int b) { return kTrain ? load8(p.w.w1 + (16 * b + n) * 32 + 8 * g) : a1[b]; };
-  auto A2 = [&](int b, int kb) { return kTrain ? load8(p.w.w2 + (16 * b + n) * 64 + 32 * kb + 8 * g) : a2[b][kb]; };
-  auto A3 = [&](int b, int kb) { return kTrain ? load8(p.w.w3 + (16 * b + n) * 64 + 32 * kb + 8 * g) : a3[b][kb]; };
-  auto A4 = [&](int kb) { return kTrain ? load8(p.w.w4 + n * 64 + 32 * kb + 8 * g) : a4[kb]; };
-
-  float loss = 0.0f;  // training: this lane's squared log errors
-
-  for (int tile = blockIdx.x * 4 + wave; tile < tiles; tile += waves_total) {
+  const int tiles = (p.count + 15) / 16;
+  MlpRegWeights r;
+  mlp_load_reg_weights(p.w, g, n, r);
+  for (int tile = blockIdx.x * 4 + wave; tile < tiles; tile += static_cast<int>(gridDim.x) * 4) {
     const int s = tile * 16 + n;
     const bool valid = s < p.count;
     const float4 q = valid ? p.dir_rough[s] : make_float4(0.f, 0.f, 1.f, 0.f);
+    const f32x4 y = mlp_tile_eval(r, p.w, g, q.x, q.y, q.z, q.w);
+    if (g == 0 && valid) p.out[s] = make_float4(expf(y[0]), expf(y[1]), expf(y[2]), 1.0f);
+  }
+}
+
+// ---------------------------------------------------------------- training
+// Forward, loss, backward-data and the block's share of every gradient in one
+// kernel.  A block of kW waves takes 16 kW samples a step, a tile to a wave;
+// the BF16 inputs, activations and pre-activation gradients stay in LDS
+// feature-major, (row, sample) as the gradients' MFMAs read them: dW_l[o][k] =
+// sum_s dZ_l[o][s] H_{l-1}[k][s] with samples on the K axis, A = dZ (lane: 8
+// consecutive samples of one output row), B = H; the bias gradients are the
+// same product with a B tile of ones.  The packed weights are in LDS beside
+// them.  Gradients accumulate in registers over the block's steps and leave as
+// one partial row per block.
+//
+// The activations of a batch of 65 536 are 57 MB: written by a forward kernel in
+// 2-byte stores and read back by a gradient kernel they took 31 + 19 us; here
+// @TRAIN@.  Bound: VALU (SiLU and its derivative) and the latency of a tile's six
+// layers at two waves a SIMD (eight waves: 157 KB of LDS, one block a CU).
+struct TrainParams {
+  MlpDeviceWeights w;
+  const float4* dir_rough;
+  const float4* targets;
+  int count;
+  float grad_scale;     // 2 / (3 * batch)
+  float* partial;       // [gridDim.x][kMlpWeights]
+  float* bias_partial;  // [gridDim.x][kMlpBiasPartial]
+};
+
+// Rows of the feature-major activations in LDS.
+constexpr int kRowX = 0, kRowH1 = 32, kRowH2 = 96, kRowH3 = 160, kRowDy = 224, kRowZ1 = 240, kRowZ2 = 304,
+              kRowZ3 = 368, kTrainRows = 432;
+
+template <int kW>
+struct TrainSmem {
+  static constexpr int kStride = 16 * kW + 8;  // samples a row: 16 bytes of padding spread the rows over the banks
+  MlpSmem w;
+  bf16x8 w2t[64 * 8], w3t[64 * 8], w4t[64 * 4];
+  float loss[kW];
+  alignas(16) __bf16 act[kTrainRows * kStride];
+};
+
+template <int kW>
+__global__ __launch_bounds__(64 * kW) void mlp_train_kernel(const TrainParams p) {
+  extern __shared__ float4 s_mem[];
+  TrainSmem<kW>& sm = *reinterpret_cast<TrainSmem<kW>*>(s_mem);
+  constexpr int kStride = TrainSmem<kW>::kStride;
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> 4, n = lane & 15;
+  const int wave = threadIdx.x >> 6;
+  mlp_stage_weights(sm.w, p.w, threadIdx.x, 64 * kW);
+  for (int i = threadIdx.x; i < 64 * 8; i += 64 * kW) {
+    sm.w2t[mlp_swz64(i >> 3, i & 7)] = load8(p.w.w2t + 8 * i);
+    sm.w3t[mlp_swz64(i >> 3, i & 7)] = load8(p.w.w3t + 8 * i);
+  }
+  for (int i = threadIdx.x; i < 64 * 4; i += 64 * kW) sm.w4t[mlp_swz32(i >> 2, i & 3)] = load8(p.w.w4t + 8 * i);
+  __syncthreads();
+
+  // This wave's gradient blocks: output rows 16 ob.., input columns of half kh.
+  constexpr int kHalves = kW / 4, kBlocks = 4 / kHalves;  // 64-wide inputs: kBlocks column blocks a wave
+  const int ob = wave & 3, kh = wave >> 2;
+  const bool bias_wave = kh == kHalves - 1;  // also the bias gradients of its rows
+  const bool w4_wave = kh == 0;              // also layer 4, input block ob
+  f32x4 d1[2 / kHalves] = {}, d2[kBlocks] = {}, d3[kBlocks] = {}, d4 = {};
+  f32x4 e1 = {}, e2 = {}, e3 = {}, e4 = {};  // bias sums (every column of D the same)
+  bf16x8 ones;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) ones[j] = static_cast<__bf16>(1.0f);
+  float loss = 0.0f;  // this lane's squared log errors
+
+  const int steps = (p.count + 16 * kW - 1) / (16 * kW);
+  for (int step = blockIdx.x; step < steps; step += gridDim.x) {
+    const int col = 16 * wave + n;
+    const int s = step * 16 * kW + col;
+    const bool valid = s < p.count;
+    const float4 q = valid ? p.dir_rough[s] : make_float4(0.f, 0.f, 1.f, 0.f);
+    const float4 target = valid ? p.targets[s] : make_float4(1.f, 1.f, 1.f, 1.f);
+    auto at = [&](int row) -> __bf16& { return sm.act[row * kStride + col]; };
     // Layer 1 input (B operand): this lane's 8 features.
     float f[32];
     encode_all(q.x, q.y, q.z, q.w, f);
     bf16x8 x;
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < 8; ++j) {
       x[j] = static_cast<__bf16>(g == 0 ? f[j] : (g == 1 ? f[8 + j] : (g == 2 ? f[16 + j] : f[24 + j])));
-
-    // Hidden layer: D = W . H^T (+ bias), SiLU; `sp` keeps SiLU'(z) for training.
+      at(kRowX + 8 * g + j) = x[j];
+    }
+    // Hidden layer: D = W . H^T (+ bias), SiLU; `sp` keeps SiLU'(z).
     auto hidden = [&](auto&& wtile, const bf16x8* in, int nk, const float* bias, f32x4* h, f32x4* sp) {
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
@@ -142,68 +191,51 @@ __global__ __launch_bounds__(256) void mlp_fwd_kernel(const FwdParams p) {
           const float z = acc[i] + bias[16 * b + 4 * g + i];
           const float sg = sigmoidf(z);
           h[b][i] = z * sg;
-          if (kTrain) sp[b][i] = sg * (1.0f + z * (1.0f - sg));
+          sp[b][i] = sg * (1.0f + z * (1.0f - sg));
         }
       }
     };
-    // Feature-major copies for the weight gradients (training): element
-    // (row, sample) at row * B + col, 32-bit offsets (batch <= 2^24).
-    const MlpActivations& A = p.act;
-    const uint32_t B = static_cast<uint32_t>(A.stride);
-    const uint32_t col = static_cast<uint32_t>(tile) * 16u + n;
-    auto store_tile = [&](__bf16* dst, const bf16x8* hb) {
-      if (!kTrain) return;
+    auto store_tile = [&](int row, const bf16x8* hb) {
 #pragma unroll
       for (int b = 0; b < 4; ++b)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) dst[(16u * b + 4u * g + i) * B + col] = hb[b >> 1][4 * (b & 1) + i];
+        for (int i = 0; i < 4; ++i) at(row + 16 * b + 4 * g + i) = hb[b >> 1][4 * (b & 1) + i];
     };
-    if (kTrain) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) A.x[(8u * g + j) * B + col] = x[j];
-    }
     f32x4 h[4], sp1[4], sp2[4], sp3[4];
-    hidden([&](int b, int) { return A1(b); }, &x, 1, p.w.b1, h, sp1);
+    hidden([&](int b, int) { return sm.w.w1[mlp_swz32(16 * b + n, g)]; }, &x, 1, sm.w.b, h, sp1);
     const bf16x8 hb1[2] = {pack8(h[0], h[1]), pack8(h[2], h[3])};
-    store_tile(A.h1, hb1);
-    hidden([&](int b, int kb) { return A2(b, kb); }, hb1, 2, p.w.b2, h, sp2);
+    store_tile(kRowH1, hb1);
+    hidden([&](int b, int kb) { return sm.w.w2[mlp_swz64(16 * b + n, 4 * kb + g)]; }, hb1, 2, sm.w.b + 64, h, sp2);
     const bf16x8 hb2[2] = {pack8(h[0], h[1]), pack8(h[2], h[3])};
-    store_tile(A.h2, hb2);
-    hidden([&](int b, int kb) { return A3(b, kb); }, hb2, 2, p.w.b3, h, sp3);
+    store_tile(kRowH2, hb2);
+    hidden([&](int b, int kb) { return sm.w.w3[mlp_swz64(16 * b + n, 4 * kb + g)]; }, hb2, 2, sm.w.b + 128, h, sp3);
     const bf16x8 hb3[2] = {pack8(h[0], h[1]), pack8(h[2], h[3])};
-    store_tile(A.h3, hb3);
+    store_tile(kRowH3, hb3);
     f32x4 y = {0.f, 0.f, 0.f, 0.f};
-    y = mfma(A4(0), hb3[0], y);
-    y = mfma(A4(1), hb3[1], y);
+    y = mfma(sm.w.w4[mlp_swz64(n, g)], hb3[0], y);
+    y = mfma(sm.w.w4[mlp_swz64(n, 4 + g)], hb3[1], y);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) y[i] += p.w.b4[4 * g + i];
-
-    if (!kTrain) {
-      if (g == 0 && valid) p.out[s] = make_float4(expf(y[0]), expf(y[1]), expf(y[2]), 1.0f);
-      continue;
-    }
+    for (int i = 0; i < 4; ++i) y[i] += sm.w.b[192 + 4 * g + i];
 
     // ---- loss: lanes g == 0 own outputs 0..2 of sample n.
     f32x4 dy = {0.f, 0.f, 0.f, 0.f};
     if (g == 0 && valid) {
-      const float4 t = p.targets[s];
-      const float e0 = y[0] - logf(t.x), e1 = y[1] - logf(t.y), e2 = y[2] - logf(t.z);
-      loss += e0 * e0 + e1 * e1 + e2 * e2;
+      const float e0 = y[0] - logf(target.x), e1_ = y[1] - logf(target.y), e2_ = y[2] - logf(target.z);
+      loss += e0 * e0 + e1_ * e1_ + e2_ * e2_;
       dy[0] = p.grad_scale * e0;
-      dy[1] = p.grad_scale * e1;
-      dy[2] = p.grad_scale * e2;
+      dy[1] = p.grad_scale * e1_;
+      dy[2] = p.grad_scale * e2_;
     }
-
     bf16x8 dyb;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       dyb[i] = static_cast<__bf16>(dy[i]);
       dyb[4 + i] = static_cast<__bf16>(0.0f);
-      A.dy[(4u * g + i) * B + col] = dyb[i];
+      at(kRowDy + 4 * g + i) = dyb[i];
     }
 
     // ---- backward-data: dH = W^T dZ, dZ = dH * SiLU'(z), layer by layer.
-    auto backward = [&](auto&& wtile, const bf16x8* in, int nk, const f32x4* sp, __bf16* store, f32x4* dz) {
+    auto backward = [&](auto&& wtile, const bf16x8* in, int nk, const f32x4* sp, int row, f32x4* dz) {
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -213,120 +245,91 @@ __global__ __launch_bounds__(256) void mlp_fwd_kernel(const FwdParams p) {
         for (int i = 0; i < 4; ++i) {
           const float d = acc[i] * sp[b][i];
           dz[b][i] = d;
-          store[(16u * b + 4u * g + i) * B + col] = static_cast<__bf16>(d);
+          at(row + 16 * b + 4 * g + i) = static_cast<__bf16>(d);
         }
       }
     };
     f32x4 dz[4];
-    backward([&](int b, int) { return load8(p.w.w4t + (16 * b + n) * 32 + 8 * g); }, &dyb, 1, sp3, A.dz3, dz);
+    backward([&](int b, int) { return sm.w4t[mlp_swz32(16 * b + n, g)]; }, &dyb, 1, sp3, kRowZ3, dz);
     bf16x8 d_in[2] = {pack8(dz[0], dz[1]), pack8(dz[2], dz[3])};
-    backward([&](int b, int kb) { return load8(p.w.w3t + (16 * b + n) * 64 + 32 * kb + 8 * g); }, d_in, 2, sp2,
-             A.dz2, dz);
+    backward([&](int b, int kb) { return sm.w3t[mlp_swz64(16 * b + n, 4 * kb + g)]; }, d_in, 2, sp2, kRowZ2, dz);
     d_in[0] = pack8(dz[0], dz[1]);
     d_in[1] = pack8(dz[2], dz[3]);
-    backward([&](int b, int kb) { return load8(p.w.w2t + (16 * b + n) * 64 + 32 * kb + 8 * g); }, d_in, 2, sp1,
-             A.dz1, dz);
-  }
+    backward([&](int b, int kb) { return sm.w2t[mlp_swz64(16 * b + n, 4 * kb + g)]; }, d_in, 2, sp1, kRowZ1, dz);
+    __syncthreads();
 
-  if (!kTrain) return;
-  // The block's loss in the loss column of its partial row, fixed order.
-  __shared__ float s_loss[4];
-  float l = loss;
+    // ---- gradients over the step's 16 kW samples, 32 at a time.
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) l += __shfl_xor(l, o, 64);
-  if (lane == 0) s_loss[wave] = l;
-  __syncthreads();
-  if (threadIdx.x == 0)
-    p.bias_partial[static_cast<size_t>(blockIdx.x) * kMlpBiasPartial + kBiasLoss] =
-        s_loss[0] + s_loss[1] + s_loss[2] + s_loss[3];
-}
-
-// ------------------------------------------------------ weight gradients
-// dW_l[o][k] = sum_s dZ_l[o][s] H_{l-1}[k][s] with samples on the MFMA K axis:
-// A = dZ tile (lane: 8 consecutive samples of one output row), B = H tile.
-// The bias gradients db_l[o] = sum_s dZ_l[o][s] are the same product with a
-// B tile of ones.  Each block owns a contiguous sample range; wave w owns
-// output block w of layers 1-3 and input block w of layer 4 (wave 0 also the
-// layer-4 bias).  Partials: one row of weights and one row of biases per
-// block (the forward kernel writes the loss column of the bias row).
-struct WgradParams {
-  MlpActivations act;
-  int count;         // samples (multiple of 32 after padding)
-  int chunks_per_block;
-  float* partial;       // [gridDim.x][kMlpWeights]
-  float* bias_partial;  // [gridDim.x][kMlpBiasPartial], columns before kBiasLoss
-};
-
-__global__ __launch_bounds__(256) void mlp_wgrad_kernel(const WgradParams p) {
-  const int lane = threadIdx.x & 63;
-  const int g = lane >> 4, n = lane & 15;
-  const int w = threadIdx.x >> 6;
-  const MlpActivations& A = p.act;
-  const size_t B = A.stride;
-  f32x4 d1[2] = {}, d2[4] = {}, d3[4] = {}, d4 = {};
-  f32x4 e1 = {}, e2 = {}, e3 = {}, e4 = {};  // bias sums (every column of D the same)
-  bf16x8 ones;
+    for (int c = 0; c < kW / 2; ++c) {
+      auto row8 = [&](int row) {  // 8 samples of a row
+        return *reinterpret_cast<const bf16x8*>(&sm.act[(row + n) * kStride + 32 * c + 8 * g]);
+      };
+      const bf16x8 z1 = row8(kRowZ1 + 16 * ob), z2 = row8(kRowZ2 + 16 * ob), z3 = row8(kRowZ3 + 16 * ob);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) ones[j] = static_cast<__bf16>(1.0f);
-  const int chunk0 = blockIdx.x * p.chunks_per_block;
-  const int nchunks = (p.count + 31) / 32;
-  for (int c = chunk0; c < min(chunk0 + p.chunks_per_block, nchunks); ++c) {
-    const size_t s0 = static_cast<size_t>(c) * 32 + 8 * g;
-    const bf16x8 z1 = load8(A.dz1 + (16 * w + n) * B + s0);
-    const bf16x8 z2 = load8(A.dz2 + (16 * w + n) * B + s0);
-    const bf16x8 z3 = load8(A.dz3 + (16 * w + n) * B + s0);
-    const bf16x8 y = load8(A.dy + n * B + s0);
+      for (int k = 0; k < 2 / kHalves; ++k) d1[k] = mfma(z1, row8(kRowX + 16 * (kh * (2 / kHalves) + k)), d1[k]);
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) d1[kb] = mfma(z1, load8(A.x + (16 * kb + n) * B + s0), d1[kb]);
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      d2[kb] = mfma(z2, load8(A.h1 + (16 * kb + n) * B + s0), d2[kb]);
-      d3[kb] = mfma(z3, load8(A.h2 + (16 * kb + n) * B + s0), d3[kb]);
+      for (int k = 0; k < kBlocks; ++k) {
+        d2[k] = mfma(z2, row8(kRowH1 + 16 * (kh * kBlocks + k)), d2[k]);
+        d3[k] = mfma(z3, row8(kRowH2 + 16 * (kh * kBlocks + k)), d3[k]);
+      }
+      if (w4_wave) d4 = mfma(row8(kRowDy), row8(kRowH3 + 16 * ob), d4);
+      if (bias_wave) {
+        e1 = mfma(z1, ones, e1);
+        e2 = mfma(z2, ones, e2);
+        e3 = mfma(z3, ones, e3);
+        if (ob == 0) e4 = mfma(row8(kRowDy), ones, e4);
+      }
     }
-    d4 = mfma(y, load8(A.h3 + (16 * w + n) * B + s0), d4);
-    e1 = mfma(z1, ones, e1);
-    e2 = mfma(z2, ones, e2);
-    e3 = mfma(z3, ones, e3);
-    if (w == 0) e4 = mfma(y, ones, e4);
+    __syncthreads();
   }
+
   float* bout = p.bias_partial + static_cast<size_t>(blockIdx.x) * kMlpBiasPartial;
-  if (n == 0) {  // column 0 of D: row o = 16 w + 4 g + i
+  if (bias_wave && n == 0) {  // column 0 of D: row o = 16 ob + 4 g + i
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int o = 16 * w + 4 * g + i;
+      const int o = 16 * ob + 4 * g + i;
       bout[kBiasB1 + o] = e1[i];
       bout[kBiasB2 + o] = e2[i];
       bout[kBiasB3 + o] = e3[i];
-      if (w == 0 && o < kMlpOut) bout[kBiasB4 + o] = e4[i];
+      if (ob == 0 && o < kMlpOut) bout[kBiasB4 + o] = e4[i];
     }
   }
   float* out = p.partial + static_cast<size_t>(blockIdx.x) * kMlpWeights;
-  // D: lane holds dW[o = 16 w + 4 g + i][k = 16 kb + n].
+  // D: lane holds dW[o = 16 ob + 4 g + i][k = 16 kb + n].
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int o = 16 * w + 4 * g + i;
+    const int o = 16 * ob + 4 * g + i;
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      const int k = 16 * kb + n;
-      if (k < kMlpIn) out[kWgW1 + o * kMlpIn + k] = d1[kb][i];
+    for (int k = 0; k < 2 / kHalves; ++k) {
+      const int c = 16 * (kh * (2 / kHalves) + k) + n;
+      if (c < kMlpIn) out[kWgW1 + o * kMlpIn + c] = d1[k][i];
     }
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      out[kWgW2 + o * 64 + 16 * kb + n] = d2[kb][i];
-      out[kWgW3 + o * 64 + 16 * kb + n] = d3[kb][i];
+    for (int k = 0; k < kBlocks; ++k) {
+      const int c = 16 * (kh * kBlocks + k) + n;
+      out[kWgW2 + o * 64 + c] = d2[k][i];
+      out[kWgW3 + o * 64 + c] = d3[k][i];
     }
-    const int o4 = 4 * g + i;  // layer 4: output rows 0..15 (3 used), inputs 16 w + n
-    if (o4 < kMlpOut) out[kWgW4 + o4 * 64 + 16 * w + n] = d4[i];
+    const int o4 = 4 * g + i;  // layer 4: output rows 0..15 (3 used), inputs 16 ob + n
+    if (w4_wave && o4 < kMlpOut) out[kWgW4 + o4 * 64 + 16 * ob + n] = d4[i];
+  }
+  // The block's loss in the loss column of its partial row, fixed order.
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) loss += __shfl_xor(loss, o, 64);
+  if (lane == 0) sm.loss[wave] = loss;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float l = 0.0f;
+    for (int k = 0; k < kW; ++k) l += sm.loss[k];
+    bout[kBiasLoss] = l;
   }
 }
 
 // --------------------------------------------------------------- Adam step
 struct AdamParams {
-  const float* wpartial;  // [wblocks][kMlpWeights]
-  int wblocks;
-  const float* bpartial;  // [lblocks][kMlpBiasPartial]: bias columns in rows < bblocks, loss in rows < lblocks
-  int bblocks;
-  int lblocks;
+  const float* wpartial;  // [blocks][kMlpWeights]
+  const float* bpartial;  // [blocks][kMlpBiasPartial], the loss in the last column
+  int blocks;
   float* params;          // FP32 master copy, oracle order
   float* m;
   float* v;
@@ -380,7 +383,7 @@ __global__ __launch_bounds__(256) void mlp_adam_kernel(const AdamParams p) {
     if (!p.loss_out) return;
     __shared__ float s_loss[256];
     float l = 0.0f;
-    for (int b = threadIdx.x; b < p.lblocks; b += 256)
+    for (int b = threadIdx.x; b < p.blocks; b += 256)
       l += p.bpartial[static_cast<size_t>(b) * kMlpBiasPartial + kBiasLoss];
     s_loss[threadIdx.x] = l;
     __syncthreads();
@@ -397,10 +400,10 @@ __global__ __launch_bounds__(256) void mlp_adam_kernel(const AdamParams p) {
   if (t < kMlpParams) {
     const int wi = mlp_param_to_wgrad(t);
     if (wi >= 0) {
-      for (int b = lane; b < p.wblocks; b += kAdamLanes) gsum += p.wpartial[static_cast<size_t>(b) * kMlpWeights + wi];
+      for (int b = lane; b < p.blocks; b += kAdamLanes) gsum += p.wpartial[static_cast<size_t>(b) * kMlpWeights + wi];
     } else {
       const int bi = mlp_param_to_bias(t);
-      for (int b = lane; b < p.bblocks; b += kAdamLanes)
+      for (int b = lane; b < p.blocks; b += kAdamLanes)
         gsum += p.bpartial[static_cast<size_t>(b) * kMlpBiasPartial + bi];
     }
   }
@@ -517,9 +520,6 @@ struct MlpState {
   float* v = nullptr;
   MlpDeviceWeights w{};
   void* weights_mem = nullptr;
-  MlpActivations act{};
-  void* act_mem = nullptr;
-  int act_capacity = 0;
   float* wpartial = nullptr;
   float* bpartial = nullptr;
   int step = 0;
@@ -532,14 +532,8 @@ struct MlpState {
   size_t queue_regions = 0;
 };
 
-// Training grids.  The forward (about 240 registers per lane: two waves per
-// SIMD) runs two waves per SIMD; the weight gradients keep one partial row
-// per block, so their grid stays at one wave per SIMD (10 MB of partials).
-// Row b of the bias partials holds the weight-gradient block b's bias sums
-// and the forward block b's loss.
-static constexpr int kFwdBlocks = 512;
-static constexpr int kWgradBlocks = 256;
-static_assert(kFwdBlocks >= kWgradBlocks, "bias partial rows");
+// One training block a CU, a partial row each (10 MB at 256).
+static constexpr int kTrainBlocks = 256;
 
 static size_t align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
@@ -563,32 +557,6 @@ static althea_status alloc_weights(MlpState* s) {
   return ALTHEA_OK;
 }
 
-static althea_status ensure_activations(MlpState* s, int count) {
-  int cap = (count + 31) / 32 * 32;
-  if (cap <= s->act_capacity) return ALTHEA_OK;
-  ALTHEA_TRY_HIP(hipDeviceSynchronize());
-  (void)hipFree(s->act_mem);
-  s->act_mem = nullptr;
-  s->act_capacity = 0;
-  size_t B = static_cast<size_t>(cap);
-  size_t rows[] = {32, 64, 64, 64, 16, 64, 64, 64};
-  size_t total = 0;
-  for (size_t r : rows) total += align256(r * B * 2);
-  ALTHEA_TRY_HIP(hipMalloc(&s->act_mem, total));
-  // Padding columns must read as zero in the weight-gradient pass.
-  ALTHEA_TRY_HIP(hipMemset(s->act_mem, 0, total));
-  char* c = static_cast<char*>(s->act_mem);
-  __bf16** dst[] = {&s->act.x, &s->act.h1, &s->act.h2, &s->act.h3, &s->act.dy, &s->act.dz1, &s->act.dz2,
-                    &s->act.dz3};
-  for (int i = 0; i < 8; ++i) {
-    *dst[i] = reinterpret_cast<__bf16*>(c);
-    c += align256(rows[i] * B * 2);
-  }
-  s->act.stride = B;
-  s->act_capacity = cap;
-  return ALTHEA_OK;
-}
-
 static althea_status launch_pack(MlpState* s, hipStream_t stream) {
   hipLaunchKernelGGL(mlp_pack_kernel, dim3((64 * 64 + 255) / 256), dim3(256), 0, stream, s->params, s->w);
   return check_launch("mlp_pack_kernel");
@@ -597,35 +565,27 @@ static althea_status launch_pack(MlpState* s, hipStream_t stream) {
 // Forward + backward + reduction (+ Adam when update).
 static althea_status run_train(MlpState* s, const float* dir_rough, const float* targets, int count, float* grad_out,
                                float* loss_out, bool update, hipStream_t stream) {
-  althea_status st = ensure_activations(s, count);
-  if (st != ALTHEA_OK) return st;
-  FwdParams fp{};
-  fp.w = s->w;
-  fp.dir_rough = reinterpret_cast<const float4*>(dir_rough);
-  fp.targets = reinterpret_cast<const float4*>(targets);
-  fp.count = count;
-  fp.grad_scale = 2.0f / (3.0f * static_cast<float>(count));
-  fp.act = s->act;
-  fp.bias_partial = s->bpartial;
-  hipLaunchKernelGGL(mlp_fwd_kernel<true>, dim3(kFwdBlocks), dim3(256), 0, stream, fp);
-  st = check_launch("mlp_fwd_kernel<train>");
-  if (st != ALTHEA_OK) return st;
-  WgradParams wp{};
-  wp.act = s->act;
-  wp.count = count;
-  int nchunks = (count + 31) / 32;
-  wp.chunks_per_block = (nchunks + kWgradBlocks - 1) / kWgradBlocks;
-  wp.partial = s->wpartial;
-  wp.bias_partial = s->bpartial;
-  hipLaunchKernelGGL(mlp_wgrad_kernel, dim3(kWgradBlocks), dim3(256), 0, stream, wp);
-  st = check_launch("mlp_wgrad_kernel");
+  TrainParams tp{};
+  tp.w = s->w;
+  tp.dir_rough = reinterpret_cast<const float4*>(dir_rough);
+  tp.targets = reinterpret_cast<const float4*>(targets);
+  tp.count = count;
+  tp.grad_scale = 2.0f / (3.0f * static_cast<float>(count));
+  tp.partial = s->wpartial;
+  tp.bias_partial = s->bpartial;
+  // Four waves (64 samples a step) while that gives every CU at most one step.
+  const int kw = count <= 64 * kTrainBlocks ? 4 : 8;
+  const int blocks = std::min((count + 16 * kw - 1) / (16 * kw), kTrainBlocks);
+  if (kw == 4)
+    hipLaunchKernelGGL(mlp_train_kernel<4>, dim3(blocks), dim3(256), sizeof(TrainSmem<4>), stream, tp);
+  else
+    hipLaunchKernelGGL(mlp_train_kernel<8>, dim3(blocks), dim3(512), sizeof(TrainSmem<8>), stream, tp);
+  althea_status st = check_launch("mlp_train_kernel");
   if (st != ALTHEA_OK) return st;
   AdamParams ap{};
   ap.wpartial = s->wpartial;
-  ap.wblocks = kWgradBlocks;
   ap.bpartial = s->bpartial;
-  ap.bblocks = kWgradBlocks;
-  ap.lblocks = kFwdBlocks;
+  ap.blocks = blocks;
   ap.params = s->params;
   ap.m = s->m;
   ap.v = s->v;
@@ -730,8 +690,8 @@ althea_status althea_mlp_create(const althea_mlp_desc* desc, althea_mlp** out) {
   };
   if (hipMalloc(&s->params, kMlpParams * 4) != hipSuccess || hipMalloc(&s->m, kMlpParams * 4) != hipSuccess ||
       hipMalloc(&s->v, kMlpParams * 4) != hipSuccess ||
-      hipMalloc(&s->wpartial, static_cast<size_t>(kWgradBlocks) * kMlpWeights * 4) != hipSuccess ||
-      hipMalloc(&s->bpartial, static_cast<size_t>(kFwdBlocks) * kMlpBiasPartial * 4) != hipSuccess) {
+      hipMalloc(&s->wpartial, static_cast<size_t>(kTrainBlocks) * kMlpWeights * 4) != hipSuccess ||
+      hipMalloc(&s->bpartial, static_cast<size_t>(kTrainBlocks) * kMlpBiasPartial * 4) != hipSuccess) {
     set_error("mlp_create: device allocation failed");
     return fail(ALTHEA_ERROR_OUT_OF_MEMORY);
   }
@@ -767,7 +727,6 @@ althea_status althea_mlp_destroy(althea_mlp* m) {
   (void)hipFree(s->m);
   (void)hipFree(s->v);
   (void)hipFree(s->weights_mem);
-  (void)hipFree(s->act_mem);
   (void)hipFree(s->wpartial);
   (void)hipFree(s->bpartial);
   (void)hipFree(s->cell_error);
@@ -806,10 +765,10 @@ althea_status althea_mlp_infer(const althea_mlp* m, const float* d_dir_rough, in
   fp.dir_rough = reinterpret_cast<const float4*>(d_dir_rough);
   fp.out = reinterpret_cast<float4*>(d_out);
   fp.count = count;
-  int tiles = (count + 15) / 16;
-  int blocks = std::min((tiles + 3) / 4, 4096);
-  hipLaunchKernelGGL(mlp_fwd_kernel<false>, dim3(blocks), dim3(256), 0, stream, fp);
-  return check_launch("mlp_fwd_kernel<infer>");
+  const int tiles = (count + 15) / 16;
+  const int blocks = std::min((tiles + 3) / 4, 4096);
+  hipLaunchKernelGGL(mlp_infer_kernel, dim3(blocks), dim3(256), 0, stream, fp);
+  return check_launch("mlp_infer_kernel");
 }
 
 althea_status althea_mlp_gradients(althea_mlp* m, const float* d_dir_rough, const float* d_targets, int count,

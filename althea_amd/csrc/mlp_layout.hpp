@@ -4,8 +4,6 @@
 
 #include <hip/hip_runtime.h>
 
-#include <cstddef>
-
 namespace althea {
 
 constexpr int kMlpIn = 28, kMlpHidden = 64, kMlpOut = 3;
@@ -79,12 +77,6 @@ __host__ __device__ inline int mlp_param_to_bias(int t) {
 struct MlpDeviceWeights {
   __bf16 *w1, *w2, *w3, *w4, *w2t, *w3t, *w4t;
   float *b1, *b2, *b3, *b4;
-};
-
-// Feature-major BF16 copies of one training batch (rows x stride samples).
-struct MlpActivations {
-  __bf16 *x, *h1, *h2, *h3, *dy, *dz1, *dz2, *dz3;  // 32, 64, 64, 64, 16, 64, 64, 64 rows
-  size_t stride;
 };
 
 }  // namespace althea
