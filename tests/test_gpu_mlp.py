@@ -90,6 +90,22 @@ def test_gradient_is_batch_size_independent_in_scale(torch):
     assert e < 2e-2, e
 
 
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 16384, 16385, 16384 + 129, 2 * 256 * 128 + 1])
+def test_gradients_at_block_edges(torch, n):
+    """Sizes around a wave's 16 samples, a block's 64 and 128, the change from
+    four waves to eight, and blocks that take a third step."""
+    net = M.PrefilterMLP(seed=9)
+    p = net.get_params()
+    dr, t = _batch(10 + n, n)
+    g, loss = net.gradients(torch.from_numpy(dr).cuda(), torch.from_numpy(t).cuda())
+    g = g.cpu().numpy().astype(np.float64)
+    ref_loss, ref = ol.mlp_loss_grad(p, dr, t, bf16=True)
+    assert abs(loss.item() - ref_loss) <= 1e-3 * ref_loss
+    for name, (lo, hi) in SLICES.items():
+        e = np.linalg.norm(g[lo:hi] - ref[lo:hi]) / max(np.linalg.norm(ref[lo:hi]), 1e-30)
+        assert e < 2e-2, (name, e)
+
+
 def test_adam_step_matches_closed_form(torch):
     net = M.PrefilterMLP(seed=7, lr=1e-3)
     p0 = net.get_params().astype(np.float64)
