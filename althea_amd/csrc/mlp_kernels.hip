@@ -79,15 +79,36 @@ struct FwdParams {
   int count;
 };
 
-// One 16-sample tile per iteration per wave, the forward operands in registers.
-__global__ __launch_bounds__(256) void mlp_infer_kernel(const FwdParams p) {
+// One 16-sample tile per iteration per wave.  The block copies the packed weights
+// into LDS once and its waves take their operands (88 registers: three waves a
+// SIMD) from there; each wave reading its 22 KB of operands from L2 by itself, in
+// rows 64 and 128 bytes apart, took as long as one or two tiles.  50 001 queries
+// 14.7 -> 8.4 us (back to back into one output), 200 000 38.6 -> 20.1, 1 000 000 99.5 -> 75.2, 4 000 000 316 ->
+// 297.  Persistent grids (256 blocks of 12 or 8 waves, 512 or 768 of 4) were no faster up to 200 000
+// and 5 to 24 % slower at 4 000 000.  Bound: VALU (encoding, SiLU).
+constexpr int kInferWaves = 4, kInferBlocks = 4096;
+
+__global__ __launch_bounds__(64 * kInferWaves) void mlp_infer_kernel(const FwdParams p) {
+  __shared__ MlpSmem sm;
   const int lane = threadIdx.x & 63;
   const int g = lane >> 4, n = lane & 15;
   const int wave = threadIdx.x >> 6;
   const int tiles = (p.count + 15) / 16;
+  mlp_stage_weights(sm, p.w, threadIdx.x, 64 * kInferWaves);
+  __syncthreads();
   MlpRegWeights r;
-  mlp_load_reg_weights(p.w, g, n, r);
-  for (int tile = blockIdx.x * 4 + wave; tile < tiles; tile += static_cast<int>(gridDim.x) * 4) {
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    r.a1[b] = sm.w1[mlp_swz32(16 * b + n, g)];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      r.a2[b][kb] = sm.w2[mlp_swz64(16 * b + n, 4 * kb + g)];
+      r.a3[b][kb] = sm.w3[mlp_swz64(16 * b + n, 4 * kb + g)];
+    }
+  }
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb) r.a4[kb] = sm.w4[mlp_swz64(n, 4 * kb + g)];
+  for (int tile = blockIdx.x * kInferWaves + wave; tile < tiles; tile += static_cast<int>(gridDim.x) * kInferWaves) {
     const int s = tile * 16 + n;
     const bool valid = s < p.count;
     const float4 q = valid ? p.dir_rough[s] : make_float4(0.f, 0.f, 1.f, 0.f);
@@ -768,8 +789,8 @@ althea_status althea_mlp_infer(const althea_mlp* m, const float* d_dir_rough, in
   fp.out = reinterpret_cast<float4*>(d_out);
   fp.count = count;
   const int tiles = (count + 15) / 16;
-  const int blocks = std::min((tiles + 3) / 4, 4096);
-  hipLaunchKernelGGL(mlp_infer_kernel, dim3(blocks), dim3(256), 0, stream, fp);
+  const int blocks = std::min((tiles + kInferWaves - 1) / kInferWaves, kInferBlocks);
+  hipLaunchKernelGGL(mlp_infer_kernel, dim3(blocks), dim3(64 * kInferWaves), 0, stream, fp);
   return check_launch("mlp_infer_kernel");
 }
 

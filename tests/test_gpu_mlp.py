@@ -56,6 +56,23 @@ def test_forward_matches_oracle(torch):
     assert np.all(out[:, 3] == 1.0)
 
 
+@pytest.mark.parametrize("n", [1, 15, 17, 63, 64, 65, 129, 4096 * 64 + 17])
+def test_forward_at_block_edges(torch, n):
+    """Sizes around a wave's 16 queries, a block's 64 and the largest grid
+    (its first blocks take a second tile)."""
+    net = M.PrefilterMLP(seed=11)
+    p = net.get_params()
+    dr, _ = _batch(12 + n, n)
+    guarded = torch.full((n + 64, 4), -7.0, device="cuda")
+    net.infer(torch.from_numpy(dr).cuda(), out=guarded[:n])
+    assert torch.all(guarded[n:] == -7.0)  # nothing past the batch
+    out = guarded[:n].cpu().numpy()
+    rows = np.arange(n) if n < 4096 else np.r_[0:512, n - 512:n]
+    err = np.abs(np.log(out[rows, :3].astype(np.float64)) - ol.mlp_forward(p, dr[rows], bf16=True))
+    assert err.max() < 2e-2 and err.mean() < 2e-3, (err.max(), err.mean())
+    assert np.all(out[:, 3] == 1.0)
+
+
 def test_gradients_match_oracle(torch):
     net = M.PrefilterMLP(seed=3)
     p = net.get_params()
