@@ -83,9 +83,10 @@ struct FwdParams {
 // into LDS once and its waves take their operands (88 registers: three waves a
 // SIMD) from there; each wave reading its 22 KB of operands from L2 by itself, in
 // rows 64 and 128 bytes apart, took as long as one or two tiles.  50 001 queries
-// 14.7 -> 8.4 us (back to back into one output), 200 000 38.6 -> 20.1, 1 000 000 99.5 -> 75.2, 4 000 000 316 ->
-// 297.  Persistent grids (256 blocks of 12 or 8 waves, 512 or 768 of 4) were no faster up to 200 000
-// and 5 to 24 % slower at 4 000 000.  Bound: VALU (encoding, SiLU).
+// 14.7 -> 8.4 us (back to back into one output), 200 000 38.6 -> 20.1, 1 000 000
+// 99.5 -> 75.2, 4 000 000 316 -> 297.  Persistent grids (256 blocks of 12 or 8
+// waves, 512 or 768 of 4) were no faster up to 200 000, and all but the first 4
+// to 16 % slower than the start at 4 000 000.  Bound: VALU (encoding, SiLU).
 constexpr int kInferWaves = 4, kInferBlocks = 4096;
 
 __global__ __launch_bounds__(64 * kInferWaves) void mlp_infer_kernel(const FwdParams p) {

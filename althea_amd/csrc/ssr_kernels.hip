@@ -44,6 +44,9 @@ constexpr int kSsrSteps = 128;        // RAYMARCH_STEPS, SSR.frag:80
 constexpr float kSsrStep = 0.005f;    // uv per step, SSR.frag:89
 constexpr float kSsrCone = 0.999f;    // cos of the accepted angle, SSR.frag:116-117
 constexpr float kSsrFar = 10000.0f;   // march target distance, SSR.frag:83
+// Bound of the relative error of the projection's sign test (ssr_capture_kernel):
+// its roundings add up to under 2^-20 of |view ray| + |EP| |m|, as do the point's.
+constexpr float kSignSlack = 1.0f / (1 << 18);
 
 struct SsrParams {
   const void* position;
@@ -62,6 +65,7 @@ struct SsrParams {
   float vp[16];                     // projection * view, column-major
   float view_z[4];                  // row 2 of the view matrix
   float eye[3];
+  float sign_slack;                 // kSignSlack * (bound of the view rays' length)
   float inv_far;                    // depth-plane value of an uncovered pixel
   float* depth;                     // depth plane in 8 x 4 texel blocks (taddr)
   int depth_tw;                     // blocks per block row, ceil(W / 8)
@@ -92,10 +96,12 @@ __device__ __forceinline__ float4 gb_bilinear(const void* plane, int W, int H, f
 }
 
 // Depth-plane layout: blocks of 8 x 4 texels, one 128-byte cache line each,
-// block rows of ceil(W / 8) blocks.  A bilinear footprint then falls in one
-// line 2 times in 3 (row-major rows always take two), and a wave's nearby
-// march points share lines in both directions.  Measured at 4K: 2.07 ms
-// against 2.43 ms row-major (4 x 8 blocks 2.24, 16 x 2 blocks 2.23).
+// block rows of ceil(W / 8) blocks.  The rays of a wave spread as they march, so
+// what the capture costs is the distinct lines its reads touch: a bilinear
+// footprint falls in one line 2 times in 3 (row-major rows always take two), and
+// nearby march points share lines in both directions.  Measured at 1080p, with
+// the pair reads below: frame 1245 us row-major, 1180 in these blocks, 1188 in
+// 16 x 2.
 __device__ __forceinline__ int taddr(int tw, int x, int y) {
   return (((y >> 2) * tw + (x >> 3)) << 5) + ((y & 3) << 3) + (x & 7);
 }
@@ -112,36 +118,43 @@ __global__ __launch_bounds__(256) void ssr_depth_kernel(const SsrParams p) {
   p.depth[taddr(p.depth_tw, x, y)] = q.w != 0.0f ? -1.0f / vz : p.inv_far;
 }
 
-// Bilinear CLAMP_TO_EDGE depth at uv: the four texel reads (depth_tap), then
-// the blend (depth_value).
-struct DepthTap {
-  float a0, b0, a1, b1, ax, ay;
-};
+// Two neighbouring texels of a block row (4-byte aligned).
+typedef float depth_pair __attribute__((ext_vector_type(2), aligned(4)));
 
-__device__ __forceinline__ DepthTap depth_tap(const float* __restrict__ d, int tw, int W, int H, float u, float v) {
+// Bilinear CLAMP_TO_EDGE depth at uv in [0, 1]^2.  Inside the frame a row's two
+// texels are one 8-byte read; the 1 in 8 footprints whose right column is the
+// next block's (+25 texels from the row's last) read that column again.
+__device__ __forceinline__ float depth_bilinear(const float* __restrict__ d, int tw, int W, int H, float u, float v) {
   const float x = fmaf(u, static_cast<float>(W), -0.5f), y = fmaf(v, static_cast<float>(H), -0.5f);
   const float fx = floorf(x), fy = floorf(y);
-  DepthTap t;
-  t.ax = x - fx;
-  t.ay = y - fy;
+  const float ax = x - fx, ay = y - fy;
   const int ix = static_cast<int>(fx), iy = static_cast<int>(fy);
-  const int x0 = min(max(ix, 0), W - 1), x1 = min(max(ix + 1, 0), W - 1);
-  const int y0 = min(max(iy, 0), H - 1), y1 = min(max(iy + 1, 0), H - 1);
-  // The other three texels from the first: +1 in a block, +25 into the next
-  // block; +8 in a block, one block row on (32 tw) less 3 rows of 8.
-  const int i00 = taddr(tw, x0, y0);
-  const int dx = x1 == x0 ? 0 : ((x0 & 7) == 7 ? 25 : 1);
-  const int dy = y1 == y0 ? 0 : ((y0 & 3) == 3 ? (tw << 5) - 24 : 8);
-  t.a0 = d[i00];
-  t.b0 = d[i00 + dx];
-  t.a1 = d[i00 + dy];
-  t.b1 = d[i00 + dy + dx];
-  return t;
-}
-
-__device__ __forceinline__ float depth_value(const DepthTap& t) {
-  const float top = fmaf(t.b0 - t.a0, t.ax, t.a0), bot = fmaf(t.b1 - t.a1, t.ax, t.a1);
-  return fmaf(bot - top, t.ay, top);
+  float a0, b0, a1, b1;
+  if (static_cast<unsigned>(ix) < static_cast<unsigned>(W - 1) &&
+      static_cast<unsigned>(iy) < static_cast<unsigned>(H - 1)) {
+    const int i = taddr(tw, ix, iy);
+    // +8 in a block, or one block row on (32 tw) less 3 rows of 8.
+    const int dy = (iy & 3) == 3 ? (tw << 5) - 24 : 8;
+    depth_pair t = *reinterpret_cast<const depth_pair*>(d + i);
+    depth_pair b = *reinterpret_cast<const depth_pair*>(d + (i + dy));
+    if ((ix & 7) == 7) {
+      t.y = d[i + 25];
+      b.y = d[i + dy + 25];
+    }
+    a0 = t.x;
+    b0 = t.y;
+    a1 = b.x;
+    b1 = b.y;
+  } else {
+    const int x0 = min(max(ix, 0), W - 1), x1 = min(max(ix + 1, 0), W - 1);
+    const int y0 = min(max(iy, 0), H - 1), y1 = min(max(iy + 1, 0), H - 1);
+    a0 = d[taddr(tw, x0, y0)];
+    b0 = d[taddr(tw, x1, y0)];
+    a1 = d[taddr(tw, x0, y1)];
+    b1 = d[taddr(tw, x1, y1)];
+  }
+  const float top = fmaf(b0 - a0, ax, a0), bot = fmaf(b1 - a1, ax, a1);
+  return fmaf(bot - top, ay, top);
 }
 
 // View ray through uv (SSR.vert:20, interpolated across the screen).
@@ -162,9 +175,9 @@ __device__ __forceinline__ f3 reconstruct(const SsrParams& p, float u, float v, 
   return mk(fmaf(ray.x, t, p.eye[0]), fmaf(ray.y, t, p.eye[1]), fmaf(ray.z, t, p.eye[2]));
 }
 
-// Tiles: 16 x 16 pixels per block, each wave an 8 x 8 quadrant, so a wave's
-// 64 rays start close together and their filtered depth reads share cache
-// lines.  The march reads far along the frame (mostly up it), so L2 reuse
+// Tiles: 16 x 16 pixels per block, each wave 16 x 4 of them, so a wave's 64 rays
+// start close together and their filtered depth reads share cache lines (1080p
+// frame: 1162 us, 1180 with 8 x 8 quadrants, 1196 with 32 x 2).  The march reads far along the frame (mostly up it), so L2 reuse
 // decides the speed: blocks are dealt to the 8 XCDs in turn (block b runs on
 // XCD b % 8), so XCD x takes the tiles of column band x, walking it column by
 // column.  Each XCD's L2 then holds one band's depth (about 4 MB at 4K)
@@ -185,8 +198,8 @@ __global__ __launch_bounds__(256) void ssr_capture_kernel(const SsrParams p, con
   if (j >= bw * tiles_y) return;  // the band has fewer tiles than the widest one
   const int tx = c0 + j / tiles_y, ty = j % tiles_y;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int px = tx * kSsrTile + (lane & 7) + 8 * (wave & 1);
-  const int py = ty * kSsrTile + (lane >> 3) + 8 * (wave >> 1);
+  const int px = tx * kSsrTile + (lane & 15);
+  const int py = ty * kSsrTile + (lane >> 4) + 4 * wave;
   const bool inside = px < p.width && py < p.height;
   const int idx = min(py, p.height - 1) * p.width + min(px, p.width - 1);
   const float4 pos = gb_load<kFmt>(p.position, idx);
@@ -223,42 +236,60 @@ __global__ __launch_bounds__(256) void ssr_capture_kernel(const SsrParams p, con
                    fmaf(p.rayv[2], sv, p.rayu[2] * su));
   const float vz0 = view_z_of(p, ray0), vzk = view_z_of(p, rk);
   const f3 EP = mk(p.eye[0] - P.x, p.eye[1] - P.y, p.eye[2] - P.z);
+  // The last step on the screen: uv0 + k step is monotone in k, so the march
+  // leaves the screen once (SSR.frag:102-104).
+  auto on_screen = [&](int k) {
+    const float u = fmaf(static_cast<float>(k), su, u0), v = fmaf(static_cast<float>(k), sv, v0);
+    return u >= 0.0f && u <= 1.0f && v >= 0.0f && v <= 1.0f;
+  };
+  const float ku = su != 0.0f ? ((su > 0.0f ? 1.0f : 0.0f) - u0) / su : 1e9f;
+  const float kv = sv != 0.0f ? ((sv > 0.0f ? 1.0f : 0.0f) - v0) / sv : 1e9f;
+  int last = 0;
+  if (active) {
+    last = static_cast<int>(fminf(fminf(ku, kv), static_cast<float>(kSsrSteps)));
+    if (!on_screen(last)) --last;
+    if (last < kSsrSteps && on_screen(last + 1)) ++last;
+  }
+  const float rp0 = dot(ray0, perp), rpk = dot(rk, perp), ep = dot(EP, perp);
+  const float ep_slack = kSignSlack * sqrtf(dot(EP, EP));
   bool hit = false;
   float hk = 0.0f;
   f3 Q = mk(0.0f, 0.0f, 0.0f), Nh = mk(0.0f, 0.0f, 0.0f);
   float prev = 0.0f;
-  // Lanes that left the march issue no loads (exec-masked): measured faster
-  // than marching every lane to the wave's end, with or without issuing the
-  // next step's loads ahead.
-  for (int i = 0; i < kSsrSteps; ++i) {
-    if (!__any(active)) break;
-    if (active) {
-      const float k = static_cast<float>(i + 1);
-      const float u = fmaf(k, su, u0), v = fmaf(k, sv, v0);
-      if (!(u >= 0.0f && u <= 1.0f && v >= 0.0f && v <= 1.0f)) {
-        active = false;  // off screen: SSR.frag:102-104
-      } else {
-        const DepthTap tap = depth_tap(p.depth, p.depth_tw, p.width, p.height, u, v);
-        const f3 ray = mk(fmaf(k, rk.x, ray0.x), fmaf(k, rk.y, ray0.y), fmaf(k, rk.z, ray0.z));
-        const float t = -rcp_fast(depth_value(tap) * fmaf(k, vzk, vz0));
-        const f3 dq = mk(fmaf(ray.x, t, EP.x), fmaf(ray.y, t, EP.y), fmaf(ray.z, t, EP.z));
-        const float rl = rsq_fast(dot(dq, dq));
-        const float proj = dot(dq, perp) * rl;
-        const float f = dot(dq, R) * rl;
-        if (i > 0 && proj * prev <= 0.0f && f > kSsrCone) {
-          const float4 n4 = gb_bilinear<kFmt>(p.normal, p.width, p.height, u, v);
-          const f3 nh = normalize_fast(mk(n4.x, n4.y, n4.z));
-          if (dot(nh, R) < 0.0f) {
-            hit = true;
-            active = false;
-            hk = k;
-            Nh = nh;
-            Q = mk(fmaf(ray.x, t, p.eye[0]), fmaf(ray.y, t, p.eye[1]), fmaf(ray.z, t, p.eye[2]));
-          }
-        }
-        prev = proj;
+  // What bounds the march is the lines its scattered reads bring into L1: with
+  // half the read instructions and 60 % of the VALU instructions, but row-major
+  // lines, it took 540 us; two steps' reads in flight or 8 waves a SIMD instead
+  // of 7 gain nothing.  1080p, shadows, 32 lights: 610 -> 453 us.
+  for (int i = 1; i <= last; ++i) {
+    const float k = static_cast<float>(i);
+    const float u = fmaf(k, su, u0), v = fmaf(k, sv, v0);
+    const float s = depth_bilinear(p.depth, p.depth_tw, p.width, p.height, u, v);
+    const float m = s * fmaf(k, vzk, vz0);
+    // The point lies at -ray / m from the eye; (-ray / m + EP) . perp has the
+    // sign of m (EP . perp m - ray . perp), both products affine in k.  Where
+    // that is clear of rounding and the last step's sign (prev, +-1), there is
+    // no crossing (SSR.frag:109) and the point is not formed: most steps.
+    const float e = fmaf(ep, m, -fmaf(k, rpk, rp0));
+    const float es = m < 0.0f ? -e : e;
+    if (es * prev > fmaf(ep_slack, fabsf(m), p.sign_slack)) continue;
+    const f3 ray = mk(fmaf(k, rk.x, ray0.x), fmaf(k, rk.y, ray0.y), fmaf(k, rk.z, ray0.z));
+    const float t = -rcp_fast(m);
+    const f3 dq = mk(fmaf(ray.x, t, EP.x), fmaf(ray.y, t, EP.y), fmaf(ray.z, t, EP.z));
+    const float rl = rsq_fast(dot(dq, dq));
+    const float proj = dot(dq, perp) * rl;
+    const float f = dot(dq, R) * rl;
+    if (i > 1 && proj * prev <= 0.0f && f > kSsrCone) {
+      const float4 n4 = gb_bilinear<kFmt>(p.normal, p.width, p.height, u, v);
+      const f3 nh = normalize_fast(mk(n4.x, n4.y, n4.z));
+      if (dot(nh, R) < 0.0f) {
+        hit = true;
+        hk = k;
+        Nh = nh;
+        Q = mk(fmaf(ray.x, t, p.eye[0]), fmaf(ray.y, t, p.eye[1]), fmaf(ray.z, t, p.eye[2]));
+        break;
       }
     }
+    prev = proj > 0.0f ? 1.0f : (proj < 0.0f ? -1.0f : proj);
   }
   const float hu = fmaf(hk, su, u0), hv = fmaf(hk, sv, v0);
   // environmentLitSample (SSR.frag:55-78): V = the reflected ray, occlusion 1.
@@ -388,6 +419,12 @@ althea_status launch_ssr_capture(const althea_gbuffer_view* g, const althea_ibl_
   p.inv_far = static_cast<float>(1.0 / far);
   p.depth = static_cast<float*>(workspace);
   p.depth_tw = (g->width + 7) / 8;
+  float rmax = 0.0f;
+  for (int c = 0; c < 3; ++c) {
+    const float r = std::fabs(p.ray0[c]) + std::fabs(p.rayu[c]) + std::fabs(p.rayv[c]);
+    rmax += r * r;
+  }
+  p.sign_slack = kSignSlack * std::sqrt(rmax);
   refl_chain(*reflection, p.out);
   const int n = g->width * g->height;
   const dim3 dgrid((n + 255) / 256);

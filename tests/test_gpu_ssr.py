@@ -129,6 +129,23 @@ def test_ssr_capture_odd_extents_match_oracle(torch, ibl, W, H):
         assert r["err"]["max"] < 2e-3, r
 
 
+@pytest.mark.parametrize("W,H", [(2, 1), (2, 2), (8, 4), (9, 5), (15, 16), (16, 17), (17, 3), (64, 40)])
+def test_ssr_capture_block_edges_match_oracle(torch, ibl, W, H):
+    """Extents at the edges of the depth plane's 8 x 4 blocks, where a pair of
+    columns crosses blocks or the clamp takes over, on the wall scene (whose
+    short rays hit at any extent) and on the heightfield."""
+    ibl_res, _ = ibl
+    wall = wall_scene(W=W, H=H)[0]
+    wall.lights = np.array([[0.0, 2.0, -4.0, 0.0, 20.0, 20.0, 20.0, 0.0]], np.float32)
+    for scene in (wall, aa.synth.scene(seed=SEED0 + 26, width=W, height=H, lights=2)):
+        refl = _capture(torch, scene, ibl_res)
+        got = refl.level(0).cpu().numpy().reshape(-1, 4).astype(np.float64)
+        r = _compare_capture(scene, ibl_res.views_numpy(), got, _all_pixels(scene))
+        assert r["disagree_clear"] == 0, r
+        if r["err"] is not None:
+            assert r["err"]["max"] < 2e-3, r
+
+
 def test_ssr_capture_wall_scene_matches_oracle(torch, ibl):
     ibl_res, _ = ibl
     scene, use_f, _, _ = wall_scene(W=320, H=180)
