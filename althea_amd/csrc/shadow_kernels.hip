@@ -265,12 +265,8 @@ __global__ __launch_bounds__(256) void shadow_raster_kernel(const ShadowParams p
 }
 
 // The scheduled path: every item's six boxes, their total texels as its run
-// of slots, then a grid of waves over equal contiguous slot ranges (the
-// G-buffer rasterizer's scheme), so boxes of every size cost the same per
-// texel.  A wave finds the items of its 64 slots from a window of 64
-// consecutive prefix sums (one coalesced load) by a binary search across the
-// lanes, instead of dependent loads per slot; the item's edge functions are
-// rebuilt per lane when its item changes.
+// of slots, then a grid of waves over equal contiguous ranges of work, so boxes
+// of every size cost the same per texel.
 __global__ __launch_bounds__(kSlotBlock) void shadow_slot_setup_kernel(const ShadowParams p) {
   __shared__ unsigned long long wave_total[kSlotBlock / 64];
   const int item = blockIdx.x * kSlotBlock + threadIdx.x;
@@ -312,66 +308,199 @@ __global__ __launch_bounds__(kSlotScan) void shadow_scan_kernel(unsigned long lo
   slot_scan_blocks(blocks, n, total, sums);
 }
 
-__global__ __launch_bounds__(256) void shadow_offset_kernel(unsigned long long* __restrict__ offsets,
-                                                            const unsigned long long* __restrict__ blocks, int n) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) offsets[t] += blocks[t / kSlotBlock];
+// The face whose texels hold texel `local` of an item on several faces, and
+// that texel's number on it.
+__device__ __forceinline__ uint2 shadow_box_of(const uint2* __restrict__ item_boxes, unsigned& local, int& face) {
+  const uint4* bx = reinterpret_cast<const uint4*>(item_boxes);
+  const uint4 q0 = bx[0], q1 = bx[1], q2 = bx[2];
+  const uint2 boxes[6] = {make_uint2(q0.x, q0.y), make_uint2(q0.z, q0.w), make_uint2(q1.x, q1.y),
+                          make_uint2(q1.z, q1.w), make_uint2(q2.x, q2.y), make_uint2(q2.z, q2.w)};
+  face = 0;
+  uint2 b = boxes[0];
+  bool found = false;
+#pragma unroll
+  for (int f = 0; f < 6; ++f) {
+    const unsigned a = (boxes[f].y & 0xffffu) * (boxes[f].y >> 16);
+    if (!found && local < a) {
+      face = f, b = boxes[f], found = true;
+    } else if (!found) {
+      local -= a;
+    }
+  }
+  return b;
 }
+
+// First slot of item i, and for i = n the slot total.
+__device__ __forceinline__ unsigned long long shadow_first_slot(const ShadowSlots& q, int i, int n) {
+  return q.offsets[i] + (i < n ? q.blocks[i / kSlotBlock] : 0ull);
+}
+
+// This wave's range of slots and the item that holds its first.  The waves share
+// slots and items evenly, an item counting as kItemSlots slots beside its own: by
+// slots alone, a wave whose items are small or culled walks many windows of them
+// (64 lights x 32 768 triangles at 256: 264 us a call against 216, at 2 and 4
+// alike; 8: 223, 16: 235).  Both ends are searched together, 64 probes a round
+// (four rounds for 2 M items, where one probe a round takes 21 dependent reads).
+// A wave takes at least kWaveSlots: 16 384 searches cost more than small draws (1
+// light, 6 000 triangles: 34 us without the bound, 28 with 256, 29 with 512, 34
+// with the first 1024 tried).
+constexpr unsigned long long kItemSlots = 4, kWaveSlots = 256;
+
+__device__ __forceinline__ void shadow_wave_range(const ShadowSlots& q, int n, int& item, unsigned long long& begin,
+                                                  unsigned long long& end) {
+  const unsigned waves = gridDim.x * (blockDim.x >> 6);
+  const unsigned wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63;
+  const unsigned long long work = q.offsets[n] + kItemSlots * static_cast<unsigned long long>(n);
+  const unsigned long long share = (work + waves - 1) / waves;
+  const unsigned long long per = share > kWaveSlots ? share : kWaveSlots;
+  const unsigned long long at[2] = {wave * per, wave * per + per};
+  item = 0;
+  begin = end = 0;
+  if (at[0] >= work) return;
+  int lo[2] = {0, 0}, hi[2] = {n, n};
+  // 64 probes a round, both ends of the range at a time.
+  while (hi[0] - lo[0] > 1 || hi[1] - lo[1] > 1) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int step = (hi[e] - lo[e] + 63) >> 6;
+      const int i = lo[e] + lane * step;
+      const bool before =
+          i < hi[e] && shadow_first_slot(q, i, n) + kItemSlots * static_cast<unsigned long long>(i) <= at[e];
+      const int count = __builtin_popcountll(__builtin_amdgcn_ballot_w64(before));
+      const int found = lo[e] + max(count - 1, 0) * step;
+      hi[e] = min(found + step, hi[e]);
+      lo[e] = found;
+    }
+  }
+  unsigned long long slot[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const unsigned long long first = slot_uniform(shadow_first_slot(q, lo[e], n));
+    const unsigned long long area = slot_uniform(shadow_first_slot(q, lo[e] + 1, n)) - first;
+    const unsigned long long in = at[e] - (first + kItemSlots * static_cast<unsigned long long>(lo[e]));
+    slot[e] = first + (in < area ? in : area);
+  }
+  item = lo[0];
+  begin = slot[0];
+  end = slot[1];
+}
+
+// The box of an item with `area` texels on one face, or its first face's box
+// and kManyFaces.
+constexpr unsigned kManyFaces = 6;
+
+__device__ __forceinline__ uint2 shadow_first_box(const uint2* __restrict__ item_boxes, unsigned area, unsigned& face) {
+  const uint4* bx = reinterpret_cast<const uint4*>(item_boxes);
+  const uint4 q0 = bx[0], q1 = bx[1], q2 = bx[2];
+  const uint2 boxes[6] = {make_uint2(q0.x, q0.y), make_uint2(q0.z, q0.w), make_uint2(q1.x, q1.y),
+                          make_uint2(q1.z, q1.w), make_uint2(q2.x, q2.y), make_uint2(q2.z, q2.w)};
+  uint2 b = boxes[0];
+  face = 0;
+#pragma unroll
+  for (int f = 5; f >= 0; --f)
+    if (boxes[f].y != 0) face = static_cast<unsigned>(f), b = boxes[f];
+  if ((b.y & 0xffffu) * (b.y >> 16) != area) face = kManyFaces;
+  return b;
+}
+
+// Windows of 64 items: lane k sets item w0 + k up once (edge functions, first
+// box) in LDS, then the window's slots are taken 64 a step, each lane with its
+// item's record from there.  Rebuilding the item in every lane at every step was
+// half of the kernel's vector instructions (64 lights x 32 768 triangles, 256^2
+// faces: 232 us of raster; a draw of it 307 -> 215 us with the even split above
+// and no pass over the offsets).  Bound: VALU issue (100 instructions a step) and
+// the window's chain of offset, box and vertex reads.  21.5 KB a block: seven
+// waves a SIMD.
+template <bool kAlpha>
+struct ShadowStage {          // one wave's window of 64 items
+  float4 n0_det[64];          // n0, det
+  float4 n1_lo[64];           // n1, low word of the cube's first texel
+  float4 n2_hi[64];           // n2, high word
+  float4 n_inv[64];           // n, 1 / box width
+  uint4 box[64];              // x0 | y0 << 16, w | h << 16, face, first slot (low word)
+  int tri[kAlpha ? 64 : 1];   // triangle
+  int mark[64];               // items that start in this step's slots
+};
 
 template <bool kAlpha>
 __global__ __launch_bounds__(256) void shadow_slot_raster_kernel(const ShadowParams p) {
-  const unsigned long long* __restrict__ offsets = p.slots.offsets;
+  __shared__ ShadowStage<kAlpha> stages[4];
+  ShadowStage<kAlpha>& st = stages[threadIdx.x >> 6];
+  const int lane = threadIdx.x & 63;
   const int n = p.light_count * p.triangle_count;
-  const unsigned long long total = offsets[n];
+  int w0;
   unsigned long long begin, end;
-  slot_range(total, begin, end);
-  if (begin >= end) return;
+  shadow_wave_range(p.slots, n, w0, begin, end);
   const int S = p.size;
   const float inv_s = 1.0f / static_cast<float>(S);
   const size_t cube_floats = static_cast<size_t>(6) * (S + 2) * (S + 2);
-  int w0 = slot_find(offsets, 0, n, begin);  // the item holding `begin`
-  int cur = -1, light = 0, t = 0;
-  ShadowTri tri{};
-  for (unsigned long long base = begin; base < end; base += 64) {
-    unsigned item_start;
-    const int item = slot_step_items(offsets, n, base, end, w0, item_start);
-    if (item < 0) continue;
-    unsigned local = static_cast<unsigned>(base + (threadIdx.x & 63)) - item_start;
-    const uint4* bx = reinterpret_cast<const uint4*>(p.slots.boxes + static_cast<size_t>(item) * 6);
-    const uint4 q0 = bx[0], q1 = bx[1], q2 = bx[2];
-    const uint2 boxes[6] = {make_uint2(q0.x, q0.y), make_uint2(q0.z, q0.w), make_uint2(q1.x, q1.y),
-                            make_uint2(q1.z, q1.w), make_uint2(q2.x, q2.y), make_uint2(q2.z, q2.w)};
-    int face = 0;
-    uint2 b = boxes[0];
-    bool found = false;
-#pragma unroll
-    for (int f = 0; f < 6; ++f) {  // the face whose texels hold `local`
-      const unsigned a = (boxes[f].y & 0xffffu) * (boxes[f].y >> 16);
-      if (!found && local < a) {
-        face = f, b = boxes[f], found = true;
-      } else if (!found) {
-        local -= a;
-      }
-    }
-    if (!found) continue;  // not reached: the runs are the boxes' areas
-    // Row and column of `local` in the box: local < w h <= 2^24 is exact in
-    // FP32, so the reciprocal's row is off by at most one, corrected here.
-    const unsigned w = b.y & 0xffffu;
-    int row = static_cast<int>(static_cast<float>(local) * rcp_fast(static_cast<float>(w)));
-    int col = static_cast<int>(local) - row * static_cast<int>(w);
-    if (col < 0) {
-      --row, col += static_cast<int>(w);
-    } else if (col >= static_cast<int>(w)) {
-      ++row, col -= static_cast<int>(w);
-    }
-    const int i = static_cast<int>(b.x & 0xffffu) + col, j = static_cast<int>(b.x >> 16) + row;
-    if (item != cur) {
+  for (unsigned long long slot = begin; slot < end; w0 += 64) {
+    // Lane k: item w0 + k, its slots [first, next).
+    const unsigned long long first = shadow_first_slot(p.slots, min(w0 + lane, n), n);
+    const unsigned long long next = shadow_first_slot(p.slots, min(w0 + lane + 1, n), n);
+    const unsigned long long last = slot_uniform(__shfl(next, 63));
+    const unsigned long long window_end = last < end ? last : end;
+    if (window_end <= slot) continue;  // 64 items without texels
+    const bool live = next > first && next > slot && first < window_end;
+    if (live) {
+      int light, t;
       f3 v[3];
-      bool live;
-      shadow_item(p, item, light, v, tri, live, t);
-      cur = item;
+      ShadowTri tri;
+      bool front;
+      shadow_item(p, w0 + lane, light, v, tri, front, t);
+      const uint2* boxes = p.slots.boxes + static_cast<size_t>(w0 + lane) * 6;
+      unsigned face = 0;
+      const uint2 b = shadow_first_box(boxes, static_cast<unsigned>(next - first), face);
+      const unsigned long long at = static_cast<unsigned long long>(light) * cube_floats;
+      st.n0_det[lane] = make_float4(tri.n0.x, tri.n0.y, tri.n0.z, tri.det);
+      st.n1_lo[lane] = make_float4(tri.n1.x, tri.n1.y, tri.n1.z, __uint_as_float(static_cast<unsigned>(at)));
+      st.n2_hi[lane] = make_float4(tri.n2.x, tri.n2.y, tri.n2.z, __uint_as_float(static_cast<unsigned>(at >> 32)));
+      st.n_inv[lane] = make_float4(tri.n.x, tri.n.y, tri.n.z, rcp_fast(static_cast<float>(b.y & 0xffffu)));
+      st.box[lane] = make_uint4(b.x, b.y, face, static_cast<unsigned>(first));
+      if (kAlpha) st.tri[lane] = t;
     }
-    shadow_texel<kAlpha>(tri, face, i, j, S, inv_s, p.cubes + light * cube_floats, kAlpha ? p.alpha + t : nullptr);
+    for (unsigned long long base = slot; base < window_end; base += 64) {
+      // The item of each slot: those that start in this step mark their first
+      // slot, and a running maximum from the item that holds `base` carries
+      // them on.
+      const unsigned long long rel = first - base;
+      st.mark[lane] = -1;
+      wave_lds_sync();
+      if (live && rel < 64) st.mark[rel] = lane;
+      wave_lds_sync();
+      const int held = 63 - __builtin_clzll(__builtin_amdgcn_ballot_w64(live && first <= base));
+      const int k = max(wave_max_scan(st.mark[lane]), held);
+      if (base + lane >= window_end) continue;
+      const uint4 bx = st.box[k];
+      const float4 r0 = st.n0_det[k], r1 = st.n1_lo[k], r2 = st.n2_hi[k], r3 = st.n_inv[k];
+      unsigned local = static_cast<unsigned>(base) + lane - bx.w;
+      uint2 b = make_uint2(bx.x, bx.y);
+      int face = static_cast<int>(bx.z);
+      float inv_w = r3.w;
+      if (bx.z == kManyFaces) {
+        b = shadow_box_of(p.slots.boxes + static_cast<size_t>(w0 + k) * 6, local, face);
+        inv_w = rcp_fast(static_cast<float>(b.y & 0xffffu));
+      }
+      // Row and column of `local` in the box: local < w h <= 2^24 is exact in
+      // FP32, so the reciprocal's row is off by at most one, corrected here.
+      const int w = static_cast<int>(b.y & 0xffffu);
+      int row = static_cast<int>(static_cast<float>(local) * inv_w);
+      int col = static_cast<int>(local) - row * w;
+      if (col < 0) {
+        --row, col += w;
+      } else if (col >= w) {
+        ++row, col -= w;
+      }
+      const int i = static_cast<int>(b.x & 0xffffu) + col, j = static_cast<int>(b.x >> 16) + row;
+      ShadowTri tri;
+      tri.n0 = mk(r0.x, r0.y, r0.z), tri.n1 = mk(r1.x, r1.y, r1.z), tri.n2 = mk(r2.x, r2.y, r2.z);
+      tri.n = mk(r3.x, r3.y, r3.z);
+      tri.det = r0.w;
+      float* cube = p.cubes + ((static_cast<size_t>(__float_as_uint(r2.w)) << 32) | __float_as_uint(r1.w));
+      shadow_texel<kAlpha>(tri, face, i, j, S, inv_s, cube, kAlpha ? p.alpha + st.tri[k] : nullptr);
+    }
+    slot = window_end;
   }
 }
 
@@ -454,9 +583,6 @@ static althea_status shadow_passes(ShadowParams& p, void* workspace, hipStream_t
     if ((st = check_launch("shadow_slot_setup_kernel")) != ALTHEA_OK) return st;
     hipLaunchKernelGGL(shadow_scan_kernel, dim3(1), dim3(kSlotScan), 0, s, p.slots.blocks, nb, p.slots.offsets + ni);
     if ((st = check_launch("shadow_scan_kernel")) != ALTHEA_OK) return st;
-    hipLaunchKernelGGL(shadow_offset_kernel, dim3((ni + 255) / 256), dim3(256), 0, s, p.slots.offsets,
-                       p.slots.blocks, ni);
-    if ((st = check_launch("shadow_offset_kernel")) != ALTHEA_OK) return st;
     if (alpha)
       hipLaunchKernelGGL(shadow_slot_raster_kernel<true>, dim3(4096), dim3(256), 0, s, p);
     else

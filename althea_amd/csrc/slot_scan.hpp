@@ -130,6 +130,17 @@ __device__ __forceinline__ int slot_step_items(const unsigned long long* __restr
   return item;
 }
 
+// Inclusive running maximum over the lanes of a wave (row shifts, then the last
+// lane of a row to the rows after it).
+__device__ __forceinline__ int wave_max_scan(int x) {
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x111, 0xf, 0xf, false));  // row_shr:1
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x112, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x114, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x118, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x142, 0xa, 0xf, false));  // row_bcast:15 into rows 1, 3
+  return max(x, __builtin_amdgcn_update_dpp(x, x, 0x143, 0xc, 0xf, false));  // row_bcast:31 into rows 2, 3
+}
+
 __device__ __forceinline__ unsigned long long slot_uniform(unsigned long long v) {
   const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(v));
   const unsigned hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(v >> 32));

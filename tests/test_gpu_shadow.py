@@ -112,6 +112,31 @@ def test_no_triangles_and_back_faces(torch):
     assert r["hits"] > 0 and r["hit_disagree"] == 0 and r["err"]["max"] < 1e-6, r
 
 
+@pytest.mark.parametrize("tris,lights_n,size,scale", [(1, 1, 1, 3.0), (63, 1, 16, 1.0), (64, 1, 33, 1.0),
+                                                      (65, 2, 64, 1.0), (257, 3, 64, 0.3), (1500, 5, 48, 0.02),
+                                                      (40, 2, 512, 8.0)])
+def test_scheduled_windows_match_the_lane_walk(torch, tris, lights_n, size, scale):
+    """The scheduled raster runs the lane walk's texel tests, so it gives its
+    bits: item counts around its windows of 64, runs of culled items longer than
+    a window, boxes of no texel, of many faces and larger than a wave's share."""
+    rng = np.random.default_rng(tris)
+    lights = np.concatenate([rng.uniform(-0.5, 0.5, (lights_n, 3)), np.zeros((lights_n, 1)),
+                             np.full((lights_n, 3), 4.0), np.zeros((lights_n, 1))], 1).astype(np.float32)
+    d = rng.normal(size=(tris, 3))
+    centre = d / np.linalg.norm(d, axis=1, keepdims=True) * rng.uniform(1.5, 6.0, (tris, 1))
+    pos = (centre[:, None, :] + scale * rng.normal(size=(tris, 3, 3))).astype(np.float32)
+    n = np.cross(pos[:, 1] - pos[:, 0], pos[:, 2] - pos[:, 0])
+    back = (n * pos[:, 0]).sum(1) > 0
+    pos[back] = pos[back][:, ::-1]  # facing the origin ...
+    pos[tris // 4:tris // 2] = pos[tris // 4:tris // 2, ::-1]  # ... but for a run of them
+    idx = np.arange(3 * tris, dtype=np.uint32).reshape(-1, 3)
+    _, walk = _gpu_cubes(torch, pos.reshape(-1, 3), idx, lights, size, scheduled=False)
+    _, got = _gpu_cubes(torch, pos.reshape(-1, 3), idx, lights, size)
+    if tris > 1:  # the single triangle covers no texel centre of the 1 x 1 faces
+        assert (walk < 1.0).any()
+    np.testing.assert_array_equal(got.view(np.uint32), walk.view(np.uint32))
+
+
 @pytest.mark.parametrize("size", [1, 2, 256])
 def test_large_occluders_span_whole_faces(torch, size):
     """A box of six inward-facing squares around the light: every face of
