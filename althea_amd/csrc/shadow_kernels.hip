@@ -341,9 +341,9 @@ __device__ __forceinline__ unsigned long long shadow_first_slot(const ShadowSlot
 // (64 lights x 32 768 triangles at 256: 264 us a call against 216, at 2 and 4
 // alike; 8: 223, 16: 235).  Both ends are searched together, 64 probes a round
 // (four rounds for 2 M items, where one probe a round takes 21 dependent reads).
-// A wave takes at least kWaveSlots: 16 384 searches cost more than small draws (1
-// light, 6 000 triangles: 34 us without the bound, 28 with 256, 29 with 512, 34
-// with the first 1024 tried).
+// A wave takes at least kWaveSlots, as 16 384 searches cost more than small draws
+// (1 light, 5 000 triangles: 34.5 us without the bound, 28.7 with 256, 29.1 with
+// 512, 34.7 with 1 024).
 constexpr unsigned long long kItemSlots = 4, kWaveSlots = 256;
 
 __device__ __forceinline__ void shadow_wave_range(const ShadowSlots& q, int n, int& item, unsigned long long& begin,
@@ -406,12 +406,11 @@ __device__ __forceinline__ uint2 shadow_first_box(const uint2* __restrict__ item
 
 // Windows of 64 items: lane k sets item w0 + k up once (edge functions, first
 // box) in LDS, then the window's slots are taken 64 a step, each lane with its
-// item's record from there.  Rebuilding the item in every lane at every step was
-// half of the kernel's vector instructions (64 lights x 32 768 triangles, 256^2
-// faces: 232 us of raster; a draw of it 307 -> 215 us with the even split above
-// and no pass over the offsets).  Bound: VALU issue (100 instructions a step) and
-// the window's chain of offset, box and vertex reads.  21.5 KB a block: seven
-// waves a SIMD.
+// item's record from there, where every lane used to rebuild its item at every
+// step.  64 lights x 32 768 triangles, 256^2 faces: raster 232 -> 144 us, the call
+// 340 -> 230 (with the even split above and no pass over the offsets).  Bound:
+// VALU issue and the window's chain of offset, box and vertex reads.  21.5 KB of
+// LDS a block: seven waves a SIMD.
 template <bool kAlpha>
 struct ShadowStage {          // one wave's window of 64 items
   float4 n0_det[64];          // n0, det
