@@ -126,9 +126,8 @@ ALTHEA_API althea_status althea_env_sample(const float* d_pyramid, int width, in
  * `samples` Hammersley half vectors, alpha = roughness, NdotL-weighted mean,
  * source LOD from the sample pdf.  d_cube holds althea_cube_texels(size, mips)
  * float4.  Sums over samples are FP64 unless ALTHEA_PRECOMPUTE_FP32_SUMS.  The
- * call's stream-ordered workspace holds the sample tables and a padded copy of
- * the pyramid (each level with its wrap-around neighbours stored around it,
- * about 1.34x the pyramid) that the sample loop reads. */
+ * call's stream-ordered workspace holds the sample tables; the sample loop reads
+ * the pyramid itself, its coarse levels through LDS. */
 ALTHEA_API althea_status althea_prefilter_cube(const float* d_pyramid, int env_width, int env_height,
                                                int size, int mips, int samples, unsigned flags,
                                                float* d_cube, hipStream_t stream);
@@ -145,9 +144,8 @@ ALTHEA_API size_t althea_prefilter_cube_scratch_bytes(int mips, int samples);
  * per-roughness GGX sample tables live in a fixed 4 MiB device array that the
  * library holds on every GPU it runs on until the process ends; requests whose
  * tables exceed ALTHEA_PREFILTER_SCRATCH_MAX_BYTES are rejected with
- * ALTHEA_ERROR_INVALID_ARGUMENT before any device work.  It reads the pyramid
- * itself, where althea_prefilter_cube reads its padded copy; the cube written
- * is bit-identical to althea_prefilter_cube's.  Every call on one GPU shares that
+ * ALTHEA_ERROR_INVALID_ARGUMENT before any device work.  The cube written is
+ * bit-identical to althea_prefilter_cube's.  Every call on one GPU shares that
  * array: calls that overlap on one GPU (other streams, other threads) race. */
 ALTHEA_API althea_status althea_prefilter_cube_noalloc(const float* d_pyramid, int env_width, int env_height,
                                                        int size, int mips, int samples, unsigned flags,
@@ -162,8 +160,9 @@ ALTHEA_API althea_status althea_prefilter_points(const float* d_pyramid, int env
 /* Diffuse irradiance cube (GenIrradianceMap.comp:106-155 per output texel):
  * theta_samples x int(H*theta_samples/W) Riemann sum (300 in the reference)
  * at source LOD log2(W/theta_samples).  d_cube holds 6*size*size float4.  The
- * call's stream-ordered workspace holds the angle tables and a padded copy of
- * the two source levels read. */
+ * call's stream-ordered workspace holds the angle tables and a copy of the two
+ * source levels read (blended, and for sample counts that allow it folded over
+ * the sphere's sign flips). */
 ALTHEA_API althea_status althea_irradiance_cube(const float* d_pyramid, int env_width, int env_height,
                                                 int size, int theta_samples, unsigned flags, float* d_cube,
                                                 hipStream_t stream);
