@@ -363,13 +363,15 @@ __device__ __forceinline__ void shadow_wave_range(const ShadowSlots& q, int n, i
   while (hi[0] - lo[0] > 1 || hi[1] - lo[1] > 1) {
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
-      const int step = (hi[e] - lo[e] + 63) >> 6;
-      const int i = lo[e] + lane * step;
+      // Unsigned, and no sum past hi: n may be 2^31 - 1.
+      const int step = ((hi[e] - lo[e] - 1) >> 6) + 1;
+      const unsigned i = static_cast<unsigned>(lo[e]) + static_cast<unsigned>(lane * step);
       const bool before =
-          i < hi[e] && shadow_first_slot(q, i, n) + kItemSlots * static_cast<unsigned long long>(i) <= at[e];
+          i < static_cast<unsigned>(hi[e]) &&
+          shadow_first_slot(q, static_cast<int>(i), n) + kItemSlots * static_cast<unsigned long long>(i) <= at[e];
       const int count = __builtin_popcountll(__builtin_amdgcn_ballot_w64(before));
       const int found = lo[e] + max(count - 1, 0) * step;
-      hi[e] = min(found + step, hi[e]);
+      hi[e] = found + min(step, hi[e] - found);
       lo[e] = found;
     }
   }
@@ -434,10 +436,10 @@ __global__ __launch_bounds__(256) void shadow_slot_raster_kernel(const ShadowPar
   const int S = p.size;
   const float inv_s = 1.0f / static_cast<float>(S);
   const size_t cube_floats = static_cast<size_t>(6) * (S + 2) * (S + 2);
-  for (unsigned long long slot = begin; slot < end; w0 += 64) {
+  for (unsigned long long slot = begin; slot < end; w0 += min(64, n - w0)) {
     // Lane k: item w0 + k, its slots [first, next).
-    const unsigned long long first = shadow_first_slot(p.slots, min(w0 + lane, n), n);
-    const unsigned long long next = shadow_first_slot(p.slots, min(w0 + lane + 1, n), n);
+    const unsigned long long first = shadow_first_slot(p.slots, w0 + min(lane, n - w0), n);
+    const unsigned long long next = shadow_first_slot(p.slots, w0 + min(lane + 1, n - w0), n);
     const unsigned long long last = slot_uniform(__shfl(next, 63));
     const unsigned long long window_end = last < end ? last : end;
     if (window_end <= slot) continue;  // 64 items without texels
