@@ -20,6 +20,7 @@
 
 #include "device_math.hpp"
 #include "internal.hpp"
+#include "irradiance_launch.hpp"
 #include "precise_lookup.hpp"
 #include "prefilter_common.hpp"
 
@@ -1120,7 +1121,7 @@ struct FoldParams {
   uint32_t rowbytes;  // kFoldNodeBytes (cols + 2)
   int size;
   int theta_samples, phi_samples;
-  int theta_steps, steps;  // 8-azimuth steps per polar group, steps in all
+  int theta_steps, polar_steps;  // groups of 8 azimuths and of 8 polar rows
   double scale;            // pi / theta_samples / phi_samples
 };
 
@@ -1166,7 +1167,7 @@ __global__ __launch_bounds__(64 * kFoldWaves) void irradiance_fold_kernel(const 
   extern __shared__ float4 s_tab[];  // the polar rows, then the azimuth rows (kLds)
   __shared__ float4 s_rec[kFoldWaves][64];
   __shared__ T s_part[kFoldWaves][3][8];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   float2* s_theta = reinterpret_cast<float2*>(s_tab + p.phi_samples);
   if (kLds) {
     for (int i = threadIdx.x; i < p.phi_samples; i += 64 * kFoldWaves) s_tab[i] = phi_glob[i];
@@ -1188,10 +1189,10 @@ __global__ __launch_bounds__(64 * kFoldWaves) void irradiance_fold_kernel(const 
   float4* rec = s_rec[wave];
   T ar = 0, ag = 0, ab = 0;
   float sr = 0.0f, sg = 0.0f, sb = 0.0f;
-  int done = 0;
-  for (int step = wave; step < p.steps; step += kFoldWaves) {
-    const int pg = step / p.theta_steps, as = step - pg * p.theta_steps;
-    const int i = as * 8 + (lane & 7), j = pg * 8 + (lane >> 3);
+  unsigned done = 0;
+  for (FoldStep st = fold_advance({0, 0}, wave, p.theta_steps); st.polar < p.polar_steps;
+       st = fold_advance(st, kFoldWaves, p.theta_steps)) {
+    const int i = st.azimuth * 8 + (lane & 7), j = st.polar * 8 + (lane >> 3);
     const bool valid = i < p.theta_samples && j < p.phi_samples;
     const float2 th = theta_tab[min(i, p.theta_samples - 1)];
     const float4 ph = phi_tab[min(j, p.phi_samples - 1)];
@@ -1295,7 +1296,7 @@ static althea_status launch_irradiance_fold(const float* pyr, const PyramidGeome
   p.theta_samples = theta_samples;
   p.phi_samples = phi;
   p.theta_steps = (theta_samples + 7) / 8;
-  p.steps = p.theta_steps * ((phi + 7) / 8);
+  p.polar_steps = (phi + 7) / 8;
   p.scale = M_PI / theta_samples / phi;
   const int half = (size + 1) / 2;
   const bool f64 = !(flags & ALTHEA_PRECOMPUTE_FP32_SUMS);
