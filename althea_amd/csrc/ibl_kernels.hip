@@ -865,25 +865,26 @@ __device__ __forceinline__ void irradiance_column(const char* __restrict__ gpyr,
 // Azimuth tables of up to this many rows are read from LDS (kLds): the
 // table's loads then leave the texture data return, which bounds the kernel.
 constexpr int kIrrThetaLdsMax = 4096;
+constexpr int kIrrWaves = 4;
 
 template <bool kF64Sums, bool kLds>
-__global__ __launch_bounds__(256) void irradiance_cube_kernel(const char* __restrict__ gpyr,
-                                                              const float2* __restrict__ theta_glob,
-                                                              const float4* __restrict__ phi_tab,
-                                                              const IrradianceParams p, float4* __restrict__ cube) {
+__global__ __launch_bounds__(64 * kIrrWaves) void irradiance_cube_kernel(const char* __restrict__ gpyr,
+                                                                         const float2* __restrict__ theta_glob,
+                                                                         const float4* __restrict__ phi_tab,
+                                                                         const IrradianceParams p, float4* __restrict__ cube) {
   extern __shared__ float2 s_theta[];  // theta_samples rows when kLds
   if (kLds) {
-    for (int i = threadIdx.x; i < p.theta_samples; i += 256) s_theta[i] = theta_glob[i];
+    for (int i = threadIdx.x; i < p.theta_samples; i += 64 * kIrrWaves) s_theta[i] = theta_glob[i];
     __syncthreads();
   }
   const float2* theta_tab = kLds ? s_theta : theta_glob;
   const int S = p.size;
-  const int texel = blockIdx.x * 4 + static_cast<int>(threadIdx.x >> 6);
-  if (texel >= 6 * S * S) return;  // whole waves; no block barrier follows
+  const int rem = blockIdx.x * kIrrWaves + static_cast<int>(threadIdx.x >> 6);
+  if (rem >= S * S) return;  // whole waves; no block barrier follows
   const int lane = threadIdx.x & 63;
-  const int face = texel / (S * S);
-  const int rem = texel - face * S * S;
+  const int face = blockIdx.y;
   const int y = rem / S, x = rem - y * S;
+  const size_t texel = static_cast<size_t>(face) * S * S + rem;
   const Frame fr = local_to_world(cube_texel_raw_dir(face, x, y, S));
   const int a = lane % kIrrThetaLanes, b = lane / kIrrThetaLanes;
   double ar = 0.0, ag = 0.0, ab = 0.0;
@@ -1179,10 +1180,9 @@ __global__ __launch_bounds__(64 * kFoldWaves) void irradiance_fold_kernel(const 
   const int S = p.size, half = (S + 1) / 2;
   // The orbit's representative with no negative component, on the lattice of
   // half-texels (cube_texel_raw_dir): the major component is S.
-  const int axis = blockIdx.x / (half * half);
-  const int rem = blockIdx.x - axis * half * half;
+  const int axis = blockIdx.y / half;
   const int even = 1 - (S & 1);
-  const int cu = 2 * (rem / half) + even, cv = 2 * (rem % half) + even;
+  const int cu = 2 * (static_cast<int>(blockIdx.y) - axis * half) + even, cv = 2 * static_cast<int>(blockIdx.x) + even;
   const int nx = axis == 0 ? S : cu, ny = axis == 1 ? S : (axis == 0 ? cu : cv), nz = axis == 2 ? S : cv;
   const Frame fr = local_to_world(mk(static_cast<float>(nx), static_cast<float>(ny), static_cast<float>(nz)));
   const uint32_t flip = static_cast<uint32_t>(lane & 7);
@@ -1298,7 +1298,7 @@ static althea_status launch_irradiance_fold(const float* pyr, const PyramidGeome
   p.theta_steps = (theta_samples + 7) / 8;
   p.polar_steps = (phi + 7) / 8;
   p.scale = M_PI / theta_samples / phi;
-  const int half = (size + 1) / 2;
+  const IrradianceGrid blocks = fold_blocks(size);
   const bool f64 = !(flags & ALTHEA_PRECOMPUTE_FP32_SUMS);
   const size_t tables = sizeof(float4) * static_cast<size_t>(phi) + sizeof(float2) * static_cast<size_t>(theta_samples);
   const bool lds = tables <= kFoldTableMax;
@@ -1311,7 +1311,7 @@ static althea_status launch_irradiance_fold(const float* pyr, const PyramidGeome
                 : variant == 5 ? irradiance_fold_kernel<true, false, true>
                 : variant == 6 ? irradiance_fold_kernel<false, true, true>
                                : irradiance_fold_kernel<true, true, true>;
-  hipLaunchKernelGGL(kernel, dim3(3 * half * half), dim3(64 * kFoldWaves), lds ? tables : 0, s,
+  hipLaunchKernelGGL(kernel, dim3(blocks.x, blocks.y), dim3(64 * kFoldWaves), lds ? tables : 0, s,
                      reinterpret_cast<const char*>(grid), theta_tab, phi_tab, p, reinterpret_cast<float4*>(cube));
   return check_launch("irradiance_fold_kernel");
 }
@@ -1377,22 +1377,23 @@ althea_status launch_irradiance(const float* pyr, int env_w, int env_h, int size
     p.lv1 = split_level(env_w, env_h, gg, p.l1);
   }
   p.scale = M_PI / theta_samples / phi;
-  const dim3 grid((6 * size * size + 3) / 4);
+  const IrradianceGrid blocks = texel_blocks(size, kIrrWaves);
+  const dim3 grid(blocks.x, blocks.y), block(64 * kIrrWaves);
   const char* g4 = reinterpret_cast<const char*>(gather);
   float4* cube4 = reinterpret_cast<float4*>(cube);
   const bool f64 = !(flags & ALTHEA_PRECOMPUTE_FP32_SUMS);
   if (theta_samples <= kIrrThetaLdsMax) {
     const size_t lds = sizeof(float2) * static_cast<size_t>(theta_samples);
     if (f64)
-      hipLaunchKernelGGL((irradiance_cube_kernel<true, true>), grid, dim3(256), lds, s, g4, theta_tab, phi_tab, p,
+      hipLaunchKernelGGL((irradiance_cube_kernel<true, true>), grid, block, lds, s, g4, theta_tab, phi_tab, p,
                          cube4);
     else
-      hipLaunchKernelGGL((irradiance_cube_kernel<false, true>), grid, dim3(256), lds, s, g4, theta_tab, phi_tab, p,
+      hipLaunchKernelGGL((irradiance_cube_kernel<false, true>), grid, block, lds, s, g4, theta_tab, phi_tab, p,
                          cube4);
   } else if (f64) {
-    hipLaunchKernelGGL((irradiance_cube_kernel<true, false>), grid, dim3(256), 0, s, g4, theta_tab, phi_tab, p, cube4);
+    hipLaunchKernelGGL((irradiance_cube_kernel<true, false>), grid, block, 0, s, g4, theta_tab, phi_tab, p, cube4);
   } else {
-    hipLaunchKernelGGL((irradiance_cube_kernel<false, false>), grid, dim3(256), 0, s, g4, theta_tab, phi_tab, p,
+    hipLaunchKernelGGL((irradiance_cube_kernel<false, false>), grid, block, 0, s, g4, theta_tab, phi_tab, p,
                        cube4);
   }
   return check_launch("irradiance_cube_kernel");

@@ -7,6 +7,10 @@
 using namespace althea;
 
 extern "C" {
+void grids(int size, int waves, unsigned* out) {
+  const IrradianceGrid f = fold_blocks(size), t = texel_blocks(size, waves);
+  out[0] = f.x, out[1] = f.y, out[2] = t.x, out[3] = t.y;
+}
 // Steps that a wave starting at step `wave` takes, `stride` apart, and the last of them.
 long long fold_walk(int wave, int stride, int theta_steps, int polar_steps, int* last) {
   long long n = 0;

@@ -452,6 +452,26 @@ def test_irradiance_folded_matches_oracle(torch, w, h, size, theta, fp32):
         assert err.max() < (1e-3 if fp32 else MAX_REL), (t, summary(err))
 
 
+@pytest.mark.parametrize("size,theta", [(2365, 8), (4096, 8), (3345, 9), (4096, 9)])
+def test_irradiance_of_the_largest_cubes(torch, size, theta):
+    """Cubes whose blocks in one row would pass 2^32 threads: of 2 365 and more
+    folded, of 3 345 and more by texel, up to the largest the call takes.  The
+    corners and some texels of every face against the oracle, and no texel left
+    out."""
+    env = aa.synth.env(seed=SEED0 + size, width=8, height=4, sigma=0.5, suns=1, peak_min=10.0, peak_max=20.0,
+                       sun_sigma_deg=30.0)
+    got = aa.irradiance_cube(aa.env_pyramid(torch.from_numpy(env).cuda()), 8, 4, size, theta).view(6, size, size, 4)
+    assert (got[..., 3] == 1.0).all()
+    rng = np.random.default_rng(size)
+    at = np.concatenate([[(0, 0), (0, size - 1), (size - 1, 0), (size - 1, size - 1), (size // 2, size // 2)],
+                         rng.integers(0, size, (20, 2))])
+    ids = np.array([(f, x, y) for f in range(6) for x, y in at], np.int32)
+    k = torch.from_numpy(ids.astype(np.int64)).cuda()
+    err = rel_err(got[k[:, 0], k[:, 2], k[:, 1], :3].cpu().numpy(), ol.Env(env).irradiance_texels(size, ids, theta),
+                  RADIANCE_FLOOR)
+    assert err.max() < MAX_REL, summary(err)
+
+
 # ------------------------------------------------------------- IBL handle
 def test_ibl_handle_matches_low_level_calls(torch):
     env = _env("config0")

@@ -20,7 +20,20 @@ def lib(tmp_path_factory):
     L = C.CDLL(str(so))
     L.fold_walk.restype = C.c_longlong
     L.fold_walk.argtypes = [C.c_int, C.c_int, C.c_int, C.c_int, C.c_void_p]
+    L.grids.argtypes = [C.c_int, C.c_int, C.c_void_p]
     return L
+
+
+@pytest.mark.parametrize("size", [1, 2, 3, 2364, 2365, 3344, 3345, 4095, 4096])
+def test_grids_stay_within_the_launch_limits(lib, size):
+    """Every size the entry points accept: less than 2^32 threads along x and
+    2^16 blocks along y, a block of 1 024 threads for each orbit of three axes,
+    a wave of 64 (four a block) for each texel of six faces."""
+    g = (C.c_uint * 4)()
+    lib.grids(size, 4, g)
+    half = (size + 1) // 2
+    assert (g[0], g[1]) == (half, 3 * half) and g[0] * 1024 < 1 << 32 and g[1] < 1 << 16
+    assert g[3] == 6 and 4 * g[2] >= size * size > 4 * (g[2] - 1) and g[2] * 256 < 1 << 32
 
 
 # (azimuths, polar samples): the smallest, ragged ones, the reference's 300 x
