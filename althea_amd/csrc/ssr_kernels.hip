@@ -66,6 +66,7 @@ struct SsrParams {
   float view_z[4];                  // row 2 of the view matrix
   float eye[3];
   float sign_slack;                 // kSignSlack * (bound of the view rays' length)
+  float m_min;                      // 2^-60 of that length: the sign test's least |m|
   float inv_far;                    // depth-plane value of an uncovered pixel
   float* depth;                     // depth plane in 8 x 4 texel blocks (taddr)
   int depth_tw;                     // blocks per block row, ceil(W / 8)
@@ -268,10 +269,13 @@ __global__ __launch_bounds__(256) void ssr_capture_kernel(const SsrParams p, con
     // The point lies at -ray / m from the eye; (-ray / m + EP) . perp has the
     // sign of m (EP . perp m - ray . perp), both products affine in k.  Where
     // that is clear of rounding and the last step's sign (prev, +-1), there is
-    // no crossing (SSR.frag:109) and the point is not formed: most steps.
+    // no crossing (SSR.frag:109) and the point is not formed: most steps.  An m
+    // near 0 (uncovered pixels under an infinite far plane) has no sign to go
+    // by: the point and its projection leave FP32's range, and no crossing is
+    // seen here or at the next step.
     const float e = fmaf(ep, m, -fmaf(k, rpk, rp0));
     const float es = m < 0.0f ? -e : e;
-    if (es * prev > fmaf(ep_slack, fabsf(m), p.sign_slack)) continue;
+    if (es * prev > fmaf(ep_slack, fabsf(m), p.sign_slack) && fabsf(m) > p.m_min) continue;
     const f3 ray = mk(fmaf(k, rk.x, ray0.x), fmaf(k, rk.y, ray0.y), fmaf(k, rk.z, ray0.z));
     const float t = -rcp_fast(m);
     const f3 dq = mk(fmaf(ray.x, t, EP.x), fmaf(ray.y, t, EP.y), fmaf(ray.z, t, EP.z));
@@ -425,6 +429,7 @@ althea_status launch_ssr_capture(const althea_gbuffer_view* g, const althea_ibl_
     rmax += r * r;
   }
   p.sign_slack = kSignSlack * std::sqrt(rmax);
+  p.m_min = std::ldexp(std::sqrt(rmax), -60);
   refl_chain(*reflection, p.out);
   const int n = g->width * g->height;
   const dim3 dgrid((n + 255) / 256);

@@ -146,6 +146,49 @@ def test_ssr_capture_block_edges_match_oracle(torch, ibl, W, H):
             assert r["err"]["max"] < 2e-3, r
 
 
+def _far_plane(scene, far):
+    """The scene under the projection of another far plane (near as it was)."""
+    P, near = np.zeros((4, 4)), 0.01
+    P[:] = scene.mat(0).reshape(4, 4).T
+    P[2, 2], P[2, 3] = (-1.0, -near) if far is None else (far / (near - far), -far * near / (far - near))
+    inv = np.zeros((4, 4))
+    inv[0, 0], inv[1, 1], inv[2, 3] = 1.0 / P[0, 0], 1.0 / P[1, 1], -1.0
+    inv[3, 2], inv[3, 3] = 1.0 / P[2, 3], P[2, 2] / P[2, 3]
+    for k, m in ((0, P), (1, inv)):
+        scene.mat(k)[:] = m.T.ravel().astype(np.float32)
+
+
+@pytest.mark.parametrize("far", [1000.0, None])
+def test_ssr_capture_marches_over_uncovered_pixels(torch, ibl, far):
+    """A floor, a near strip that the reflected rays pass behind, sky, and a far
+    strip that most of them pass over.  Under an infinite far plane (1 / far = 0)
+    an uncovered pixel has no point and no side of the ray: the strips on its
+    two sides, in front of the ray and behind it, are no crossing.  The oracle's
+    margins are 0 beside such a step, so every decision is compared, but for 1 in
+    2 000 (a sky step read as one side of the ray is 48 hits too many)."""
+    ibl_res, _ = ibl
+    scene, use_f, use_w, d = wall_scene(W=64, H=1440)
+    eye = scene.mat(4)[12:15].astype(np.float64)
+    with np.errstate(divide="ignore", invalid="ignore"):
+        near = eye + ((-2.0 - eye[2]) / d[..., 2])[..., None] * d
+    strip = (d[..., 2] < 0) & (near[..., 1] > 1.1) & (near[..., 1] < 1.3)
+    sky = (use_w & ~((scene.position[..., 1] > 1.2) & (scene.position[..., 1] < 1.6))) | \
+          (use_f & (scene.position[..., 2] < -6.0))
+    for plane in (scene.position, scene.normal, scene.albedo, scene.material):
+        plane[sky] = 0.0
+    scene.position[strip] = np.concatenate([near[strip], np.ones((int(strip.sum()), 1))], 1)
+    scene.normal[strip] = (0.0, 0.0, 1.0, 0.0)
+    scene.albedo[strip], scene.material[strip] = (0.8, 0.6, 0.4, 1.0), (0.0, 0.3, 1.0, 0.0)
+    _far_plane(scene, far)
+    got = _capture(torch, scene, ibl_res).level(0).cpu().numpy().reshape(-1, 4)
+    _, _, step, _, _ = ol.ssr(scene, ibl_res.views_numpy(), _all_pixels(scene))
+    floor = (use_f & ~sky & ~strip).ravel()
+    hit, ref = got[floor, 3] == 1.0, step[floor] >= 0
+    print("SSR over sky", far, int(floor.sum()), int(ref.sum()), int(hit.sum()), int((hit != ref).sum()))
+    assert floor.sum() > 10000 and ref.sum() > 1000
+    assert (hit != ref).sum() <= floor.sum() // 2000, (int(hit.sum()), int(ref.sum()), int((hit != ref).sum()))
+
+
 def test_ssr_capture_wall_scene_matches_oracle(torch, ibl):
     ibl_res, _ = ibl
     scene, use_f, _, _ = wall_scene(W=320, H=180)
