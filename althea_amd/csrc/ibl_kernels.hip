@@ -1044,11 +1044,14 @@ __global__ __launch_bounds__(256) void blend_grid_kernel(const float4* __restric
 // 0 is the node at x' = 1, just across the fold.  Two more columns hold the
 // precompute's pole branch (|xz| <= 0.001 reads yaw 0 whatever the signs of
 // x and z): the nodes beside yaw 0 in every slot, without the x and z flips.
+// The row after the last, all zeros, is what the lanes past the last azimuth
+// or polar row read (an infinite texel times their weight 0 would be NaN).
 struct FoldGrid {
   bool ok;
   int w0, h0, blend;
   int cols, rows;  // columns without the two pole columns
-  size_t nodes;    // stored nodes, pole columns included
+  size_t cells;    // nodes of the grid, pole columns included
+  size_t nodes;    // stored nodes: the grid and, after it, a row and two nodes of zeros
 };
 constexpr int kFoldNodeBytes = 96;
 constexpr size_t kFoldMaxBytes = size_t{1} << 30;
@@ -1064,7 +1067,8 @@ static FoldGrid fold_grid(int w, int h, int theta, const IrradianceLod& lod) {
   if (f.w0 % 8 != 0 || f.h0 % 4 != 0) return f;
   f.cols = (f.blend ? 3 * f.w0 / 8 : f.w0 / 4) + 2;
   f.rows = (f.blend ? 3 * f.h0 / 4 : f.h0 / 2) + 2;
-  f.nodes = static_cast<size_t>(f.cols + 2) * f.rows;
+  f.cells = static_cast<size_t>(f.cols + 2) * f.rows;
+  f.nodes = f.cells + (f.cols + 2) + 2;
   f.ok = kFoldNodeBytes * f.nodes <= kFoldMaxBytes;
   return f;
 }
@@ -1093,7 +1097,12 @@ __global__ __launch_bounds__(256) void fold_grid_kernel(const float4* __restrict
                                                         float* __restrict__ out) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
   const uint32_t cols = static_cast<uint32_t>(p.cols) + 2u;
-  if (i >= 8u * cols * static_cast<uint32_t>(p.rows)) return;
+  const uint32_t cells = cols * static_cast<uint32_t>(p.rows);
+  if (i >= 8u * (cells + cols + 2u)) return;
+  if (i >= 8u * cells) {
+    for (int k = 0; k < 3; ++k) out[3 * static_cast<size_t>(i) + k] = 0.0f;
+    return;
+  }
   const int slot = static_cast<int>(i & 7u);
   const int r = static_cast<int>((i >> 3) / cols), c = static_cast<int>((i >> 3) - static_cast<uint32_t>(r) * cols);
   const int W = p.src.w0, H = p.src.h0;
@@ -1120,6 +1129,7 @@ struct FoldParams {
   float kx, ky;  // x' = yaw kx + 3/2, y' = pitch ky + 3/2
   int cols;
   uint32_t rowbytes;  // kFoldNodeBytes (cols + 2)
+  uint32_t zeros;     // byte offset of the row of zeros
   int size;
   int theta_samples, phi_samples;
   int theta_steps, polar_steps;  // groups of 8 azimuths and of 8 polar rows
@@ -1209,7 +1219,7 @@ __global__ __launch_bounds__(64 * kFoldWaves) void irradiance_fold_kernel(const 
     const uint32_t signs = (__float_as_uint(d.x) >> 31) | (__float_as_uint(d.z) >> 31 << 1) |
                            (__float_as_uint(d.y) >> 31 << 2);
     const uint32_t off = static_cast<uint32_t>(row) * p.rowbytes + static_cast<uint32_t>(col * kFoldNodeBytes);
-    rec[lane] = make_float4(__uint_as_float(off | signs), fx, fy, valid ? ph.z : 0.0f);
+    rec[lane] = make_float4(__uint_as_float(valid ? off | signs : p.zeros), fx, fy, valid ? ph.z : 0.0f);
     wave_lds_sync();
 #pragma unroll 4
     for (int k = 0; k < 8; ++k) {
@@ -1292,6 +1302,7 @@ static althea_status launch_irradiance_fold(const float* pyr, const PyramidGeome
   p.ky = -c0.ky;
   p.cols = fg.cols;
   p.rowbytes = static_cast<uint32_t>(kFoldNodeBytes * (fg.cols + 2));
+  p.zeros = static_cast<uint32_t>(kFoldNodeBytes * fg.cells);
   p.size = size;
   p.theta_samples = theta_samples;
   p.phi_samples = phi;

@@ -452,6 +452,27 @@ def test_irradiance_folded_matches_oracle(torch, w, h, size, theta, fp32):
         assert err.max() < (1e-3 if fp32 else MAX_REL), (t, summary(err))
 
 
+@pytest.mark.parametrize("size,theta", [(1, 100), (1, 101), (2, 66), (3, 100), (3, 70)])
+def test_irradiance_of_an_infinite_texel(torch, size, theta):
+    """A source with one infinite texel, read at level 0 with azimuth and polar
+    counts that are no multiples of 8: a texel whose samples reach it is infinite,
+    every other one finite, and none is NaN (samples past the counts add
+    nothing)."""
+    w, h = 64, 32
+    env = aa.synth.env(seed=SEED0 + 3, width=w, height=h, sigma=0.2, suns=0)
+    x = int((0.5 + 90.0 / 360.0) * w)  # yaw 90 degrees, pitch 45: on the horizons of +X and of -X
+    y = int((0.5 - 45.0 / 180.0) * h)
+    ids = np.array([(f, i, j) for f in range(6) for j in range(size) for i in range(size)], np.int32)
+    bright = env.copy()
+    bright[y, x, :3] = 1e30
+    reached = ol.Env(bright).irradiance_texels(size, ids, theta) > 1e20
+    env[y, x, :3] = np.inf
+    got = aa.irradiance_cube(aa.env_pyramid(torch.from_numpy(env).cuda()), w, h, size, theta).cpu().numpy()[:, :3]
+    assert reached.any() and not reached.all()
+    assert not np.isnan(got).any(), np.argwhere(np.isnan(got))
+    np.testing.assert_array_equal(np.isinf(got), reached)
+
+
 @pytest.mark.parametrize("size,theta", [(2365, 8), (4096, 8), (3345, 9), (4096, 9)])
 def test_irradiance_of_the_largest_cubes(torch, size, theta):
     """Cubes whose blocks in one row would pass 2^32 threads: of 2 365 and more
