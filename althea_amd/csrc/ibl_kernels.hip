@@ -21,6 +21,7 @@
 #include "device_math.hpp"
 #include "internal.hpp"
 #include "irradiance_launch.hpp"
+#include "point_launch.hpp"
 #include "precise_lookup.hpp"
 #include "prefilter_common.hpp"
 
@@ -676,7 +677,7 @@ __global__ __launch_bounds__(64 * kPointWaves) void prefilter_points_kernel(cons
   char* lds = reinterpret_cast<char*>(s_levels);
   PointLevel* levels = reinterpret_cast<PointLevel*>(lds + p.level_off);
   float* table = reinterpret_cast<float*>(lds + p.table_off);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   stage_levels<kPointWaves>(p.pyr, p.lv, p.slv, p.first, p.levels, lds);
   if (static_cast<int>(threadIdx.x) < p.levels) {
     const LevelC& c = p.lv[threadIdx.x];
@@ -693,9 +694,9 @@ __global__ __launch_bounds__(64 * kPointWaves) void prefilter_points_kernel(cons
   __syncthreads();
   const float max_lod = static_cast<float>(p.levels - 1);
   const float half_sa = -0.5f * p.log2_sa_texel;
-  for (int query = static_cast<int>(blockIdx.x) * kPointWaves + wave; query < p.count;
-       query += static_cast<int>(gridDim.x) * kPointWaves) {
-    const float4 q = dir_rough[__builtin_amdgcn_readfirstlane(query)];
+  const PointWalk walk = point_walk(blockIdx.x, gridDim.x, wave, kPointWaves);
+  for (size_t query = walk.first; query < static_cast<size_t>(p.count); query += walk.stride) {
+    const float4 q = dir_rough[query];
     const Frame fr = local_to_world(mk(q.x, q.y, q.z));
     const float rough = fabsf(q.w), a2 = rough * rough, a2m1 = a2 - 1.0f, a2p1 = a2 + 1.0f;
     const float kd = static_cast<float>(p.samples) * kInvPi / a2;  // n D = kd den^2
@@ -752,7 +753,7 @@ __global__ __launch_bounds__(64 * kPointWaves) void prefilter_points_kernel(cons
     for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     const double w = __shfl(v, 48, 64);
     if ((lane & 15) == 0)
-      out[4 * static_cast<size_t>(query) + (lane >> 4)] = lane == 48 ? 1.0f : static_cast<float>(v / w);
+      out[4 * query + (lane >> 4)] = lane == 48 ? 1.0f : static_cast<float>(v / w);
   }
 }
 
@@ -777,7 +778,7 @@ althea_status launch_prefilter_points(const float* pyr, int env_w, int env_h, in
   int dev = 0, cus = 256;
   ALTHEA_TRY_HIP(hipGetDevice(&dev));
   ALTHEA_TRY_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  const int blocks = std::min((count + kPointWaves - 1) / kPointWaves, 3 * cus);
+  const int blocks = point_blocks(count, kPointWaves, 3 * cus);
   auto kernel = table ? prefilter_points_kernel<true> : prefilter_points_kernel<false>;
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kPointWaves), lds, s, p,
                      reinterpret_cast<const float4*>(dir_rough), out);
