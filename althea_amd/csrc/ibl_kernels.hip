@@ -596,11 +596,12 @@ althea_status launch_prefilter_cube(const float* pyr, int env_w, int env_h, int 
 }
 
 // -------------------------------------------------------- point prefilter
-// Same estimator at a query's (direction, roughness r).  A wave takes a query,
-// its lanes the samples; lane l takes samples l C + t, t = 0..C - 1 (C = n / 64
-// rounded up), so with C a power of two the lanes of a step have radical
-// inverses within 1 / C: nearly one source LOD, spread around a ring of the
-// lobe, and the steps outside the hemisphere are skipped whole.
+// Same estimator at a query's (direction, roughness r).  kLanes lanes of a wave
+// take a query, each its samples: lane l takes samples l C + t, t = 0..C - 1
+// (C = n / kLanes rounded up), so with C a power of two the lanes of a step have
+// radical inverses within 1 / C: nearly one source LOD, spread around a ring of
+// the lobe, and with the whole wave on a query the steps outside the hemisphere
+// are skipped whole.  point_lanes says which kLanes a call takes.
 //
 // With x2 the radical inverse and den = 1 + (r^2 - 1) x2, the GGX half vector
 // has cos^2 = (1 - x2) / den and sin^2 = r^2 x2 / den, so L in the frame is
@@ -621,7 +622,7 @@ struct PointParams {
   StagedLevel slv[kMaxLevels];
   const char* pyr;
   int first, levels;
-  int samples, steps;  // steps = ceil(samples / 64)
+  int samples, steps;  // steps = ceil(samples / kLanes)
   int count;
   int level_off, table_off;  // byte offsets in LDS of the level records and the sample table
   float log2_sa_texel;
@@ -667,12 +668,14 @@ __device__ __forceinline__ void point_lookup(const char* __restrict__ pyr, const
 }
 
 constexpr int kPointWaves = 8;
+constexpr int kPointBlocks = 768;  // three a CU walk the queries: the staging and the table are per block
 constexpr int kPointTableMax = 2048;  // samples whose table stays in LDS (24 KB)
 
-template <bool kTable>
+template <int kLanes, bool kTable>
 __global__ __launch_bounds__(64 * kPointWaves) void prefilter_points_kernel(const PointParams p,
                                                                             const float4* __restrict__ dir_rough,
                                                                             float* __restrict__ out) {
+  constexpr int kQueries = 64 / kLanes;
   extern __shared__ float s_levels[];
   char* lds = reinterpret_cast<char*>(s_levels);
   PointLevel* levels = reinterpret_cast<PointLevel*>(lds + p.level_off);
@@ -686,17 +689,20 @@ __global__ __launch_bounds__(64 * kPointWaves) void prefilter_points_kernel(cons
   }
   if (kTable) {
     // Step t's lanes side by side.
-    for (int i = threadIdx.x; i < 64 * p.steps; i += 64 * kPointWaves) {
-      const f3 v = point_sample((i & 63) * p.steps + (i >> 6), p.samples);
+    for (int i = threadIdx.x; i < kLanes * p.steps; i += 64 * kPointWaves) {
+      const f3 v = point_sample(i % kLanes * p.steps + i / kLanes, p.samples);
       table[3 * i] = v.x, table[3 * i + 1] = v.y, table[3 * i + 2] = v.z;
     }
   }
   __syncthreads();
   const float max_lod = static_cast<float>(p.levels - 1);
   const float half_sa = -0.5f * p.log2_sa_texel;
-  const PointWalk walk = point_walk(blockIdx.x, gridDim.x, wave, kPointWaves);
-  for (size_t query = walk.first; query < static_cast<size_t>(p.count); query += walk.stride) {
-    const float4 q = dir_rough[query];
+  const int sub = lane % kLanes;
+  const size_t count = static_cast<size_t>(p.count);
+  const PointWalk walk = point_walk(blockIdx.x, gridDim.x, wave, kPointWaves, kQueries);
+  for (size_t base = walk.first; base < count; base += walk.stride) {
+    const size_t query = base + lane / kLanes;  // lanes past the count repeat the last query
+    const float4 q = dir_rough[query < count ? query : count - 1];
     const Frame fr = local_to_world(mk(q.x, q.y, q.z));
     const float rough = fabsf(q.w), a2 = rough * rough, a2m1 = a2 - 1.0f, a2p1 = a2 + 1.0f;
     const float kd = static_cast<float>(p.samples) * kInvPi / a2;  // n D = kd den^2
@@ -705,10 +711,10 @@ __global__ __launch_bounds__(64 * kPointWaves) void prefilter_points_kernel(cons
     for (int t = 0; t < p.steps; ++t) {
       f3 e;
       if (kTable) {
-        const float* v = table + 3 * (64 * t + lane);
+        const float* v = table + 3 * (kLanes * t + sub);
         e = mk(v[0], v[1], v[2]);
       } else {
-        e = point_sample(lane * p.steps + t, p.samples);
+        e = point_sample(sub * p.steps + t, p.samples);
       }
       const float num = fmaf(-e.z, a2p1, 1.0f);
       if (num > 0.0f) {
@@ -741,19 +747,27 @@ __global__ __launch_bounds__(64 * kPointWaves) void prefilter_points_kernel(cons
       }
     }
     ar += s[0], ag += s[1], ab += s[2], aw += sw;
-    // Four sums over 64 lanes: halves exchange two sums, quarters one, then one
-    // value is summed over 16 lanes (lane 0: r, 16: g, 32: b, 48: w).
-    const bool hi = lane & 32, hi2 = lane & 16;
-    double k0 = hi ? ab : ar, k1 = hi ? aw : ag;
-    k0 += __shfl_xor(hi ? ar : ab, 32, 64);
-    k1 += __shfl_xor(hi ? ag : aw, 32, 64);
-    double v = hi2 ? k1 : k0;
-    v += __shfl_xor(hi2 ? k0 : k1, 16, 64);
+    if constexpr (kLanes == 1) {
+      if (query < count)
+        reinterpret_cast<float4*>(out)[query] = make_float4(static_cast<float>(ar / aw), static_cast<float>(ag / aw),
+                                                            static_cast<float>(ab / aw), 1.0f);
+    } else {
+      // Four sums over the query's lanes: halves exchange two sums, quarters
+      // one, then one value is summed over a quarter (first r, then g, b, w).
+      constexpr int kHalf = kLanes / 2, kQuarter = kLanes / 4;
+      const bool hi = lane & kHalf, hi2 = lane & kQuarter;
+      double k0 = hi ? ab : ar, k1 = hi ? aw : ag;
+      k0 += __shfl_xor(hi ? ar : ab, kHalf, 64);
+      k1 += __shfl_xor(hi ? ag : aw, kHalf, 64);
+      double v = hi2 ? k1 : k0;
+      v += __shfl_xor(hi2 ? k0 : k1, kQuarter, 64);
 #pragma unroll
-    for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    const double w = __shfl(v, 48, 64);
-    if ((lane & 15) == 0)
-      out[4 * query + (lane >> 4)] = lane == 48 ? 1.0f : static_cast<float>(v / w);
+      for (int o = kQuarter / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+      const double w = __shfl(v, lane | kHalf | kQuarter, 64);
+      const int component = sub / kQuarter;
+      if (sub % kQuarter == 0 && query < count)
+        out[4 * query + component] = component == 3 ? 1.0f : static_cast<float>(v / w);
+    }
   }
 }
 
@@ -762,26 +776,27 @@ althea_status launch_prefilter_points(const float* pyr, int env_w, int env_h, in
   if (count == 0) return ALTHEA_OK;
   PointParams p{};
   pyramid_levels(env_w, env_h, p.lv);
+  const bool table = samples <= kPointTableMax;
+  const int lanes = point_lanes(samples, count);
   size_t staged = 0;
-  p.first = staged_levels(env_w, env_h, 0, p.slv, &staged);
   p.levels = althea_env_levels(env_w, env_h);
+  p.first = p.levels;
+  if (point_stages(samples, lanes)) p.first = staged_levels(env_w, env_h, 0, p.slv, &staged);
   p.pyr = reinterpret_cast<const char*>(pyr);
   p.samples = samples;
-  p.steps = (samples + 63) / 64;
+  p.steps = (samples + lanes - 1) / lanes;
   p.count = count;
   p.level_off = static_cast<int>((staged + 15) & ~size_t{15});
   p.table_off = p.level_off + static_cast<int>(sizeof(PointLevel)) * kMaxLevels;
   p.log2_sa_texel = static_cast<float>(std::log2(4.0 * M_PI / (6.0 * static_cast<double>(env_w) * env_h)));
-  const bool table = samples <= kPointTableMax;
-  const size_t lds = p.table_off + (table ? sizeof(float) * 3 * 64 * p.steps : size_t{0});
-  // Three blocks a CU walk the queries; the staging and the table are per block.
-  int dev = 0, cus = 256;
-  ALTHEA_TRY_HIP(hipGetDevice(&dev));
-  ALTHEA_TRY_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  const int blocks = point_blocks(count, kPointWaves, 3 * cus);
-  auto kernel = table ? prefilter_points_kernel<true> : prefilter_points_kernel<false>;
-  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kPointWaves), lds, s, p,
-                     reinterpret_cast<const float4*>(dir_rough), out);
+  const size_t lds = p.table_off + (table ? sizeof(float) * 3 * lanes * p.steps : size_t{0});
+  auto kernel = !table        ? prefilter_points_kernel<64, false>
+                : lanes == 1  ? prefilter_points_kernel<1, true>
+                : lanes == 4  ? prefilter_points_kernel<4, true>
+                : lanes == 16 ? prefilter_points_kernel<16, true>
+                              : prefilter_points_kernel<64, true>;
+  hipLaunchKernelGGL(kernel, dim3(point_blocks(count, kPointWaves, 64 / lanes, kPointBlocks)), dim3(64 * kPointWaves), lds, s,
+                     p, reinterpret_cast<const float4*>(dir_rough), out);
   return check_launch("prefilter_points_kernel");
 }
 

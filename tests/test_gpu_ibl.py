@@ -328,6 +328,36 @@ def test_prefilter_points_shapes(torch, w, h, count, samples):
     assert err.max() < MAX_REL and (got[:, 3] == 1.0).all(), summary(err)
 
 
+@pytest.mark.parametrize("count,samples", [(40961, 1), (70003, 2), (98305, 3), (131077, 4), (163847, 5),  # a lane
+                                           (8193, 1), (10007, 4), (40963, 17), (131075, 64),  # 4 lanes
+                                           (2049, 16), (8195, 63), (10243, 65), (32771, 255), (32769, 256)])  # 16
+def test_prefilter_points_of_few_samples(torch, count, samples):
+    """Several queries a wave, the last wave's ragged: the oracle's values, the
+    values of the same queries a few at a time (a wave a query), and nothing
+    written past the last query."""
+    w, h = 512, 256
+    env = aa.synth.env(seed=SEED0 + samples, width=w, height=h, sigma=0.2, suns=1, peak_min=5.0, peak_max=5.0,
+                       sun_sigma_deg=30.0)
+    q = aa.synth.dir_rough(seed=count, n=count, rmin=0.0, rmax=1.0)
+    q[0, 3] = 0.0
+    q[-1, 3] = 1.0
+    pyr, dev = aa.env_pyramid(torch.from_numpy(env).cuda()), torch.from_numpy(q).cuda()
+    out = torch.full((count + 64, 4), -7.0, device="cuda")
+    from althea_amd import _lib
+
+    _lib.check(_lib.lib().althea_prefilter_points(pyr.data_ptr(), w, h, samples, dev.data_ptr(), count,
+                                                  out.data_ptr(), torch.cuda.current_stream().cuda_stream), "points")
+    assert (out[count:] == -7.0).all()
+    got = out[:count].cpu().numpy()
+    rows = np.r_[0:300, count - 300:count]
+    err = rel_err(got[rows, :3], ol.Env(env).prefilter_points(samples, q[rows]), RADIANCE_FLOOR)
+    assert err.max() < MAX_REL and (got[:, 3] == 1.0).all(), summary(err)
+    wave = np.concatenate([aa.prefilter_points(pyr, w, h, samples, dev[k:k + 1000].contiguous()).cpu().numpy()
+                           for k in range(0, count, 1000)])
+    err = rel_err(got[:, :3], wave[:, :3], RADIANCE_FLOOR)
+    assert err.max() < MAX_REL, summary(err)
+
+
 def test_prefilter_points_agree_with_cube_texels(torch):
     # The point kernel at a cube texel's direction and roughness m/(mips-1)
     # estimates the same quantity as the cube kernel (same samples).
