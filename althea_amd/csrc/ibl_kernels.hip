@@ -806,8 +806,8 @@ althea_status launch_prefilter_points(const float* pyr, int env_w, int env_h, in
 // read at the fixed source LOD log2(W / theta_samples), times
 // pi / (theta_samples phi_samples).  An even azimuth count over a source
 // whose level is at least 8 x 4 takes the folded kernel below; the kernel
-// here, one wave per texel, serves odd azimuth counts, smaller levels, and
-// two levels that are not an exact halving.
+// here, one wave per texel, serves odd azimuth counts, smaller levels, few
+// samples (kFoldMinSteps), and two levels that are not an exact halving.
 struct IrradianceParams {
   SplitLevel lv0, lv1;  // the two source levels around LOD log2(W / theta_samples), split gather copies
   SplitLevel grid;      // their blend grid (blend)
@@ -1072,9 +1072,18 @@ struct FoldGrid {
 constexpr int kFoldNodeBytes = 96;
 constexpr size_t kFoldMaxBytes = size_t{1} << 30;
 
+// Steps of an orbit from which the folded kernel takes a call.  Its block of 16
+// waves stands idle for the rest of them, and orders its waves and adds their sums
+// whatever the steps: 128^2 x 6 texels of a 512 x 256 source take 53 us by texel
+// and 126 folded at 1 step (8 azimuths), 118 and 180 at 6 (24), 152 and 197 at 8
+// (30), 286 and 280 at 15 (40), 360 and 309 at 18 (48).
+constexpr int kFoldMinSteps = 14;
+
 static FoldGrid fold_grid(int w, int h, int theta, const IrradianceLod& lod) {
   FoldGrid f{};
   if (w <= 0 || h <= 0 || theta % 2 != 0) return f;
+  const long long polar = (irradiance_phi_samples(w, h, theta) + 7) / 8, azimuth = (theta + 7) / 8;
+  if (polar * azimuth < kFoldMinSteps) return f;
   const PyramidGeometry g = pyramid_geometry(w, h);
   f.blend = lod.delta != 0.0f ? 1 : 0;
   if (f.blend && !blend_grid(w, h, lod).ok) return f;

@@ -462,10 +462,13 @@ def test_irradiance_edge_shapes(torch, size, theta):
 @pytest.mark.parametrize("w,h,size,theta,fp32", [(8, 4, 2, 2, False), (8, 4, 3, 8, False), (16, 8, 1, 6, True),
                                                   (64, 32, 9, 30, False), (64, 32, 4, 64, True),
                                                   (128, 512, 7, 20, False), (2048, 4, 4, 1500, False),
-                                                  (256, 128, 1, 2048, False), (256, 128, 1, 2050, False)])
+                                                  (256, 128, 1, 2048, False), (256, 128, 1, 2050, False),
+                                                  (8, 4, 3, 40, False), (8, 4, 2, 66, True), (16, 8, 1, 34, False),
+                                                  (64, 32, 5, 30, False), (64, 32, 5, 34, False), (8, 64, 3, 8, False)])
 def test_irradiance_folded_matches_oracle(torch, w, h, size, theta, fp32):
-    """The folded irradiance (even azimuth counts): the smallest level it
-    takes, one level and two, odd and single-texel faces (texels that several
+    """The folded irradiance (even azimuth counts of 14 steps or more) and, below
+    that, the general kernel: the smallest level it takes, both sides of the
+    least steps, one level and two, odd and single-texel faces (texels that several
     sign flips name), FP32 sums, azimuth and polar tables at both sides of
     the 32 KB that LDS holds; and odd counts beside it on the general kernel,
     every texel.  Tolerance: the contract (1e-3 for FP32 sums)."""
@@ -503,7 +506,7 @@ def test_irradiance_of_an_infinite_texel(torch, size, theta):
     np.testing.assert_array_equal(np.isinf(got), reached)
 
 
-@pytest.mark.parametrize("size,theta", [(2365, 8), (4096, 8), (3345, 9), (4096, 9)])
+@pytest.mark.parametrize("size,theta", [(2365, 64), (4096, 64), (3345, 9), (4096, 9)])
 def test_irradiance_of_the_largest_cubes(torch, size, theta):
     """Cubes whose blocks in one row would pass 2^32 threads: of 2 365 and more
     folded, of 3 345 and more by texel, up to the largest the call takes.  The
