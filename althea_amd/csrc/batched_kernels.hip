@@ -22,6 +22,7 @@
 #include <new>
 #include <vector>
 
+#include "batch_launch.hpp"
 #include "device_math.hpp"
 #include "internal.hpp"
 #include "prefilter_common.hpp"
@@ -194,7 +195,7 @@ althea_status launch_persistent(const althea_prefilter_batch* b, int shape, int 
   hipLaunchKernelGGL(batch_reset_kernel, dim3(1), dim3(64), 0, s, b->d_counter);
   althea_status st = check_launch("batch_reset_kernel");
   if (st != ALTHEA_OK) return st;
-  const int blocks = std::max(1, b->cus * waves_per_cu / kBatchWaves);
+  const int blocks = batch_blocks(b->cus, waves_per_cu, kBatchWaves);
   if (b->flags & ALTHEA_PRECOMPUTE_FP32_SUMS)
     launch_persistent_t<false>(b, shape, blocks, work, tiles, s);
   else

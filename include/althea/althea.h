@@ -184,7 +184,8 @@ typedef struct althea_env_view {
 } althea_env_view;
 
 /* Launch shape of the persistent prefilter: a wave shades a tile_w x tile_h
- * texel tile (8x8, 16x4 or 4x16); the grid holds waves_per_cu waves per CU. */
+ * texel tile (8x8, 16x4 or 4x16); the grid holds waves_per_cu waves per CU, in
+ * blocks of 8 (one block per CU at least). */
 typedef struct althea_tuning {
   int tile_w, tile_h;
   int waves_per_cu;

@@ -84,6 +84,21 @@ def test_batch_autotune_and_oracle_spot_check(torch):
     assert err.max() < MAX_REL, summary(err)
 
 
+def test_every_launch_shape_gives_the_same_bits(torch):
+    """Tiles and waves per CU change the schedule only: from one block of eight
+    waves a CU (settings of 4 to 8) to four."""
+    maps = _maps(torch, [256, 64, 128], seed0=400, sigma=0.0)
+    b = PrefilterBatch(maps, [64, 16, 32], mips=4, samples=128)
+    ref = None
+    for tw, th in ((8, 8), (16, 4), (4, 16)):
+        for waves in (4, 5, 7, 8, 12, 32):
+            b.set_tuning(tw, th, waves)
+            b.run()
+            got = [b.cube(i) for i in range(3)]
+            ref = ref or got
+            assert all(torch.equal(g, r) for g, r in zip(got, ref)), (tw, th, waves)
+
+
 def test_config3_full_batch_matches_single_map_kernel(torch):
     """The configured batch (config 3): 64 environment maps, widths drawn from
     {256 .. 4096} by batch_widths(64) (height W/2, the config-0 radiance
