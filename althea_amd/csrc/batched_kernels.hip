@@ -59,7 +59,10 @@ __global__ __launch_bounds__(64 * kBatchWaves) __attribute__((amdgpu_waves_per_e
       __syncthreads();
       staged = w.x;
     }
-    prefilter_block<kF64Sums, kTW, kTH, kBatchWaves, true, true>(p, w.y, w.z, lds);
+    if (p.alone)
+      prefilter_block<kF64Sums, kTW, kTH, kBatchWaves, true, true, true>(p, w.y, w.z, lds);
+    else
+      prefilter_block<kF64Sums, kTW, kTH, kBatchWaves, true, true, false>(p, w.y, w.z, lds);
     if (rough && p.split > 1) staged = -1;
   }
 }
@@ -109,6 +112,7 @@ struct althea_prefilter_batch {
   LevelC* d_levels = nullptr;
   StagedLevel* d_slevels = nullptr;
   std::vector<int> waves;  // per map: waves per tile of a rough mip
+  std::vector<char> alone;  // per map: texels by themselves, not in pairs
   size_t lds_bytes = 0;
   GgxEntry* d_tables = nullptr;
   int* d_counts = nullptr;
@@ -157,8 +161,9 @@ std::vector<int4> build_work(const althea_prefilter_batch* b, int tw, int th, si
       const int S = std::max(1, b->sizes[i] >> m);
       const bool mirror = m == 0 || b->mips == 1;
       const int active = std::min(S, tw) * std::min(S, th);
-      const double cost = mip_cost[m] * active * (mirror ? kBatchWaves : 2.0 * kBatchWaves / b->waves[i]);
-      const int blocks = prefilter_blocks(b->sizes[i], b->mips, m, b->waves[i], tw, th, kBatchWaves);
+      const double cost =
+          mip_cost[m] * active * (mirror ? kBatchWaves : (b->alone[i] ? 1.0 : 2.0) * kBatchWaves / b->waves[i]);
+      const int blocks = prefilter_blocks(b->sizes[i], b->mips, m, b->waves[i], b->alone[i], tw, th, kBatchWaves);
       for (int k = 0; k < blocks; ++k) items.push_back({cost, make_int4(i, m, k, 0)});
       tex += 6ull * S * S;
     }
@@ -289,6 +294,7 @@ static althea_status batch_create(const althea_env_view* envs, int count, const 
   b->pyramids.assign(count, nullptr);
   b->cubes.assign(count, nullptr);
   b->waves.assign(count, 1);
+  b->alone.assign(count, 0);
   b->owns_buffers = ext_pyramids == nullptr;
   for (int i = 0; i < count; ++i) {
     const auto ext = std::make_pair(envs[i].width, envs[i].height);
@@ -321,6 +327,7 @@ static althea_status batch_create(const althea_env_view* envs, int count, const 
     p.mips = mips;
     p.samples = samples;
     p.split = prefilter_split(face_sizes[i], mips, samples, p.chunk);
+    p.alone = b->alone[i] = prefilter_alone(w, h, face_sizes[i], mips, samples) ? 1 : 0;
     p.waves = b->waves[i] = std::min(p.split, kBatchWaves);
     if (mips > 1) b->lds_bytes = std::max(b->lds_bytes, prefilter_lds_bytes(staged, p.split, p.waves, kBatchWaves));
   }

@@ -296,7 +296,7 @@ constexpr int kPrefilterTile = 8;
 // waves a SIMD.
 constexpr int kPrefilterWide = 16, kPrefilterNarrow = 8;
 
-template <bool kF64Sums, int kWaves>
+template <bool kF64Sums, int kWaves, bool kTogether, bool kSingle>
 __device__ __forceinline__ void prefilter_cube(const PrefilterParams& p, float* s_levels) {
   const int b = blockIdx.x;
   int m = 0;
@@ -309,21 +309,28 @@ __device__ __forceinline__ void prefilter_cube(const PrefilterParams& p, float* 
     stage_levels<kWaves>(map.pyr, map.lv, map.slv, map.first, map.levels, lds);
     __syncthreads();
   }
-  prefilter_block<kF64Sums, kPrefilterTile, kPrefilterTile, kWaves, kWaves == kPrefilterWide, false>(
+  prefilter_block<kF64Sums, kPrefilterTile, kPrefilterTile, kWaves, kTogether, false, kSingle>(
       map, m, b - p.block_start[m], lds);
 }
 
 template <bool kF64Sums>
 __global__ __launch_bounds__(64 * kPrefilterWide) void prefilter_wide_kernel(const PrefilterParams p) {
   extern __shared__ float s_levels[];
-  prefilter_cube<kF64Sums, kPrefilterWide>(p, s_levels);
+  prefilter_cube<kF64Sums, kPrefilterWide, true, false>(p, s_levels);
 }
 
 template <bool kF64Sums>
 __global__ __launch_bounds__(64 * kPrefilterNarrow) __attribute__((amdgpu_waves_per_eu(6))) void prefilter_cube_kernel(
     const PrefilterParams p) {
   extern __shared__ float s_levels[];
-  prefilter_cube<kF64Sums, kPrefilterNarrow>(p, s_levels);
+  prefilter_cube<kF64Sums, kPrefilterNarrow, false, false>(p, s_levels);
+}
+
+template <bool kF64Sums, int kWaves>
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(4))) void prefilter_alone_kernel(
+    const PrefilterParams p) {
+  extern __shared__ float s_levels[];
+  prefilter_cube<kF64Sums, kWaves, false, true>(p, s_levels);
 }
 
 // Chunks of a rough mip's table: doubled while the pairs of tiles times the
@@ -332,13 +339,18 @@ __global__ __launch_bounds__(64 * kPrefilterNarrow) __attribute__((amdgpu_waves_
 // samples of the smoothest), as long as a chunk keeps 32 entries.  Chunks are
 // multiples of the 32-entry FP32 blocks; one chunk is longer than any table.
 // The batched kernel cuts each map's sums the same way.
-int prefilter_split(int size, int mips, int samples, int& chunk) {
+static long long prefilter_pair_tiles(int size, int mips) {
   long long rough = 0;
   for (int m = 1; m < mips; ++m) {
     const int S = std::max(1, size >> m);
     const int tpf = (S + kPrefilterTile - 1) / kPrefilterTile;
     rough += 3ll * tpf * tpf;
   }
+  return rough;
+}
+
+int prefilter_split(int size, int mips, int samples, int& chunk) {
+  const long long rough = prefilter_pair_tiles(size, mips);
   int k = 1;
   while (k < kPrefilterMaxSplit && rough > 0 && rough * k < (k < 8 ? 32768 : 4096) && samples / (2 * k) >= kBlockSums) k *= 2;
   chunk = k == 1 ? (1 << 30) : ((samples + k - 1) / k + kBlockSums - 1) / kBlockSums * kBlockSums;
@@ -353,15 +365,21 @@ void pyramid_levels(int w, int h, LevelC* out) {
 }
 
 // ------------------------------------------------------------ staged levels
+// Source LOD of sample 0 (the half vector N) at a roughness, not clamped to the
+// pyramid.
+static double prefilter_lod(int w, int h, double rough, int samples) {
+  const double a2 = rough * rough;
+  const double pdf = 1.0 / (M_PI * a2 * (4.0 + 0.00001));
+  const double sa_texel = 4.0 * M_PI / (6.0 * static_cast<double>(w) * h);
+  return 0.5 * std::log2(1.0 / (samples * pdf + 0.0001) / sa_texel);
+}
+
 // The lowest source level the sample tables name: the source LOD grows with
 // roughness and away from the lobe's centre, so it is that of sample 0 (the
 // half vector N) at the lowest sampled roughness, 1 / (mips - 1); a margin of
 // 1e-4 level covers the device's rounding.
 int prefilter_first_level(int w, int h, int mips, int samples) {
-  const double rough = mips > 1 ? 1.0 / (mips - 1) : 1.0, a2 = rough * rough;
-  const double pdf = 1.0 / (M_PI * a2 * (4.0 + 0.00001));
-  const double sa_texel = 4.0 * M_PI / (6.0 * static_cast<double>(w) * h);
-  const double lod = 0.5 * std::log2(1.0 / (samples * pdf + 0.0001) / sa_texel);
+  const double lod = prefilter_lod(w, h, mips > 1 ? 1.0 / (mips - 1) : 1.0, samples);
   return std::min(std::max(static_cast<int>(std::floor(lod - 1e-4)), 0), althea_env_levels(w, h) - 1);
 }
 
@@ -386,6 +404,28 @@ int staged_levels(int w, int h, int lowest, StagedLevel* out, size_t* bytes) {
   }
   *bytes = total;
   return first;
+}
+
+// Whether a call's texels are summed by themselves instead of in pairs.  Where the
+// samples' levels are mostly finer than the staged ones, the lines that the
+// lookups touch in global memory bound a CU, as many for a pair as for two texels,
+// and the pairs' half as many blocks leave CUs idle.  The measure is the level of
+// sample 0 at roughness 1 against the first staged level.  Us a cube, pairs and
+// alone (texels gathered from a padded copy of the pyramid took the third):
+//   512 x 256 source,  32^2 x 6, 5 mips,  32 768 samples (0.7 finer)  8 121  4 027  5 761
+//   512 x 256,         64^2, 4 mips,     131 072 (1.7)               32 188 15 606 20 949
+//   64 x 1024,         64^2, 4 mips,       4 096 (-0.3)                 764    374    616
+//   64 x 1024,        128^2, 5 mips,       8 192 (0.2)                2 674  1 979  2 331
+//   64 x 1024,        512^2, 4 mips,       4 096 (-0.3)               5 059  4 794  6 955
+//   512 x 512,        512^2, 4 mips,       4 096 (-0.3)               4 217  4 374  6 634
+//   16 x 2048,        256^2, 6 mips,       8 192 (0.7)               10 000  9 156  8 334
+bool prefilter_alone(int w, int h, int size, int mips, int samples) {
+  StagedLevel staged[kMaxLevels];
+  size_t bytes = 0;
+  const int first = staged_levels(w, h, 0, staged, &bytes);
+  if (mips < 2 || first == 0) return false;
+  const double finer = first - std::max(prefilter_lod(w, h, 1.0, samples), 0.0);
+  return finer > 0.0 || (finer > -0.5 && prefilter_pair_tiles(size, mips) < 256);
 }
 
 size_t prefilter_lds_bytes(size_t staged, int split, int waves, int block_waves) {
@@ -582,14 +622,21 @@ althea_status launch_prefilter_cube(const float* pyr, int env_w, int env_h, int 
   p.map.mips = mips;
   p.map.samples = samples;
   p.map.split = p.map.waves = prefilter_split(size, mips, samples, p.map.chunk);
+  p.map.alone = prefilter_alone(env_w, env_h, size, mips, samples) ? 1 : 0;
   const bool wide = p.map.waves > kPrefilterNarrow;
   const int waves = wide ? kPrefilterWide : kPrefilterNarrow;
   for (int m = 0; m < mips; ++m)
-    p.block_start[m + 1] = p.block_start[m] + prefilter_blocks(size, mips, m, p.map.waves, kPrefilterTile,
+    p.block_start[m + 1] = p.block_start[m] + prefilter_blocks(size, mips, m, p.map.waves, p.map.alone, kPrefilterTile,
                                                                kPrefilterTile, waves);
-  const bool f64 = !(flags & ALTHEA_PRECOMPUTE_FP32_SUMS);
-  auto kernel = wide ? (f64 ? prefilter_wide_kernel<true> : prefilter_wide_kernel<false>)
-                     : (f64 ? prefilter_cube_kernel<true> : prefilter_cube_kernel<false>);
+  const int variant = (flags & ALTHEA_PRECOMPUTE_FP32_SUMS ? 0 : 1) | (wide ? 2 : 0) | (p.map.alone ? 4 : 0);
+  auto kernel = variant == 0   ? prefilter_cube_kernel<false>
+                : variant == 1 ? prefilter_cube_kernel<true>
+                : variant == 2 ? prefilter_wide_kernel<false>
+                : variant == 3 ? prefilter_wide_kernel<true>
+                : variant == 4 ? prefilter_alone_kernel<false, kPrefilterNarrow>
+                : variant == 5 ? prefilter_alone_kernel<true, kPrefilterNarrow>
+                : variant == 6 ? prefilter_alone_kernel<false, kPrefilterWide>
+                               : prefilter_alone_kernel<true, kPrefilterWide>;
   hipLaunchKernelGGL(kernel, dim3(p.block_start[mips]), dim3(64 * waves),
                      mips > 1 ? prefilter_lds_bytes(staged, p.map.split, p.map.waves, waves) : 0, s, p);
   return check_launch("prefilter_cube_kernel");

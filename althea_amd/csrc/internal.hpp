@@ -70,6 +70,8 @@ size_t prefilter_lds_bytes(size_t staged, int split, int waves, int block_waves)
 size_t prefilter_table_bytes(int mips, int samples);
 // Chunks that a cube's rough mips cut their tables into, and entries per chunk.
 int prefilter_split(int size, int mips, int samples, int& chunk);
+// Whether its texels are summed by themselves instead of in pairs.
+bool prefilter_alone(int w, int h, int size, int mips, int samples);
 
 // Kernel launchers (ibl_kernels.hip).
 althea_status launch_ggx_tables(int samples, int mips, int env_w, int env_h, GgxEntry* tables, int* counts,

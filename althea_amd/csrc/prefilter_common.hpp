@@ -1,5 +1,5 @@
-// GGX prefilter of texel pairs shared by the single-map and the batched
-// (persistent) kernels, so both produce bit-identical texels.
+// GGX prefilter of texel pairs, or single texels, shared by the single-map and
+// the batched (persistent) kernels, so both produce bit-identical texels.
 #pragma once
 
 #include <type_traits>
@@ -34,8 +34,8 @@ constexpr int kBlockSums = 32;  // FP32 partial sums flushed to FP64 every 32 sa
 //   kTurnX (otherwise):  F = (x, -y, -z), yaw' = -yaw, pitch' = -pitch.
 // Both act on a level's texel lattice exactly (an even or unit width), so the
 // partner's lookup takes the same fractions and weights at a shifted, or
-// mirrored, cell.
-enum PairTurn { kTurnY, kTurnX };
+// mirrored, cell.  kAlone: a texel by itself (prefilter_alone).
+enum PairTurn { kTurnY, kTurnX, kAlone };
 
 // Partner of texel (face, x, y) of an S x S face, face +X, +Y or +Z.
 __device__ __forceinline__ void pair_partner(int face, int x, int y, int S, bool turn_y, int& face2, int& x2,
@@ -46,12 +46,13 @@ __device__ __forceinline__ void pair_partner(int face, int x, int y, int S, bool
   y2 = mirror ? S - 1 - y : y;
 }
 
-// Sums of the NdotL-weighted source for a pair of texels: FP64 (kF64Sums) or
-// FP32 totals, and the FP32 weight sum of the all-FP32 variant.
-template <bool kF64Sums>
+// Sums of the NdotL-weighted source for a pair of texels (kN = 6: RGB of the
+// texel, RGB of its partner) or one (3): FP64 (kF64Sums) or FP32 totals, and the
+// FP32 weight sum of the all-FP32 variant.
+template <bool kF64Sums, int kN>
 struct PrefilterSums {
   using T = typename std::conditional<kF64Sums, double, float>::type;
-  T v[6] = {0, 0, 0, 0, 0, 0};  // RGB of the texel, RGB of its partner
+  T v[kN] = {};
   float w = 0.0f;
 };
 
@@ -79,9 +80,10 @@ struct StagedAcc {
     const uint32_t o = staged_offset(g, q.ix, q.iy);
     PairTaps t;
     staged_texels(lds, g, o, t.a);
-    staged_texels(lds, g,
-                  kTurn == kTurnY ? o + static_cast<uint32_t>(__mul24(turn, static_cast<int>(g.half))) : g.mirror - o,
-                  t.b);
+    if (kTurn != kAlone)
+      staged_texels(lds, g,
+                    kTurn == kTurnY ? o + static_cast<uint32_t>(__mul24(turn, static_cast<int>(g.half))) : g.mirror - o,
+                    t.b);
     t.a.ax = q.ax, t.a.ay = q.ay;
     return t;
   }
@@ -94,22 +96,23 @@ struct StagedAcc {
     level_texels(pyr, c, q.ix, q.iy, t.a);
     if (kTurn == kTurnY)
       level_texels(pyr, c, q.ix + __mul24(turn, W >> 1), q.iy, t.b);
-    else
+    else if (kTurn == kTurnX)
       level_texels(pyr, c, W - 2 - q.ix, H - 2 - q.iy, t.b);
     t.a.ax = q.ax, t.a.ay = q.ay;
     return t;
   }
   template <PairTurn kTurn>
-  __device__ __forceinline__ static void sum(const PairTaps& t, float w, float s[6]) {
+  __device__ __forceinline__ static void sum(const PairTaps& t, float w, float* s) {
     const TapWeights k = tap_weights(t.a.ax, t.a.ay, w);
     taps_acc(t.a, k, s[0], s[1], s[2]);
-    taps_acc(t.b, kTurn == kTurnY ? k : TapWeights{k.w11, k.w01, k.w10, k.w00}, s[3], s[4], s[5]);
+    if (kTurn != kAlone)
+      taps_acc(t.b, kTurn == kTurnY ? k : TapWeights{k.w11, k.w01, k.w10, k.w00}, s[3], s[4], s[5]);
   }
   // A table entry's two levels.  kTogether: the reads of both are in flight
   // together where both are staged (48 registers of texels), for four waves a
   // SIMD; with six, a level at a time.
   template <PairTurn kTurn>
-  __device__ __forceinline__ void add(const GgxEntry& e, float yaw, float pitch, int turn, float s[6]) const {
+  __device__ __forceinline__ void add(const GgxEntry& e, float yaw, float pitch, int turn, float* s) const {
     const bool two = __float_as_uint(e.w1) != 0u;
     if (kTogether && two && e.l0 >= first) {
       const PairTaps t0 = staged<kTurn>(e.l0, yaw, pitch, turn), t1 = staged<kTurn>(e.l1, yaw, pitch, turn);
@@ -129,16 +132,17 @@ struct StagedAcc {
   }
 };
 
-// Table entries [lo, hi) for one pair (PreFilterEnvMap.comp:147-169): the
+// Table entries [lo, hi) for one pair, or texel (PreFilterEnvMap.comp:147-169): the
 // FP32 per-sample body (each level's bilinear in weight form, added into
 // running FP32 sums); kF64Sums flushes the FP32 sums into FP64 every
 // kBlockSums entries (blocks aligned at multiples of kBlockSums).
-template <bool kF64Sums, PairTurn kTurn, class Acc>
-__device__ __forceinline__ PrefilterSums<kF64Sums> prefilter_pair_range(const Acc& acc,
-                                                                        const GgxEntry* __restrict__ tab, int lo,
-                                                                        int hi, const Frame& fr) {
-  PrefilterSums<kF64Sums> t;
-  float s[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+template <bool kF64Sums, PairTurn kTurn, int kN, class Acc>
+__device__ __forceinline__ PrefilterSums<kF64Sums, kN> prefilter_pair_range(const Acc& acc,
+                                                                            const GgxEntry* __restrict__ tab, int lo,
+                                                                            int hi, const Frame& fr) {
+  static_assert(kN == (kTurn == kAlone ? 3 : 6), "three sums a texel");
+  PrefilterSums<kF64Sums, kN> t;
+  float s[kN] = {};
   GgxEntry next = tab[lo < hi ? lo : 0];
   for (int e = lo; e < hi; ++e) {
     const GgxEntry en = next;
@@ -160,21 +164,21 @@ __device__ __forceinline__ PrefilterSums<kF64Sums> prefilter_pair_range(const Ac
     if (kF64Sums) {
       if ((e & (kBlockSums - 1)) == kBlockSums - 1) {
 #pragma unroll
-        for (int c = 0; c < 6; ++c) t.v[c] += s[c], s[c] = 0.0f;
+        for (int c = 0; c < kN; ++c) t.v[c] += s[c], s[c] = 0.0f;
       }
     } else {
       t.w += en.weight;
     }
   }
 #pragma unroll
-  for (int c = 0; c < 6; ++c) t.v[c] += s[c];
+  for (int c = 0; c < kN; ++c) t.v[c] += s[c];
   return t;
 }
 
 // The pair's values from its sums: FP64 sums over the FP64 weight sum, or
 // all-FP32 sums over their own weight sum.
-template <bool kF64Sums>
-__device__ __forceinline__ float4 prefilter_value(const PrefilterSums<kF64Sums>& t, int texel, double wsum) {
+template <bool kF64Sums, int kN>
+__device__ __forceinline__ float4 prefilter_value(const PrefilterSums<kF64Sums, kN>& t, int texel, double wsum) {
   const int c = 3 * texel;
   if (kF64Sums) {
     const double inv = 1.0 / wsum;
@@ -222,10 +226,11 @@ struct PrefilterMap {
   int split;  // chunks of a rough mip's table, a power of two
   int chunk;  // table entries per chunk, a multiple of kBlockSums
   int waves;  // waves per tile of a rough mip: split, or half of it
+  int alone;  // texels by themselves (prefilter_alone)
 };
 
 constexpr int kPrefilterMaxSplit = 16;
-constexpr int kPrefilterPart = 6 * 64 + 1;  // sums of a chunk: a tile's six, the weight
+constexpr int kPrefilterPart = 6 * 64 + 1;  // sums of a chunk: a tile's six (or three), the weight
 
 // LDS texels of levels first..levels - 1, block-cooperative; the caller
 // synchronises the block.
@@ -253,14 +258,14 @@ __device__ __forceinline__ void stage_levels(const char* __restrict__ pyr, const
 constexpr int kPairUnits = 4;
 
 // Blocks of mip m: a wave per tile of a roughness-0 mip (all six faces),
-// `waves` waves per unit of a rough one.
-__host__ __device__ inline int prefilter_blocks(int size, int mips, int m, int waves, int tw, int th,
-                                                int block_waves) {
+// `waves` waves per unit of a rough one (of texels alone: per tile).
+__host__ __device__ inline int prefilter_blocks(int size, int mips, int m, int waves, bool alone,
+                                                int tw, int th, int block_waves) {
   const int S = size >> m > 1 ? size >> m : 1;
   const int tiles = ((S + tw - 1) / tw) * ((S + th - 1) / th);
   const bool mirror = m == 0 || mips == 1;
   const int per = mirror ? block_waves : block_waves / waves;
-  return ((mirror ? 6 : kPairUnits) * tiles + per - 1) / per;
+  return ((mirror || alone ? 6 : kPairUnits) * tiles + per - 1) / per;
 }
 
 // One block of mip m, the levels staged by the caller.  A rough mip's table is
@@ -276,17 +281,19 @@ __host__ __device__ inline int prefilter_blocks(int size, int mips, int m, int w
 // Measured beside it: 48-byte records of a cell's four texels in global memory
 // (three gathers a lookup) 2.7 ms, the records of neighbouring lanes spreading
 // over more lines than their texels.
-template <bool kF64Sums, int kTW, int kTH, int kWaves, bool kTogether, bool kTwoChunks>
+template <bool kF64Sums, int kTW, int kTH, int kWaves, bool kTogether, bool kTwoChunks, bool kSingle>
 __device__ __forceinline__ void prefilter_block(const PrefilterMap& p, int m, int block, char* lds) {
   static_assert(kTW * kTH == 64, "one wave per tile");
-  using T = typename PrefilterSums<kF64Sums>::T;
+  constexpr int kN = kSingle ? 3 : 6;
+  using Sums = PrefilterSums<kF64Sums, kN>;
+  using T = typename Sums::T;
   const int S = max(1, p.size >> m);
   const int tpr = (S + kTW - 1) / kTW, tiles = tpr * ((S + kTH - 1) / kTH);
   const int wave = static_cast<int>(threadIdx.x >> 6), lane = static_cast<int>(threadIdx.x & 63);
   const bool mirror = m == 0 || p.mips == 1;  // roughness m / (mips - 1) == 0 (block-uniform)
   const int waves = mirror ? 1 : p.waves;
   const int local = (block * kWaves + wave) / waves;
-  const int lt = min(local, (mirror ? 6 : kPairUnits) * tiles - 1);
+  const int lt = min(local, (mirror || kSingle ? 6 : kPairUnits) * tiles - 1);
   const int f = lt / tiles, t = lt - f * tiles;
   const int x = (t % tpr) * kTW + (lane % kTW);
   const int y = (t / tpr) * kTH + (lane / kTW);
@@ -303,32 +310,33 @@ __device__ __forceinline__ void prefilter_block(const PrefilterMap& p, int m, in
     if (active) out[(static_cast<size_t>(f) * S + y) * S + x] = v;
     return;
   }
-  const int face = 2 * min(f, 2);
+  const int face = kSingle ? f : 2 * min(f, 2);
   const bool turn_y = (f & 1) == 0;
   const f3 raw = cube_texel_raw_dir(face, xc, yc, S);
   const Frame fr = local_to_world(raw);
-  const bool mine = (fabsf(raw.x) > fabsf(raw.y)) == turn_y;
+  const bool mine = kSingle || (fabsf(raw.x) > fabsf(raw.y)) == turn_y;
   const bool any = __builtin_amdgcn_ballot_w64(mine) != 0;  // the same for every wave of the unit
   const int count = p.counts[m], part = __builtin_amdgcn_readfirstlane(wave & (waves - 1));
   const StagedAcc<kTogether> acc{lds, p.slv, p.pyr, p.lv, p.first};
   const GgxEntry* tab = p.tables + static_cast<size_t>(m) * p.samples;
-  PrefilterSums<kF64Sums> tot;
-  PrefilterSums<kF64Sums> first;
+  Sums tot, first;
   for (int k = part;;) {
     const int lo = min(count, k * min(p.chunk, count)), hi = any ? min(count, lo + min(p.chunk, count)) : lo;
-    if (turn_y)
-      tot = prefilter_pair_range<kF64Sums, kTurnY>(acc, tab, lo, hi, fr);
+    if constexpr (kSingle)
+      tot = prefilter_pair_range<kF64Sums, kAlone, kN>(acc, tab, lo, hi, fr);
+    else if (turn_y)
+      tot = prefilter_pair_range<kF64Sums, kTurnY, kN>(acc, tab, lo, hi, fr);
     else
-      tot = prefilter_pair_range<kF64Sums, kTurnX>(acc, tab, lo, hi, fr);
+      tot = prefilter_pair_range<kF64Sums, kTurnX, kN>(acc, tab, lo, hi, fr);
     if (!kTwoChunks || (k += waves) >= p.split) break;
     first = tot;
   }
   if (p.split > 1) {
     // The partials take the staged texels' place.
     T* s_part = reinterpret_cast<T*>(lds) + static_cast<size_t>(wave / waves) * p.split * kPrefilterPart;
-    const auto store = [&](int k, const PrefilterSums<kF64Sums>& t) {
+    const auto store = [&](int k, const Sums& t) {
 #pragma unroll
-      for (int c = 0; c < 6; ++c) s_part[k * kPrefilterPart + 64 * c + lane] = t.v[c];
+      for (int c = 0; c < kN; ++c) s_part[k * kPrefilterPart + 64 * c + lane] = t.v[c];
       if (lane == 0) s_part[k * kPrefilterPart + 6 * 64] = static_cast<T>(t.w);
     };
     __syncthreads();
@@ -340,18 +348,19 @@ __device__ __forceinline__ void prefilter_block(const PrefilterMap& p, int m, in
     }
     __syncthreads();
     if (part != 0) return;
-    tot = PrefilterSums<kF64Sums>();
+    tot = Sums();
     for (int k = 0; k < p.split; ++k) {
 #pragma unroll
-      for (int c = 0; c < 6; ++c) tot.v[c] += s_part[k * kPrefilterPart + 64 * c + lane];
+      for (int c = 0; c < kN; ++c) tot.v[c] += s_part[k * kPrefilterPart + 64 * c + lane];
       tot.w += static_cast<float>(s_part[k * kPrefilterPart + 6 * 64]);
     }
   }
   if (!active || !mine) return;
+  out[(static_cast<size_t>(face) * S + y) * S + x] = prefilter_value<kF64Sums>(tot, 0, p.wsum[m]);
+  if (kSingle) return;
   int face2, x2, y2;
   pair_partner(face, x, y, S, turn_y, face2, x2, y2);
-  out[(static_cast<size_t>(face) * S + y) * S + x] = prefilter_value<kF64Sums>(tot, 0, p.wsum[m]);
-  out[(static_cast<size_t>(face2) * S + y2) * S + x2] = prefilter_value<kF64Sums>(tot, 1, p.wsum[m]);
+  out[(static_cast<size_t>(face2) * S + y2) * S + x2] = prefilter_value<kF64Sums>(tot, kSingle ? 0 : 1, p.wsum[m]);
 }
 
 }  // namespace althea
