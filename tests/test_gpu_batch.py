@@ -99,6 +99,21 @@ def test_every_launch_shape_gives_the_same_bits(torch):
             assert all(torch.equal(g, r) for g, r in zip(got, ref)), (tw, th, waves)
 
 
+def test_batch_of_paired_and_single_texels_matches_single_maps(torch):
+    """At 4 096 samples a 64 x 32 source is all in LDS and its texels are paired;
+    most lookups of the tall and the square one go to finer levels, and their
+    texels are summed by themselves.  Each cube has the single-map kernel's bits."""
+    ext = [(64, 32), (64, 1024), (512, 512)]
+    maps = [torch.from_numpy(aa.synth.env(seed=500 + i, width=w, height=h, sigma=0.3, suns=0)).cuda()
+            for i, (w, h) in enumerate(ext)]
+    sizes = [16, 32, 8]
+    b = PrefilterBatch(maps, sizes, mips=4, samples=4096)
+    b.run()
+    for i, (w, h) in enumerate(ext):
+        ref = aa.prefilter_cube(aa.env_pyramid(maps[i]), w, h, sizes[i], 4, 4096)
+        assert torch.equal(b.cube(i), ref), i
+
+
 def test_config3_full_batch_matches_single_map_kernel(torch):
     """The configured batch (config 3): 64 environment maps, widths drawn from
     {256 .. 4096} by batch_widths(64) (height W/2, the config-0 radiance
