@@ -343,8 +343,12 @@ __device__ __forceinline__ unsigned long long shadow_first_slot(const ShadowSlot
 // (four rounds for 2 M items, where one probe a round takes 21 dependent reads).
 // A wave takes at least kWaveSlots, as 16 384 searches cost more than small draws
 // (1 light, 5 000 triangles: 34.5 us without the bound, 28.7 with 256, 29.1 with
-// 512, 34.7 with 1 024).
-constexpr unsigned long long kItemSlots = 4, kWaveSlots = 256;
+// 512, 34.7 with 1 024); where that is more waves than the GPU holds at a time
+// (kRoundWaves, seven a SIMD), as many slots as leave one round of waves, to
+// kWaveSlotsMost (8 lights, 131 072 triangles at 128: 70.5 us with 256 at least,
+// 57.7 so, and 62.9 before the windows; 32 lights, 32 768 triangles at 64: 71.5,
+// 57.9, 66.9; to 512 at most, the first 64).
+constexpr unsigned long long kItemSlots = 4, kWaveSlots = 256, kWaveSlotsMost = 768, kRoundWaves = 7168;
 
 __device__ __forceinline__ void shadow_wave_range(const ShadowSlots& q, int n, int& item, unsigned long long& begin,
                                                   unsigned long long& end) {
@@ -353,7 +357,9 @@ __device__ __forceinline__ void shadow_wave_range(const ShadowSlots& q, int n, i
   const int lane = threadIdx.x & 63;
   const unsigned long long work = q.offsets[n] + kItemSlots * static_cast<unsigned long long>(n);
   const unsigned long long share = (work + waves - 1) / waves;
-  const unsigned long long per = share > kWaveSlots ? share : kWaveSlots;
+  const unsigned long long round = (work + kRoundWaves - 1) / kRoundWaves;
+  const unsigned long long least = round < kWaveSlots ? kWaveSlots : (round < kWaveSlotsMost ? round : kWaveSlotsMost);
+  const unsigned long long per = share > least ? share : least;
   const unsigned long long at[2] = {wave * per, wave * per + per};
   item = 0;
   begin = end = 0;

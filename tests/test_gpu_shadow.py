@@ -114,11 +114,12 @@ def test_no_triangles_and_back_faces(torch):
 
 @pytest.mark.parametrize("tris,lights_n,size,scale", [(1, 1, 1, 3.0), (63, 1, 16, 1.0), (64, 1, 33, 1.0),
                                                       (65, 2, 64, 1.0), (257, 3, 64, 0.3), (1500, 5, 48, 0.02),
-                                                      (40, 2, 512, 8.0)])
+                                                      (40, 2, 512, 8.0), (24000, 20, 32, 0.05), (65000, 16, 64, 0.03)])
 def test_scheduled_windows_match_the_lane_walk(torch, tris, lights_n, size, scale):
     """The scheduled raster runs the lane walk's texel tests, so it gives its
     bits: item counts around its windows of 64, runs of culled items longer than
-    a window, boxes of no texel, of many faces and larger than a wave's share."""
+    a window, boxes of no texel, of many faces and larger than a wave's share,
+    and item counts whose work makes one round of waves."""
     rng = np.random.default_rng(tris)
     lights = np.concatenate([rng.uniform(-0.5, 0.5, (lights_n, 3)), np.zeros((lights_n, 1)),
                              np.full((lights_n, 3), 4.0), np.zeros((lights_n, 1))], 1).astype(np.float32)
