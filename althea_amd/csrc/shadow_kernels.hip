@@ -348,10 +348,25 @@ __device__ __forceinline__ unsigned long long shadow_first_slot(const ShadowSlot
 // kWaveSlotsMost (8 lights, 131 072 triangles at 128: 70.5 us with 256 at least,
 // 57.7 so, and 62.9 before the windows; 32 lights, 32 768 triangles at 64: 71.5,
 // 57.9, 66.9; to 512 at most, the first 64).
-constexpr unsigned long long kItemSlots = 4, kWaveSlots = 256, kWaveSlotsMost = 768, kRoundWaves = 7168;
+//
+// Under the alpha test a slot costs its texture reads and an item next to nothing
+// beside them: 1 slot an item, 128 to 512 a wave.  With the figures above, 32
+// lights over 32 768 triangles at 64 took 104.9 us (82.8 by slots alone), 4 over
+// 18 432 at 128 45.2 (38.5); here 82.0 and 38.9.  Of 1, 2 and 4 an item, 1 to 256 at
+// least and 64 to 1 024 at most, no other is within 6 % of slots alone everywhere.
+template <bool kAlpha>
+struct ShadowSplit {
+  static constexpr unsigned long long kItemSlots = kAlpha ? 1 : 4, kWaveSlots = kAlpha ? 128 : 256,
+                                      kWaveSlotsMost = kAlpha ? 512 : 768;
+};
+constexpr unsigned long long kRoundWaves = 7168;
 
+template <bool kAlpha>
 __device__ __forceinline__ void shadow_wave_range(const ShadowSlots& q, int n, int& item, unsigned long long& begin,
                                                   unsigned long long& end) {
+  constexpr unsigned long long kItemSlots = ShadowSplit<kAlpha>::kItemSlots;
+  constexpr unsigned long long kWaveSlots = ShadowSplit<kAlpha>::kWaveSlots;
+  constexpr unsigned long long kWaveSlotsMost = ShadowSplit<kAlpha>::kWaveSlotsMost;
   const unsigned waves = gridDim.x * (blockDim.x >> 6);
   const unsigned wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
   const int lane = threadIdx.x & 63;
@@ -438,7 +453,7 @@ __global__ __launch_bounds__(256) void shadow_slot_raster_kernel(const ShadowPar
   const int n = p.light_count * p.triangle_count;
   int w0;
   unsigned long long begin, end;
-  shadow_wave_range(p.slots, n, w0, begin, end);
+  shadow_wave_range<kAlpha>(p.slots, n, w0, begin, end);
   const int S = p.size;
   const float inv_s = 1.0f / static_cast<float>(S);
   const size_t cube_floats = static_cast<size_t>(6) * (S + 2) * (S + 2);
