@@ -119,19 +119,28 @@ __global__ __launch_bounds__(256) void ssr_depth_kernel(const SsrParams p) {
   p.depth[taddr(p.depth_tw, x, y)] = q.w != 0.0f ? -1.0f / vz : p.inv_far;
 }
 
+// Frames of more pixels than this read a footprint's rows in pairs.  On a small
+// frame the march is a chain of steps with few waves beside it, and the pairs'
+// branches lengthen every step: capture with 8 shadowed lights, pairs and single
+// reads, 64 x 40 70.2 and 55.5 us, 240 x 135 68.4 and 64.2, 480 x 270 79.3 and 78.5,
+// 640 x 360 82.5 and 118.8, 1280 x 720 196 and 298.
+constexpr int kSsrPairPixels = 1 << 17;
+
 // Two neighbouring texels of a block row (4-byte aligned).
 typedef float depth_pair __attribute__((ext_vector_type(2), aligned(4)));
 
-// Bilinear CLAMP_TO_EDGE depth at uv in [0, 1]^2.  Inside the frame a row's two
-// texels are one 8-byte read; the 1 in 8 footprints whose right column is the
-// next block's (+25 texels from the row's last) read that column again.
+// Bilinear CLAMP_TO_EDGE depth at uv in [0, 1]^2.  kPairs: inside the frame a
+// row's two texels are one 8-byte read; the 1 in 8 footprints whose right column
+// is the next block's (+25 texels from the row's last) read that column again.
+// Otherwise four reads without a branch.  The same texels either way.
+template <bool kPairs>
 __device__ __forceinline__ float depth_bilinear(const float* __restrict__ d, int tw, int W, int H, float u, float v) {
   const float x = fmaf(u, static_cast<float>(W), -0.5f), y = fmaf(v, static_cast<float>(H), -0.5f);
   const float fx = floorf(x), fy = floorf(y);
   const float ax = x - fx, ay = y - fy;
   const int ix = static_cast<int>(fx), iy = static_cast<int>(fy);
   float a0, b0, a1, b1;
-  if (static_cast<unsigned>(ix) < static_cast<unsigned>(W - 1) &&
+  if (kPairs && static_cast<unsigned>(ix) < static_cast<unsigned>(W - 1) &&
       static_cast<unsigned>(iy) < static_cast<unsigned>(H - 1)) {
     const int i = taddr(tw, ix, iy);
     // +8 in a block, or one block row on (32 tw) less 3 rows of 8.
@@ -149,10 +158,15 @@ __device__ __forceinline__ float depth_bilinear(const float* __restrict__ d, int
   } else {
     const int x0 = min(max(ix, 0), W - 1), x1 = min(max(ix + 1, 0), W - 1);
     const int y0 = min(max(iy, 0), H - 1), y1 = min(max(iy + 1, 0), H - 1);
-    a0 = d[taddr(tw, x0, y0)];
-    b0 = d[taddr(tw, x1, y0)];
-    a1 = d[taddr(tw, x0, y1)];
-    b1 = d[taddr(tw, x1, y1)];
+    // The other three texels from the first: +1 in a block, +25 into the next
+    // block; dy as above.
+    const int i = taddr(tw, x0, y0);
+    const int dx = x1 == x0 ? 0 : ((x0 & 7) == 7 ? 25 : 1);
+    const int dy = y1 == y0 ? 0 : ((y0 & 3) == 3 ? (tw << 5) - 24 : 8);
+    a0 = d[i];
+    b0 = d[i + dx];
+    a1 = d[i + dy];
+    b1 = d[i + dy + dx];
   }
   const float top = fmaf(b0 - a0, ax, a0), bot = fmaf(b1 - a1, ax, a1);
   return fmaf(bot - top, ay, top);
@@ -191,7 +205,7 @@ __host__ __device__ inline int ssr_band_tiles(int tiles_x, int tiles_y) {
   return ((tiles_x + kXcds - 1) / kXcds) * tiles_y;
 }
 
-template <int kFmt, bool kShadow = false>
+template <int kFmt, bool kShadow, bool kPairs>
 __global__ __launch_bounds__(256) void ssr_capture_kernel(const SsrParams p, const float4* __restrict__ lights) {
   const int tiles_x = (p.width + kSsrTile - 1) / kSsrTile, tiles_y = (p.height + kSsrTile - 1) / kSsrTile;
   const int band = blockIdx.x % kXcds, j = blockIdx.x / kXcds;
@@ -264,7 +278,7 @@ __global__ __launch_bounds__(256) void ssr_capture_kernel(const SsrParams p, con
   for (int i = 1; i <= last; ++i) {
     const float k = static_cast<float>(i);
     const float u = fmaf(k, su, u0), v = fmaf(k, sv, v0);
-    const float s = depth_bilinear(p.depth, p.depth_tw, p.width, p.height, u, v);
+    const float s = depth_bilinear<kPairs>(p.depth, p.depth_tw, p.width, p.height, u, v);
     const float m = s * fmaf(k, vzk, vz0);
     // The point lies at -ray / m from the eye; (-ray / m + EP) . perp has the
     // sign of m (EP . perp m - ray . perp), both products affine in k.  Where
@@ -462,19 +476,19 @@ althea_status launch_ssr_capture(const althea_gbuffer_view* g, const althea_ibl_
     p.prefiltered = reinterpret_cast<const float4*>(pref_b);
     p.irradiance = reinterpret_cast<const float4*>(irr_b);
   }
-  if (g->format == ALTHEA_GBUFFER_FP32) {
-    hipLaunchKernelGGL((ssr_depth_kernel<ALTHEA_GBUFFER_FP32>), dgrid, dim3(256), 0, s, p);
-    if (sh)
-      hipLaunchKernelGGL((ssr_capture_kernel<ALTHEA_GBUFFER_FP32, true>), grid, dim3(256), 0, s, p, lights4);
-    else
-      hipLaunchKernelGGL((ssr_capture_kernel<ALTHEA_GBUFFER_FP32>), grid, dim3(256), 0, s, p, lights4);
-  } else {
-    hipLaunchKernelGGL((ssr_depth_kernel<ALTHEA_GBUFFER_FP16>), dgrid, dim3(256), 0, s, p);
-    if (sh)
-      hipLaunchKernelGGL((ssr_capture_kernel<ALTHEA_GBUFFER_FP16, true>), grid, dim3(256), 0, s, p, lights4);
-    else
-      hipLaunchKernelGGL((ssr_capture_kernel<ALTHEA_GBUFFER_FP16>), grid, dim3(256), 0, s, p, lights4);
-  }
+  const bool fp32 = g->format == ALTHEA_GBUFFER_FP32;
+  auto depth = fp32 ? ssr_depth_kernel<ALTHEA_GBUFFER_FP32> : ssr_depth_kernel<ALTHEA_GBUFFER_FP16>;
+  hipLaunchKernelGGL(depth, dgrid, dim3(256), 0, s, p);
+  const int variant = (fp32 ? 0 : 1) | (sh ? 2 : 0) | (n > kSsrPairPixels ? 4 : 0);
+  auto capture = variant == 0   ? ssr_capture_kernel<ALTHEA_GBUFFER_FP32, false, false>
+                 : variant == 1 ? ssr_capture_kernel<ALTHEA_GBUFFER_FP16, false, false>
+                 : variant == 2 ? ssr_capture_kernel<ALTHEA_GBUFFER_FP32, true, false>
+                 : variant == 3 ? ssr_capture_kernel<ALTHEA_GBUFFER_FP16, true, false>
+                 : variant == 4 ? ssr_capture_kernel<ALTHEA_GBUFFER_FP32, false, true>
+                 : variant == 5 ? ssr_capture_kernel<ALTHEA_GBUFFER_FP16, false, true>
+                 : variant == 6 ? ssr_capture_kernel<ALTHEA_GBUFFER_FP32, true, true>
+                                : ssr_capture_kernel<ALTHEA_GBUFFER_FP16, true, true>;
+  hipLaunchKernelGGL(capture, grid, dim3(256), 0, s, p, lights4);
   const althea_status st = check_launch("ssr_capture_kernel");
   if (border_mem) (void)hipFreeAsync(border_mem, s);
   return st;

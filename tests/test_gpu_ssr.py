@@ -146,6 +146,22 @@ def test_ssr_capture_block_edges_match_oracle(torch, ibl, W, H):
             assert r["err"]["max"] < 2e-3, r
 
 
+@pytest.mark.parametrize("W,H", [(9, 14565), (17, 8192), (513, 256), (1032, 129), (512, 256)])
+def test_ssr_capture_of_larger_frames_matches_oracle(torch, ibl, W, H):
+    """Frames of more than 2^17 pixels read a row's two texels at once: widths at
+    the edges of the depth plane's blocks, as above, with enough rows (and the
+    largest frame that does not)."""
+    ibl_res, _ = ibl
+    scene = wall_scene(W=W, H=H)[0]
+    scene.lights = np.array([[0.0, 2.0, -4.0, 0.0, 20.0, 20.0, 20.0, 0.0]], np.float32)
+    got = _capture(torch, scene, ibl_res).level(0).cpu().numpy().reshape(-1, 4).astype(np.float64)
+    pix = _all_pixels(scene)[np.random.default_rng(W).permutation(W * H)[:12000]]
+    r = _compare_capture(scene, ibl_res.views_numpy(), got[pix[:, 1] * W + pix[:, 0]], pix)
+    print("SSR", W, H, r)
+    assert r["hits"] > 100 and r["clear"] > 0.5, r
+    assert r["disagree_clear"] == 0 and r["err"]["max"] < 2e-3, r
+
+
 def _far_plane(scene, far):
     """The scene under the projection of another far plane (near as it was)."""
     P, near = np.zeros((4, 4)), 0.01
