@@ -5,7 +5,7 @@
 // cost (largest first), and blocks of a grid sized to the machine pull items
 // from an atomic counter until the list is exhausted (greedy list scheduling
 // of the longest items first).  Every texel runs the single-map
-// kernel's sums (prefilter_pair_sums), so batched and single results are
+// kernel's sums (prefilter_block), so batched and single results are
 // bit-identical.
 //
 // A run replays one hipGraph: the pyramid chains of all maps, the sample
@@ -34,8 +34,9 @@ namespace althea {
 // taken their place.  Blocks of 8 waves: two a CU at the default 16 waves (four
 // a SIMD, both levels of a sample in flight), so one stages or combines beside
 // another's samples.  12 maps of 1024, 512 and 256 texels width in one run: 2.91
-// ms gathering from global memory, 2.05 here; blocks of 16 waves 2.22, of 4 with
-// a whole tile to a wave 2.63; a level at a time at six waves a SIMD 2.27.
+// ms gathering from global memory, 2.05 here (1.78 since all maps' pyramids share
+// their launches); beside the 2.05, blocks of 16 waves 2.22, of 4 with a whole
+// tile to a wave 2.63; a level at a time at six waves a SIMD 2.27.
 constexpr int kBatchWaves = 8;
 
 template <bool kF64Sums, int kTW, int kTH, bool kAlone>

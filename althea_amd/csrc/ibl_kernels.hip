@@ -656,9 +656,10 @@ althea_status launch_prefilter_cube(const float* pyr, int env_w, int env_h, int 
 // whose r-free parts are a table of the sample set, and D = den^2 / (pi r^2):
 // one reciprocal a sample, no square root.  pdf = D cos / (4 cos + 1e-5)
 // (PreFilterEnvMap.comp:155-161) takes D (1/4 - 1e-5 / (16 cos)) with 1 / cos =
-// 1.415 - 0.425 L.z on the kept range, 5e-8 of the pdf.
+// 1.415 - 0.425 L.z on the kept range, off by up to 0.05: 1.3e-7 of the pdf.
 //
-// Bound: VALU (about 140 a step).  One lane per query walked its samples alone,
+// Bound: VALU (about 140 a step with the wave on a query, 0.93 of the nominal
+// issue rate).  One lane per query walked its samples alone,
 // 250 VALU each with IEEE roots and quotients, its lookups unrelated to its
 // neighbours': 2^18 queries of 1024 samples from 1024 x 512, 2.06 ms, here 0.91;
 // 1 394 queries of 605 samples, 598 us (a wave's latency of all samples), here
@@ -1226,9 +1227,9 @@ __device__ __forceinline__ int fold_cell(float x, float& t) {
 //
 // Bound: the gathers. A gather instruction whose lanes each read 12 or 16
 // bytes takes 16 cycles of the texture data return; the eight lanes of a
-// sample read one node's 96 bytes, so a round's loads stay at 16.5 cycles
-// (31 for 64 unrelated lookups, irradiance_cube_kernel) and the return is 93 %
-// busy, and a lookup costs about 30 VALU instead of 115.  512 x 256 source,
+// sample read one node's 96 bytes, so a round's loads stay at 16.4 cycles
+// (31 for 64 unrelated lookups, irradiance_cube_kernel) and the return is 94 %
+// busy, and a lookup costs 36 VALU in all instead of 115.  512 x 256 source,
 // 32^2 x 6 texels, 300 x 150 samples: 1.09 -> 0.51 ms.  Measured beside it
 // for the whole precompute (0.816 ms): 16-byte slots 0.84 (4.8 MB of nodes
 // against 3.6 MB in a 4 MB L2), RG and B planes (eight narrower loads a
@@ -1491,8 +1492,9 @@ althea_status launch_irradiance(const float* pyr, int env_w, int env_h, int size
 // each in turn.  32-sample FP32 block sums flushed into FP64, the waves' FP64
 // partials combined in wave order, FP64 normalisation.
 //
-// Bound: VALU, 19 a column and sample (about 120 with the half vector formed by
-// every lane): 128^2 x 1024 samples, 62 -> 15 us.
+// Bound: VALU, 30 a column and sample in all, 19 of them the loop's (about 120
+// with the half vector formed by every lane), at 0.87 of the nominal issue rate:
+// 128^2 x 1024 samples, 62 -> 14 us.
 constexpr int kLutWaves = 16;
 
 __global__ __launch_bounds__(64 * kLutWaves) void brdf_lut_kernel(int size, int samples, int chunk,

@@ -83,10 +83,13 @@ struct FwdParams {
 // into LDS once and its waves take their operands (88 registers: three waves a
 // SIMD) from there; each wave reading its 22 KB of operands from L2 by itself, in
 // rows 64 and 128 bytes apart, took as long as one or two tiles.  50 001 queries
-// 14.7 -> 8.4 us (back to back into one output), 200 000 38.6 -> 20.1, 1 000 000
-// 99.5 -> 75.2, 4 000 000 316 -> 297.  Persistent grids (256 blocks of 12 or 8
-// waves, 512 or 768 of 4) were no faster up to 200 000, and all but the first 4
-// to 16 % slower than the start at 4 000 000.  Bound: VALU (encoding, SiLU).
+// 14.3 -> 8.0 us into one output again and again, 14.2 -> 8.9 on buffers that no
+// recent call has touched; 200 000 38.6 -> 20.1, 1 000 000 99.5 -> 75.2, 4 000 000
+// 316 -> 297.  Persistent grids (256 blocks of 12 or 8 waves, 512 or 768 of 4) were
+// no faster up to 200 000, and all but the first 4 to 16 % slower at 4 000 000 than
+// the kernel that read from L2.  Bound: VALU (encoding, SiLU) from some 10^5
+// queries on; below, the launch and one tile's chain (50 001: 0.37 of the VALU
+// issue rate at one wave a SIMD).
 constexpr int kInferWaves = 4, kInferBlocks = 4096;
 
 __global__ __launch_bounds__(64 * kInferWaves) void mlp_infer_kernel(const FwdParams p) {
@@ -131,10 +134,11 @@ __global__ __launch_bounds__(64 * kInferWaves) void mlp_infer_kernel(const FwdPa
 //
 // The activations of a batch of 65 536 are 57 MB: written by a forward kernel in
 // 2-byte stores and read back by a gradient kernel they took 31 + 19 us under
-// the profiler, this kernel 24.  A call of the gradients, with the reduction:
-// 65 536 samples 56 -> 27 us, 16 384 32 -> 22, 1 000 28 -> 13.  Bound: VALU (SiLU
-// and its derivative) and the latency of a tile's six layers at two waves a SIMD
-// (eight waves: 157 KB of LDS, one block a CU).
+// the profiler, this kernel 23.5.  A call of the gradients, with the reduction:
+// 65 536 samples 56 -> 27 us, 16 384 32 -> 22, 1 000 28 -> 13.  Bound: the latency
+// of a tile's six layers at no more than two waves a SIMD (eight waves: 157 KB of
+// LDS, one block a CU), most of it VALU (SiLU and its derivative) that issues at
+// 0.30 of its rate.
 struct TrainParams {
   MlpDeviceWeights w;
   const float4* dir_rough;
@@ -665,8 +669,7 @@ static size_t queue_count_bytes(size_t regions) { return (regions * sizeof(uint3
 althea_status mlp_resolve_queue(const althea_mlp* m, size_t regions, MlpInferenceView* v) {
   althea_status st = mlp_inference_view(m, v);
   if (st != ALTHEA_OK) return st;
-  // The queue is the handle's scratch (like its activations), so a const
-  // handle may grow it.
+  // The queue is the handle's scratch, so a const handle may grow it.
   MlpState* s = const_cast<MlpState*>(&m->s);
   if (regions > s->queue_regions) {
     ALTHEA_TRY_HIP(hipDeviceSynchronize());  // an earlier frame may still read the old queue

@@ -273,9 +273,9 @@ __host__ __device__ inline int prefilter_blocks(int size, int mips, int m, int w
 // where the block has half as many waves as the table has chunks) two; the
 // chunks' partials are added in chunk order, so the bits are the same.
 //
-// Bound: VALU (86 % busy at four waves a SIMD).  A sample costs a pair of
-// texels about 160 VALU (66 for the shared direction and angles) and 24
-// ds_read2_b32; one texel alone, gathering from global memory, took 115 VALU
+// Bound: VALU (the nominal issue rate, one wave instruction a SIMD per 4 cycles,
+// is reached).  A sample costs a pair of texels about 160 VALU (66 for the shared
+// direction and angles; 173 over the launch) and 24 ds_read2_b32; one texel alone, gathering from global memory, took 115 VALU
 // and eight gathers at 16 cycles of the texture data return, which was 98 %
 // busy.  2048 x 1024 source to 512^2 x 6 mips at 1024 samples: 1.83 ms -> 0.95.
 // Measured beside it: 48-byte records of a cell's four texels in global memory
