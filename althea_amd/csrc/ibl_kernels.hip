@@ -333,12 +333,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(4))
   prefilter_cube<kF64Sums, kWaves, false, true>(p, s_levels);
 }
 
-// Chunks of a rough mip's table: doubled while the pairs of tiles times the
-// chunks stay under 4096 waves (to 16), or to 8 while they stay under 32 768
-// (finer blocks level the last round, the roughest tiles having half the kept
-// samples of the smoothest), as long as a chunk keeps 32 entries.  Chunks are
-// multiples of the 32-entry FP32 blocks; one chunk is longer than any table.
-// The batched kernel cuts each map's sums the same way.
+// Pairs of 8 x 8 tiles of the rough mips.
 static long long prefilter_pair_tiles(int size, int mips) {
   long long rough = 0;
   for (int m = 1; m < mips; ++m) {
@@ -349,6 +344,12 @@ static long long prefilter_pair_tiles(int size, int mips) {
   return rough;
 }
 
+// Chunks of a rough mip's table: doubled while the pairs of tiles times the
+// chunks stay under 4096 waves (to 16), or to 8 while they stay under 32 768
+// (finer blocks level the last round, the roughest tiles having half the kept
+// samples of the smoothest), as long as a chunk keeps 32 entries.  Chunks are
+// multiples of the 32-entry FP32 blocks; one chunk is longer than any table.
+// The batched kernel cuts each map's sums the same way.
 int prefilter_split(int size, int mips, int samples, int& chunk) {
   const long long rough = prefilter_pair_tiles(size, mips);
   int k = 1;
@@ -659,12 +660,11 @@ althea_status launch_prefilter_cube(const float* pyr, int env_w, int env_h, int 
 // 1.415 - 0.425 L.z on the kept range, off by up to 0.05: 1.3e-7 of the pdf.
 //
 // Bound: VALU (about 140 a step with the wave on a query, 0.93 of the nominal
-// issue rate).  One lane per query walked its samples alone,
-// 250 VALU each with IEEE roots and quotients, its lookups unrelated to its
-// neighbours': 2^18 queries of 1024 samples from 1024 x 512, 2.06 ms, here 0.91;
-// 1 394 queries of 605 samples, 598 us (a wave's latency of all samples), here
-// 18.  The error against 64 bits went from 2.1e-5 (sin and cos of theta by FP32
-// roots) to 4.8e-7.
+// issue rate).  One lane per query walked its samples alone, 250 VALU each with
+// IEEE roots and quotients, its lookups unrelated to its neighbours': 2^18 queries
+// of 1024 samples from 1024 x 512, 2.06 ms, here 0.91; 1 394 queries of 605
+// samples, 598 us (a wave's latency of all samples), here 18.  The error against
+// 64 bits went from 2.1e-5 (sin and cos of theta by FP32 roots) to 4.8e-7.
 struct PointParams {
   LevelC lv[kMaxLevels];
   StagedLevel slv[kMaxLevels];

@@ -275,12 +275,13 @@ __host__ __device__ inline int prefilter_blocks(int size, int mips, int m, int w
 //
 // Bound: VALU (the nominal issue rate, one wave instruction a SIMD per 4 cycles,
 // is reached).  A sample costs a pair of texels about 160 VALU (66 for the shared
-// direction and angles; 173 over the launch) and 24 ds_read2_b32; one texel alone, gathering from global memory, took 115 VALU
-// and eight gathers at 16 cycles of the texture data return, which was 98 %
-// busy.  2048 x 1024 source to 512^2 x 6 mips at 1024 samples: 1.83 ms -> 0.95.
-// Measured beside it: 48-byte records of a cell's four texels in global memory
-// (three gathers a lookup) 2.7 ms, the records of neighbouring lanes spreading
-// over more lines than their texels.
+// direction and angles; 173 over the launch) and 24 ds_read2_b32; one texel
+// alone, gathering from global memory, took 115 VALU and eight gathers at 16
+// cycles of the texture data return, which was 98 % busy.  2048 x 1024 source to
+// 512^2 x 6 mips at 1024 samples: 1.83 ms -> 0.95.  Measured beside it: 48-byte
+// records of a cell's four texels in global memory (three gathers a lookup) 2.7
+// ms, the records of neighbouring lanes spreading over more lines than their
+// texels.
 template <bool kF64Sums, int kTW, int kTH, int kWaves, bool kTogether, bool kTwoChunks, bool kSingle>
 __device__ __forceinline__ void prefilter_block(const PrefilterMap& p, int m, int block, char* lds) {
   static_assert(kTW * kTH == 64, "one wave per tile");
